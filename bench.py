@@ -696,7 +696,7 @@ def chunk_leg(w, steps: int, warmup: int, with_bwd: bool) -> dict:
         elif rid == 0:
             bwd_name = f"chunk_bwd_dscan<{w.d}> + chunk_bwd_pair<{w.d}>"
         elif w.d == 128:
-            bwd_name = "chunk_prep<128,2> + scan_bwd_rows<128,2> (fp32) + chunk_bwd_tok<128,2>"
+            bwd_name = "chunk_prep<128,2> + scan_bwd_adamf<128> (fp32) + chunk_bwd_tok<128,2>"
         else:
             bwd_name = f"chunk_bwd_ascan<{w.d}> + chunk_bwd_tok_range<{w.d},{rid}> (2 segments, two streams)"
         out["roofline"] = roof(bwd_name, bwd_bytes_per_token_head(w) * units,

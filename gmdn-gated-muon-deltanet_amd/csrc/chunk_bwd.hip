@@ -783,7 +783,7 @@ static hipError_t launch_bwd_muon_chunks(const ChunkArgs& a, int ns, int precisi
 // token gradients with Gb_i = dU_i.  states = [S | M | V | Kw | Uv | a b m n].
 size_t chunk_bwd_adam_mat_ws_floats(int64_t BH, int64_t N, int d) {
   const int64_t BHN = BH * N;
-  return (size_t)(3 * BHN * (int64_t)d * d + 8 * BHN + BHN * (d / 16) * 4 + 64);
+  return (size_t)(2 * BHN * (int64_t)d * d + 8 * BHN + BHN * (d / 16) * 4 + 64);
 }
 
 hipError_t chunk_bwd_adam_mat_launch(const ChunkArgs& a, int d, float* ws, hipStream_t stream) {
@@ -796,8 +796,7 @@ hipError_t chunk_bwd_adam_mat_launch(const ChunkArgs& a, int d, float* ws, hipSt
   const float* abm = S + 5 * BHN * mat;
   float* gS = ws;
   float* dU = gS + BHN * mat;
-  float* dK = dU + BHN * mat;
-  float* abm2 = dK + BHN * mat;  // the prep kernel's copy of the scalars (unused)
+  float* abm2 = dU + BHN * mat;  // the prep kernel's copy of the scalars (unused)
   float* sc = abm2 + 4 * BHN;    // da, db, dm, dn
   float* part = ws + ((sc + 4 * BHN - ws + 63) & ~(int64_t)63);
   hipError_t e = chunk_prep_launch(a, D, 2, false, true, nullptr, nullptr, gS, abm2, stream);
@@ -805,7 +804,7 @@ hipError_t chunk_bwd_adam_mat_launch(const ChunkArgs& a, int d, float* ws, hipSt
   ScanArgs sa{};
   sa.U = Uv; sa.K = Kw; sa.a = abm; sa.b = abm + BHN; sa.m = abm + 2 * BHN; sa.n = abm + 3 * BHN;
   sa.S_all = a.states; sa.M_all = a.states + BHN * mat; sa.V_all = a.states + 2 * BHN * mat;
-  sa.gS = gS; sa.dU = dU; sa.dK = dK;
+  sa.gS = gS; sa.dU = dU;  // no dK: the E-form below accounts for every path through K
   sa.da = sc; sa.db = sc + BHN; sa.dm = sc + 2 * BHN; sa.dn = sc + 3 * BHN;
   sa.BH = BH; sa.N = a.N; sa.dh = D; sa.rule = 2; sa.ns = 0; sa.precision = GMDN_PREC_IEEE;
   sa.stream = stream;

@@ -18,7 +18,8 @@ struct ScanArgs {
 // delta / adam (rows of the state are independent)
 hipError_t scan_fwd_rows_launch(const ScanArgs& s);
 hipError_t scan_bwd_rows_launch(const ScanArgs& s, float* part);
-// chunk-parallel dK_i = -S_i^T dU_i plus scalar gradients (all rules)
+// chunk-parallel dK_i = -S_i^T dU_i plus scalar gradients (all rules);
+// adam with dK null: the scalar gradients only
 hipError_t scan_bwd_dk_launch(const ScanArgs& s, const float* part);
 // muon (msign couples the whole state)
 hipError_t scan_fwd_muon_launch(const ScanArgs& s);

@@ -3,15 +3,13 @@
 //
 // Row-separable rules (delta, adam).  Row r of G_i = U_i - S_i K_i needs only
 // row r of S_i, and the delta/adam updates are elementwise, so every 16-row
-// tile of S is an independent recurrence.  One wave owns one row tile for the
-// whole sequence and keeps it in registers as D-layout tiles of S^T (lane <->
-// row r, registers <-> columns c); a workgroup of two waves shares one
-// LDS-staged copy of each chunk's K (fp32, swizzled, double buffered and
-// filled by global_load_lds_dwordx4 while the previous chunk computes).
+// tile of S is an independent recurrence.  A workgroup owns 16 rows (exact
+// float32 products: scan_fwd_rowsf, scan_bwd_rowsf) or 32 rows (bf16x3:
+// scan_fwd_rows8, scan_bwd_rows8) for the whole sequence; its waves hold
+// D-layout tiles of S^T (lane <-> row r, registers <-> columns c).
 //
-//   forward, chunk i, wave tile rows r:
-//     G^T = U^T - K^T S^T       (MFMA tiles: A = K^T rows (LDS column reads),
-//                                B = -S^T from the wave's own tiles, pair order)
+//   forward, chunk i, rows r:
+//     G^T = U^T - K^T S^T       (MFMA tiles: A = K^T, B = -S^T)
 //     delta: S^T <- a S^T + G^T
 //     adam : M^T <- m M^T + (1-m) G^T ; V^T <- n V^T + (1-n) G^T.^2 ;
 //            S^T <- a S^T + b M^T / (sqrt(V^T) + eps)
@@ -19,17 +17,13 @@
 //   backward (reverse over chunks; Sb = dL/dS_{i+1}):
 //     delta: Gb = Sb
 //     adam : elementwise VJP of the moments (fast_scan.py:167-182)
-//     dU_i = Gb ;  Sb <- a Sb - Gb K^T + gS_i   (A = K rows (LDS row reads),
-//                                                B = -Gb^T from registers)
+//     dU_i = Gb ;  Sb <- a Sb - Gb K^T + gS_i   (A = K rows, B = -Gb^T)
 //   dK_i = -S_i^T Gb_i and the scalar gradients are formed per chunk by a
 //   second, chunk-parallel kernel (contraction over all rows of S).
 #include "prec.h"
 #include "scan_a.h"
 
 namespace gmdn {
-
-constexpr int A_WAVES = 2;                 // row tiles per workgroup
-constexpr int A_THREADS = A_WAVES * 64;
 
 // blockIdx -> (bh, row block).  Workgroups are dispatched round-robin over
 // the 8 XCDs; keep all row blocks of one (b, h) on one XCD so they share its
@@ -46,89 +40,118 @@ GMDN_DEV void map_rows_block(int64_t BH, int nblk, int64_t& bh, int& blk) {
   }
 }
 
-template <int D, int RULE, int PREC>
-__global__ void __launch_bounds__(A_THREADS)
-scan_fwd_rows(const float* __restrict__ U, const float* __restrict__ K,
-              const float* __restrict__ av, const float* __restrict__ bv,
-              const float* __restrict__ mv, const float* __restrict__ nv,
-              float* __restrict__ S_all, float* __restrict__ M_all,
-              float* __restrict__ V_all, int64_t BH, int N) {
-  using P = typename PrecSel<PREC>::T;
-  constexpr int NT = D / 16;   // 16-wide column tiles of a row tile
-  constexpr int NKB = D / 32;  // 32-wide k-blocks
-  extern __shared__ __align__(16) float smem[];
+// ------------------------------------ exact float32: D/16 waves per 16 rows
+// One workgroup of D/16 waves per 16 rows of S; wave w holds column tile w
+// (one D-layout tile of S^T per lane, four values).  v_mfma_f32_16x16x4_f32
+// steps take the contraction in the order k = 16 t + 4 G + e (tile t, step e,
+// lane group G), so that the shared operand, the workgroup's 16 rows of S, is
+// one 16-byte LDS read per tile from an exchange each wave writes one 16-byte
+// piece of (padded rows: conflict-free; double buffered: one barrier a chunk).
+// A wave reads its own 16 columns of K_i only, so K_i goes straight from
+// global memory to the operand registers, two chunks in flight, and never
+// through LDS.
+//
+// Bound: the MFMA pipe (D/4 products of 32 cycles per wave and chunk, two
+// waves a SIMD at D = 128: 0.85 us a chunk) and the chain around it.  The
+// rows used to be split over waves (16 rows x all columns a wave, K_i through
+// LDS as float32): eight times the products and the elementwise update in one
+// wave's chain, two of the four SIMDs idle. Measured (adam, d = 128, 32 chunks):
+// 423 -> 77 us at 16 heads, 445 -> 235 us at 64; adam d = 64, 8 heads, 16
+// chunks 60 -> 19 us; delta d = 128, 64 heads, 64 chunks 478 -> 330 us.
+template <int D>
+struct RowsfLds {
+  static constexpr int LD = D + 4;          // padded row of the exchange
+  static constexpr int X = 16 * LD;         // floats of one buffer
+};
+
+template <int D, int RULE>
+__global__ void __launch_bounds__(D * 4)
+scan_fwd_rowsf(const float* __restrict__ U, const float* __restrict__ K,
+               const float* __restrict__ av, const float* __restrict__ bv,
+               const float* __restrict__ mv, const float* __restrict__ nv,
+               float* __restrict__ S_all, float* __restrict__ M_all,
+               float* __restrict__ V_all, int64_t BH, int N) {
+  constexpr int NT = D / 16;
+  constexpr int LD = RowsfLds<D>::LD;
+  __shared__ __align__(16) float xs[2][RowsfLds<D>::X];
 
   int64_t bh;
   int blk;
-  map_rows_block(BH, D / (16 * A_WAVES), bh, blk);
+  map_rows_block(BH, NT, bh, blk);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = lane_id(), G = l >> 4, rl = l & 15;
-  const int r0 = (blk * A_WAVES + wave_id()) * 16;  // first row of this wave's tile
   const int64_t mat = (int64_t)D * D;
-  const float* Ub = U + bh * N * mat;
-  const float* Kb = K + bh * N * mat;
+  const int64_t base = bh * N * mat;
+  // 32-bit lane offsets from scalar bases
+  const uint32_t so = (16 * blk + rl) * D + 16 * w + 4 * G;  // this lane's piece of a state
+  const uint32_t ko = 4 * G * D + 16 * w + rl;               // K columns of tile w
 
-  f32x4 S[NT], M[NT], V[NT];
+  struct Chunk {  // one chunk's operands of this lane
+    float k[NT][4];
+    f32x4 u;
+    float a, b, m, n;
+  };
+  auto load = [&](Chunk& c, int i) {
+    const int64_t o = base + i * mat;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) S[t] = M[t] = V[t] = zero4();
-
-  // row r0+rl, columns 16t + 4G .. +3 of a (D x D) matrix at base
-  auto roff = [&](int t) { return (int64_t)(r0 + rl) * D + 16 * t + 4 * G; };
-
-  if (N > 0) lds_dma_matrix<D, A_THREADS>(smem, Kb);
-  f32x4 Unext[NT];
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-  for (int t = 0; t < NT; ++t) Unext[t] = *reinterpret_cast<const f32x4*>((Ub + roff(t)));
-  wait_vmem();
-  __syncthreads();
-
-  for (int i = 0; i < N; ++i) {
-    const float* kl = (smem + (i & 1) * D * D);
-    f32x4 Ucur[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) Ucur[t] = Unext[t];
-    if (i + 1 < N) {
-      lds_dma_matrix<D, A_THREADS>((smem + ((i + 1) & 1) * D * D), Kb + (i + 1) * mat);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) Unext[t] = *reinterpret_cast<const f32x4*>((Ub + (i + 1) * mat + roff(t)));
-    }
+      for (int e = 0; e < 4; ++e) c.k[t][e] = (K + o + (16 * t + e) * D)[ko];
+    c.u = *reinterpret_cast<const f32x4*>(U + o + so);
     const int64_t si = bh * N + i;
-    // pre-update states
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      *reinterpret_cast<f32x4*>((S_all + si * mat + roff(t))) = S[t];
-      if constexpr (RULE == 2) {
-        if (M_all) *reinterpret_cast<f32x4*>((M_all + si * mat + roff(t))) = M[t];
-        if (V_all) *reinterpret_cast<f32x4*>((V_all + si * mat + roff(t))) = V[t];
-      }
-    }
-    // B operands: -S^T, one per k-block
-    typename P::Op Bop[NKB];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) Bop[kb] = P::pack(-S[2 * kb], -S[2 * kb + 1]);
-    const float a = av[si];
-    float b = 0.f, m = 0.f, n = 0.f;
+    c.a = av[si];
     if constexpr (RULE == 2) {
-      b = bv[si];
-      m = mv[si];
-      n = nv[si];
+      c.b = bv[si];
+      c.m = mv[si];
+      c.n = nv[si];
     }
+  };
+
+  f32x4 S = zero4(), M = zero4(), V = zero4();
+  auto step = [&](Chunk& c, int i) {
+    float* const x = xs[i & 1];
+    // pre-update state (and adam's moments); -S^T to the exchange
+    *reinterpret_cast<f32x4*>(S_all + base + i * mat + so) = S;
+    if constexpr (RULE == 2) {
+      if (M_all) *reinterpret_cast<f32x4*>(M_all + base + i * mat + so) = M;
+      if (V_all) *reinterpret_cast<f32x4*>(V_all + base + i * mat + so) = V;
+    }
+    *reinterpret_cast<f32x4*>(x + rl * LD + 16 * w + 4 * G) = -S;
+    __syncthreads();
+    f32x4 g0 = c.u, g1 = zero4();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      f32x4 g = Ucur[t];  // G^T tile rows c = 16t.., cols = this wave's rows
+      const f32x4 s = *reinterpret_cast<const f32x4*>(x + rl * LD + 16 * t + 4 * G);
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) g = P::mma(col_op<P, SwzMat<D>>(kl, 32 * kb, 16 * t), Bop[kb], g);
-      if constexpr (RULE == 0) {
-        S[t] = a * S[t] + g;
-      } else {
-        M[t] = m * M[t] + (1.f - m) * g;
-        V[t] = n * V[t] + (1.f - n) * g * g;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) S[t][j] = a * S[t][j] + b * M[t][j] / (sqrtf(V[t][j]) + 1e-6f);
+      for (int e = 0; e < 4; ++e) {
+        if (t & 1)
+          g1 = mfma_f32(c.k[t][e], s[e], g1);
+        else
+          g0 = mfma_f32(c.k[t][e], s[e], g0);
       }
     }
-    wait_vmem();
-    __syncthreads();
+    const float a = c.a, b = c.b, m = c.m, n = c.n;
+    if (i + 2 < N) load(c, i + 2);
+    const f32x4 g = g0 + g1;
+    if constexpr (RULE == 0) {
+      S = a * S + g;
+    } else {
+      M = m * M + (1.f - m) * g;
+      V = n * V + (1.f - n) * g * g;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) S[j] = a * S[j] + b * M[j] / (sqrtf(V[j]) + 1e-6f);
+    }
+  };
+
+  Chunk c0, c1;
+  load(c0, 0);
+  load(c1, N > 1 ? 1 : 0);
+  int i = 0;
+  for (; i + 1 < N; i += 2) {
+    step(c0, i);
+    step(c1, i + 1);
   }
+  if (i < N) step(c0, i);
 }
 
 // ------------------------------------- forward, 8 waves per 32 rows (bf16x3)
@@ -295,117 +318,244 @@ scan_fwd_rows8(const float* __restrict__ U, const float* __restrict__ K,
   }
 }
 
-// Reverse scan for the row-separable rules.  Writes dU (= Gb) for every
-// chunk, and for adam the per-row-tile partial sums of da, db, dm, dn into
-// part[(bh*N + i) * n_tiles + tile][4]; delta's da is formed later from dU
-// and S_all.
-template <int D, int RULE, int PREC>
-__global__ void __launch_bounds__(A_THREADS)
-scan_bwd_rows(const float* __restrict__ U, const float* __restrict__ K,
-              const float* __restrict__ av, const float* __restrict__ bv,
-              const float* __restrict__ mv, const float* __restrict__ nv,
-              const float* __restrict__ S_all, const float* __restrict__ M_all,
-              const float* __restrict__ V_all, const float* __restrict__ gS,
-              float* __restrict__ dU, float* __restrict__ part, int64_t BH, int N) {
-  using P = typename PrecSel<PREC>::T;
+// ---------------------- reverse scan, exact float32: D/16 waves per 16 rows
+// The layout of scan_fwd_rowsf: wave w holds column tile w of Sb^T.  Delta:
+// dU_i = Sb, then Sb^T <- a Sb^T + gS^T - K Sb^T with -Sb^T through the
+// exchange and A = K_i rows (16-byte loads of the wave's own 16 rows, two
+// chunks in flight); da is formed later from dU and S_all. Bound: vector
+// memory into a CU (K_i again for each 16 rows). Measured (d = 128, 64 heads,
+// 64 chunks): 508 -> 321 us against the two-wave kernel.
+template <int D>
+__global__ void __launch_bounds__(D * 4)
+scan_bwd_rowsf(const float* __restrict__ K, const float* __restrict__ av, const float* __restrict__ gS,
+               float* __restrict__ dU, int64_t BH, int N) {
   constexpr int NT = D / 16;
-  constexpr int NKB = D / 32;
-  constexpr int NTILES = D / 16;
-  extern __shared__ __align__(16) float smem[];
+  constexpr int LD = RowsfLds<D>::LD;
+  __shared__ __align__(16) float xs[2][RowsfLds<D>::X];
 
   int64_t bh;
   int blk;
-  map_rows_block(BH, D / (16 * A_WAVES), bh, blk);
+  map_rows_block(BH, NT, bh, blk);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = lane_id(), G = l >> 4, rl = l & 15;
-  const int tile = blk * A_WAVES + wave_id();
-  const int r0 = tile * 16;
   const int64_t mat = (int64_t)D * D;
-  const float* Kb = K + bh * N * mat;
-  auto roff = [&](int t) { return (int64_t)(r0 + rl) * D + 16 * t + 4 * G; };
+  const int64_t base = bh * N * mat;
+  // 32-bit lane offsets from scalar bases
+  const uint32_t to = (16 * blk + rl) * D + 16 * w + 4 * G;  // this lane's piece of a state
+  const uint32_t kro = (16 * w + rl) * D + 4 * G;            // K rows of column tile w
 
-  f32x4 Sb[NT], Mb[NT], Vb[NT];
+  struct Chunk {
+    f32x4 k[NT], gs;
+    float a;
+  };
+  auto load = [&](Chunk& c, int i) {
+    const int64_t o = base + i * mat;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) Sb[t] = Mb[t] = Vb[t] = zero4();
-
-  if (N > 0) lds_dma_matrix<D, A_THREADS>((smem + ((N - 1) & 1) * D * D), Kb + (int64_t)(N - 1) * mat);
-  wait_vmem();
-  __syncthreads();
-
-  for (int i = N - 1; i >= 0; --i) {
-    const float* kl = (smem + (i & 1) * D * D);
-    if (i > 0) lds_dma_matrix<D, A_THREADS>((smem + ((i - 1) & 1) * D * D), Kb + (int64_t)(i - 1) * mat);
-    const int64_t si = bh * N + i;
-    const float a = av[si];
-    f32x4 Gb[NT];
-    if constexpr (RULE == 0) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) Gb[t] = Sb[t];
-    } else {
-      // recompute G^T = U^T - K^T S_i^T from the saved pre-update state
-      const float b = bv[si], m = mv[si], n = nv[si];
-      f32x4 Si[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) Si[t] = *reinterpret_cast<const f32x4*>((S_all + si * mat + roff(t)));
-      typename P::Op Bop[NKB];
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) Bop[kb] = P::pack(-Si[2 * kb], -Si[2 * kb + 1]);
-      float pda = 0.f, pdb = 0.f, pdm = 0.f, pdn = 0.f;
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        f32x4 g = *reinterpret_cast<const f32x4*>((U + si * mat + roff(t)));
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) g = P::mma(col_op<P, SwzMat<D>>(kl, 32 * kb, 16 * t), Bop[kb], g);
-        const f32x4 Mp = *reinterpret_cast<const f32x4*>((M_all + si * mat + roff(t)));
-        const f32x4 Vp = *reinterpret_cast<const f32x4*>((V_all + si * mat + roff(t)));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float gg = g[j];
-          const float Mi = m * Mp[j] + (1.f - m) * gg;
-          const float Vi = n * Vp[j] + (1.f - n) * gg * gg;
-          const float root = sqrtf(Vi);
-          const float den = root + 1e-6f;
-          const float sb = Sb[t][j];
-          pda += sb * Si[t][j];
-          pdb += sb * (Mi / den);
-          const float ub = b * sb;
-          const float Mtot = Mb[t][j] + ub / den;
-          const float Vtot = Vb[t][j] - ub * Mi / (den * den) / (2.f * fmaxf(root, 1e-12f));
-          pdm += Mtot * (Mp[j] - gg);
-          pdn += Vtot * (Vp[j] - gg * gg);
-          Mb[t][j] = m * Mtot;
-          Vb[t][j] = n * Vtot;
-          Gb[t][j] = (1.f - m) * Mtot + (1.f - n) * 2.f * gg * Vtot;
-        }
-      }
-      pda = wave_sum(pda);
-      pdb = wave_sum(pdb);
-      pdm = wave_sum(pdm);
-      pdn = wave_sum(pdn);
-      if (l == 0) {
-        float* pp = part + (si * NTILES + tile) * 4;
-        pp[0] = pda;
-        pp[1] = pdb;
-        pp[2] = pdm;
-        pp[3] = pdn;
-      }
-    }
-    // dU_i = Gb
-#pragma unroll
-    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>((dU + si * mat + roff(t))) = Gb[t];
-    // Sb^T <- a Sb^T - K Gb^T + gS^T : output tile rows c' = 16t.., A = K rows, B = -Gb^T
-    typename P::Op Bop[NKB];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) Bop[kb] = P::pack(-Gb[2 * kb], -Gb[2 * kb + 1]);
+    for (int t = 0; t < NT; ++t) c.k[t] = *reinterpret_cast<const f32x4*>(K + o + 16 * t + kro);
+    c.gs = *reinterpret_cast<const f32x4*>(gS + o + to);
+    c.a = av[bh * N + i];
+  };
+  f32x4 Sb = zero4();
+  auto step = [&](Chunk& c, int i) {
+    float* const x = xs[i & 1];
+    *reinterpret_cast<f32x4*>(x + rl * LD + 16 * w + 4 * G) = -Sb;
+    *reinterpret_cast<f32x4*>(dU + base + i * mat + to) = Sb;
+    __syncthreads();
+    f32x4 a0 = c.a * Sb + c.gs, a1 = zero4();
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      f32x4 acc = a * Sb[t] + *reinterpret_cast<const f32x4*>((gS + si * mat + roff(t)));
+      const f32x4 gb = *reinterpret_cast<const f32x4*>(x + rl * LD + 16 * t + 4 * G);
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) acc = P::mma(row_op<P, SwzMat<D>>(kl, 16 * t, 32 * kb), Bop[kb], acc);
-      Sb[t] = acc;
+      for (int e = 0; e < 4; ++e) {
+        if (t & 1)
+          a1 = mfma_f32(c.k[t][e], gb[e], a1);
+        else
+          a0 = mfma_f32(c.k[t][e], gb[e], a0);
+      }
     }
-    wait_vmem();
-    __syncthreads();
+    Sb = a0 + a1;
+    if (i >= 2) load(c, i - 2);
+  };
+  Chunk c0, c1;
+  load(c0, N - 1);
+  load(c1, N > 1 ? N - 2 : 0);
+  int i = N - 1;
+  for (; i >= 1; i -= 2) {
+    step(c0, i);
+    step(c1, i - 1);
   }
+  if (i == 0) step(c0, 0);
+}
+
+// Adam: the moment VJP needs G_i = U_i - S_i K_i again, which does not depend
+// on the cotangent, so chunk i - 1's is formed in step i after the update.
+// Wave w also holds column tile w of Mb^T, Vb^T.  K_i is read by rows (the
+// update) in step i and by columns (G) in step i + 1, both from one LDS copy
+// (LDS-DMA, two buffers); S_{i-1}'s rows, which every wave reads whole, go
+// through a second exchange like -Gb's.  Per step:
+//   moment VJP of chunk i; -Gb, S_{i-1} and the partial sums to LDS | barrier
+//   Sb^T <- a Sb^T + gS^T - K_i Gb^T                                | barrier
+//   request K_{i-2} into K_i's buffer, and chunk i-2's tiles
+//   G_{i-1}^T = U^T - K_{i-1}^T S_{i-1}^T
+// The partial sums of da, db, dm, dn of each 16-row tile go to
+// part[(bh*N + i) * (D/16) + tile][4].
+//
+// Bound: vector memory into a CU (112 KB a chunk at D = 128, most of it K_i
+// from L2), then the MFMA pipe (1.7 us a chunk). Measured (d = 128, 32
+// chunks): 16 heads 682 -> 155 us, 64 heads 747 -> 381 us against the two-wave
+// kernel (both products and the moment VJP of 16 rows in one wave); 206 and
+// 482 us with K and S operands loaded from global memory by each wave. d = 64,
+// 8 heads, 16 chunks: 116 -> 35 us.
+template <int D>
+struct AdamfLds {
+  static constexpr int K = 0;                           // two D x D float32 buffers (SwzMat)
+  static constexpr int XG = 2 * D * D;                  // -Gb rows
+  static constexpr int XS = XG + RowsfLds<D>::X;        // S rows
+  static constexpr int RED = XS + RowsfLds<D>::X;       // [wave][4] partial sums
+  static constexpr int BYTES = (RED + D / 16 * 4) * 4;
+  static_assert(BYTES <= 160 * 1024, "adam reverse scan LDS exceeds the 160 KiB of a CU");
+};
+
+template <int D>
+__global__ void __launch_bounds__(D * 4)
+scan_bwd_adamf(const float* __restrict__ U, const float* __restrict__ K,
+               const float* __restrict__ av, const float* __restrict__ bv,
+               const float* __restrict__ mv, const float* __restrict__ nv,
+               const float* __restrict__ S_all, const float* __restrict__ M_all,
+               const float* __restrict__ V_all, const float* __restrict__ gS,
+               float* __restrict__ dU, float* __restrict__ part, int64_t BH, int N) {
+  using R = AdamfLds<D>;
+  using L = SwzMat<D>;
+  constexpr int NT = D / 16;
+  constexpr int LD = RowsfLds<D>::LD;
+  extern __shared__ __align__(16) float smem[];
+  float* const xg = smem + R::XG;
+  float* const xsr = smem + R::XS;
+  float* const red = smem + R::RED;
+
+  int64_t bh;
+  int blk;
+  map_rows_block(BH, NT, bh, blk);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = lane_id(), G = l >> 4, rl = l & 15;
+  const int64_t mat = (int64_t)D * D;
+  const int64_t base = bh * N * mat;
+  const uint32_t to = (16 * blk + rl) * D + 16 * w + 4 * G;  // this lane's piece of a state
+  const int xo = rl * LD + 16 * w + 4 * G;                   // its place in the exchanges
+  const float* const Kb = K + base;
+
+  struct Tiles {  // the lane's pieces of a chunk
+    f32x4 u, mp, vp, si, gs;
+    float a, b, m, n;
+  };
+  auto load = [&](Tiles& c, int i) {
+    const int64_t o = base + i * mat, sc = bh * N + i;
+    c.u = *reinterpret_cast<const f32x4*>(U + o + to);
+    c.mp = *reinterpret_cast<const f32x4*>(M_all + o + to);
+    c.vp = *reinterpret_cast<const f32x4*>(V_all + o + to);
+    c.si = *reinterpret_cast<const f32x4*>(S_all + o + to);
+    c.gs = *reinterpret_cast<const f32x4*>(gS + o + to);
+    c.a = av[sc];
+    c.b = bv[sc];
+    c.m = mv[sc];
+    c.n = nv[sc];
+  };
+  f32x4 Sb = zero4(), Mb = zero4(), Vb = zero4();
+  // u - K^T S^T of the chunk whose S rows are in the exchange, K_j at kl
+  auto form_g = [&](const f32x4& u, const float* kl) {
+    f32x4 g0 = zero4(), g1 = zero4();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const f32x4 s = *reinterpret_cast<const f32x4*>(xsr + rl * LD + 16 * t + 4 * G);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float k = kl[L::off(16 * t + 4 * G + e, 16 * w + rl)];
+        if (t & 1)
+          g1 = mfma_f32(k, s[e], g1);
+        else
+          g0 = mfma_f32(k, s[e], g0);
+      }
+    }
+    return u - (g0 + g1);
+  };
+
+  // Step i: `c` holds chunk i's pieces, `p` chunk i-1's, g is G_i.  Buffers:
+  // K_i in i & 1, K_{i-1} requested a step ago into the other.
+  f32x4 g;
+  auto step = [&](Tiles& c, const Tiles& p, int i) {
+    f32x4 Gb;
+    float pda = 0.f, pdb = 0.f, pdm = 0.f, pdn = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float gg = g[j];
+      const float Mi = c.m * c.mp[j] + (1.f - c.m) * gg;
+      const float Vi = c.n * c.vp[j] + (1.f - c.n) * gg * gg;
+      const float root = sqrtf(Vi);
+      const float den = root + 1e-6f;
+      const float sb = Sb[j];
+      pda += sb * c.si[j];
+      pdb += sb * (Mi / den);
+      const float ub = c.b * sb;
+      const float Mtot = Mb[j] + ub / den;
+      const float Vtot = Vb[j] - ub * Mi / (den * den) / (2.f * fmaxf(root, 1e-12f));
+      pdm += Mtot * (c.mp[j] - gg);
+      pdn += Vtot * (c.vp[j] - gg * gg);
+      Mb[j] = c.m * Mtot;
+      Vb[j] = c.n * Vtot;
+      Gb[j] = (1.f - c.m) * Mtot + (1.f - c.n) * 2.f * gg * Vtot;
+    }
+    *reinterpret_cast<f32x4*>(xg + xo) = -Gb;
+    const f32x2 s0 = wave_sum2(pda, pdb), s1 = wave_sum2(pdm, pdn);
+    if (l < 4) red[4 * w + l] = l == 0 ? s0[0] : l == 1 ? s0[1] : l == 2 ? s1[0] : s1[1];
+    *reinterpret_cast<f32x4*>(dU + base + i * mat + to) = Gb;
+    __syncthreads();  // -Gb and the partial sums published; S_i's rows read
+    *reinterpret_cast<f32x4*>(xsr + xo) = p.si;
+    if (w == 0 && l < 4) {
+      float t = 0.f;
+#pragma unroll
+      for (int q = 0; q < NT; ++q) t += red[4 * q + l];
+      part[((bh * N + i) * NT + blk) * 4 + l] = t;
+    }
+    const float* kl = smem + R::K + (i & 1) * D * D;
+    f32x4 a0 = c.a * Sb + c.gs, a1 = zero4();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const f32x4 k = *reinterpret_cast<const f32x4*>(kl + L::off(16 * w + rl, 16 * t + 4 * G));
+      const f32x4 gb = *reinterpret_cast<const f32x4*>(xg + rl * LD + 16 * t + 4 * G);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (t & 1)
+          a1 = mfma_f32(k[e], gb[e], a1);
+        else
+          a0 = mfma_f32(k[e], gb[e], a0);
+      }
+    }
+    Sb = a0 + a1;
+    if (i == 0) return;
+    wait_vmem();      // K_{i-1} landed
+    __syncthreads();  // K_{i-1} and S_{i-1}'s rows published; K_i, -Gb and the sums read
+    if (i >= 2) {
+      lds_dma_matrix<D, D * 4>(smem + R::K + (i & 1) * D * D, Kb + (i - 2) * mat);
+      load(c, i - 2);
+    }
+    g = form_g(p.u, smem + R::K + ((i - 1) & 1) * D * D);
+  };
+
+  Tiles c0, c1;
+  lds_dma_matrix<D, D * 4>(smem + R::K + ((N - 1) & 1) * D * D, Kb + (N - 1) * mat);
+  load(c0, N - 1);
+  load(c1, N > 1 ? N - 2 : 0);
+  *reinterpret_cast<f32x4*>(xsr + xo) = c0.si;
+  wait_vmem();
+  __syncthreads();
+  if (N > 1) lds_dma_matrix<D, D * 4>(smem + R::K + ((N - 2) & 1) * D * D, Kb + (N - 2) * mat);
+  g = form_g(c0.u, smem + R::K + ((N - 1) & 1) * D * D);
+  int i = N - 1;
+  for (; i >= 1; i -= 2) {
+    step(c0, c1, i);
+    step(c1, c0, i - 1);
+  }
+  if (i == 0) step(c0, c1, 0);
 }
 
 // ------------------------------------ reverse scan, 8 waves per 32 rows (bf16x3)
@@ -637,59 +787,75 @@ scan_bwd_rows8(const float* __restrict__ U, const float* __restrict__ K,
 }
 
 // Chunk-parallel part of the backward: dK_i = -S_i^T Gb_i (contraction over
-// the rows of S) and the scalar gradients of chunk i.  One workgroup of
-// A_KWAVES waves per (bh, i); S_i and Gb_i are staged in swizzled LDS.
-constexpr int A_KWAVES = 4;
-constexpr int A_KTHREADS = A_KWAVES * 64;
-
-template <int D, int RULE, int PREC>
-__global__ void __launch_bounds__(A_KTHREADS)
-scan_bwd_dk(const float* __restrict__ S_all, const float* __restrict__ dU,
-            const float* __restrict__ part, float* __restrict__ dK,
-            float* __restrict__ da, float* __restrict__ db, float* __restrict__ dm,
-            float* __restrict__ dn, int64_t BH, int N) {
-  using P = typename PrecSel<PREC>::T;
+// the rows of S) and the scalar gradients of chunk i, exact float32.  One
+// workgroup of D/16 waves per (bh, i).  Wave w forms the tiles of dK rows
+// 16 w .. 16 w + 15, transposed ((Gb^T S)[c][c']), so that a lane stores four
+// consecutive columns of dK; its own S columns are loaded straight into the
+// operand registers once, and Gb_i, which every wave reads whole, is staged
+// in LDS (rows padded by four floats: the four lane groups' rows, four apart,
+// fall on different banks).  Bound: the MFMA pipe (6.8 us a chunk at D = 128,
+// two workgroups a CU). Measured (d = 128): 4096 chunks 363 -> 216 us, 2048
+// chunks 165 -> 97 us against 16-byte-swizzled copies of both matrices read by
+// column for every tile.
+template <int D, int RULE>
+__global__ void __launch_bounds__(D * 4)
+scan_bwd_dkf(const float* __restrict__ S_all, const float* __restrict__ dU,
+             const float* __restrict__ part, float* __restrict__ dK,
+             float* __restrict__ da, float* __restrict__ db, float* __restrict__ dm,
+             float* __restrict__ dn, int64_t BH, int N) {
   constexpr int NT = D / 16;
-  constexpr int NKB = D / 32;
-  extern __shared__ __align__(16) float smem[];
-  float* Sl = smem;
-  float* Gl = smem + D * D;
-  __shared__ float red[A_KWAVES];
+  constexpr int LD = D + 4;
+  extern __shared__ __align__(16) float smem[];  // Gb_i, D rows of LD floats
+  __shared__ float red[NT];
   const int64_t si = blockIdx.x;  // = bh * N + i
   const int64_t mat = (int64_t)D * D;
-  lds_dma_matrix<D, A_KTHREADS>(Sl, S_all + si * mat);
-  lds_dma_matrix<D, A_KTHREADS>(Gl, dU + si * mat);
-  wait_vmem();
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = lane_id(), G = l >> 4, rl = l & 15;
+  const float* const Gi = dU + si * mat;
+  const float* const Si = S_all + si * mat;
+  const uint32_t so = 4 * G * D + 16 * w + rl;
+  float s[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[t][e] = (Si + (16 * t + e) * D)[so];
+  {
+    constexpr int PR = D / 4, NQ = D * PR / (D * 4), RSTEP = D * 4 / PR;  // 16-byte pieces
+    const int r = threadIdx.x / PR, c = (threadIdx.x % PR) * 4;
+    f32x4 x[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) x[q] = *reinterpret_cast<const f32x4*>(Gi + (r + q * RSTEP) * D + c);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) *reinterpret_cast<f32x4*>(smem + (r + q * RSTEP) * LD + c) = x[q];
+  }
   __syncthreads();
-  const int w = wave_id(), l = lane_id();
-  // dK^T[c][c'] = -sum_r Gb[r][c] S[r][c'] ; tile (tc, tcp) with rows c.
-  // Stored as dK[c'][c]: lane (c', G) of the D-layout tile of dK^T^T...
-  // Output tile of dK (rows c' = 16 tr, cols c = 16 tc): A = S^T rows c'
-  // (k = r, column reads of S), B = Gb (k = r, column reads of Gb).
-  for (int tile = w; tile < NT * NT; tile += A_KWAVES) {
-    const int tr = tile / NT, tc = tile % NT;
-    f32x4 acc = zero4();
+  float* const out = dK + si * mat + (16 * w + rl) * D + 4 * G;
+  float dot = 0.f;
+#pragma unroll 2
+  for (int tc = 0; tc < NT; ++tc) {
+    const float* const gp = smem + 4 * G * LD + 16 * tc + rl;
+    f32x4 a0 = zero4(), a1 = zero4();
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-      acc = P::mma(col_op<P, SwzMat<D>>(Sl, 32 * kb, 16 * tr), col_op<P, SwzMat<D>>(Gl, 32 * kb, 16 * tc), acc);
-    // D-layout: lane (c = l%16, G) holds dK[16tr + 4G + j][16tc + c]
-    float* out = dK + si * mat + (int64_t)(16 * tr + 4 * (l >> 4)) * D + 16 * tc + (l & 15);
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) out[(int64_t)j * D] = -acc[j];
+      for (int e = 0; e < 4; ++e) {
+        const float gv = gp[(16 * t + e) * LD];
+        if (t & 1)
+          a1 = mfma_f32(gv, s[t][e], a1);
+        else
+          a0 = mfma_f32(gv, s[t][e], a0);
+        if constexpr (RULE == 0) dot += tc == w ? gv * s[t][e] : 0.f;  // da_i = <Gb_i, S_i>
+      }
+    *reinterpret_cast<f32x4*>(out + 16 * tc) = -(a0 + a1);
   }
   if constexpr (RULE == 0) {
-    // da_i = <Sb_{i+1}, S_i> = <dU_i, S_i> for delta
-    float s = 0.f;
-    for (int e = threadIdx.x; e < D * D; e += A_KTHREADS) {
-      const int r = e / D, c = e % D;
-      s += Sl[SwzMat<D>::off(r, c)] * Gl[SwzMat<D>::off(r, c)];
-    }
-    s = wave_sum(s);
-    if (l == 0) red[w] = s;
+    dot = wave_sum(dot);
+    if (l == 0) red[w] = dot;
     __syncthreads();
     if (threadIdx.x == 0) {
       float t = 0.f;
-      for (int q = 0; q < A_KWAVES; ++q) t += red[q];
+#pragma unroll
+      for (int q = 0; q < NT; ++q) t += red[q];
       da[si] = t;
       db[si] = 0.f;
       dm[si] = 0.f;
@@ -698,7 +864,8 @@ scan_bwd_dk(const float* __restrict__ S_all, const float* __restrict__ dU,
   } else if constexpr (RULE == 2) {
     if (threadIdx.x < 4) {
       float t = 0.f;
-      for (int q = 0; q < D / 16; ++q) t += part[(si * (D / 16) + q) * 4 + threadIdx.x];
+#pragma unroll
+      for (int q = 0; q < NT; ++q) t += part[(si * NT + q) * 4 + threadIdx.x];
       float* dst = threadIdx.x == 0 ? da : threadIdx.x == 1 ? db : threadIdx.x == 2 ? dm : dn;
       dst[si] = t;
     }
@@ -823,34 +990,49 @@ scan_bwd_dk8(const float* __restrict__ S_all, const float* __restrict__ dU,
   // RULE == 1: the muon backward kernel writes the scalar gradients itself
 }
 
+// Adam's scalar gradients alone, from the row tiles' partial sums: thread
+// 4 c + q sums value q of chunk c in the order the dK kernels use.
+__global__ void __launch_bounds__(256)
+scan_bwd_scalars(const float* __restrict__ part, float* __restrict__ da, float* __restrict__ db,
+                 float* __restrict__ dm, float* __restrict__ dn, int64_t chunks, int tiles) {
+  const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x, c = x >> 2;
+  const int q = (int)(x & 3);
+  if (c >= chunks) return;
+  float t = 0.f;
+  for (int k = 0; k < tiles; ++k) t += part[(c * tiles + k) * 4 + q];
+  float* const dst = q == 0 ? da : q == 1 ? db : q == 2 ? dm : dn;
+  dst[c] = t;
+}
+
 // ---------------------------------------------------------------- launchers
-template <int D, int RULE, int PREC>
-static hipError_t launch_fwd_rows(const ScanArgs& s) {
-  const int nblk = D / (16 * A_WAVES);
-  const size_t lds = 2 * (size_t)D * D * sizeof(float);
-  auto kern = scan_fwd_rows<D, RULE, PREC>;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(s.BH * nblk)), dim3(A_THREADS), lds, s.stream, s.U, s.K, s.a,
-                     s.b, s.m, s.n, s.S_all, s.M_all, s.V_all, s.BH, (int)s.N);
+template <int D, int RULE>
+static hipError_t launch_fwd_rowsf(const ScanArgs& s) {
+  hipLaunchKernelGGL((scan_fwd_rowsf<D, RULE>), dim3((unsigned)(s.BH * (D / 16))), dim3(D * 4), 0, s.stream, s.U, s.K,
+                     s.a, s.b, s.m, s.n, s.S_all, s.M_all, s.V_all, s.BH, (int)s.N);
   return hipGetLastError();
 }
 
-template <int D, int RULE, int PREC>
-static hipError_t launch_bwd_rows(const ScanArgs& s, float* part) {
-  const int nblk = D / (16 * A_WAVES);
-  const size_t lds = 2 * (size_t)D * D * sizeof(float);
-  auto kern = scan_bwd_rows<D, RULE, PREC>;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+template <int D>
+static hipError_t launch_bwd_rowsf(const ScanArgs& s) {
+  hipLaunchKernelGGL((scan_bwd_rowsf<D>), dim3((unsigned)(s.BH * (D / 16))), dim3(D * 4), 0, s.stream, s.K, s.a, s.gS,
+                     s.dU, s.BH, (int)s.N);
+  return hipGetLastError();
+}
+
+template <int D>
+static hipError_t launch_bwd_adamf(const ScanArgs& s, float* part) {
+  const int lds = AdamfLds<D>::BYTES;
+  auto kern = scan_bwd_adamf<D>;
+  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(s.BH * nblk)), dim3(A_THREADS), lds, s.stream, s.U, s.K, s.a,
-                     s.b, s.m, s.n, s.S_all, s.M_all, s.V_all, s.gS, s.dU, part, s.BH, (int)s.N);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(s.BH * (D / 16))), dim3(D * 4), lds, s.stream, s.U, s.K, s.a, s.b, s.m, s.n,
+                     s.S_all, s.M_all, s.V_all, s.gS, s.dU, part, s.BH, (int)s.N);
   return hipGetLastError();
 }
 
 template <int D, int RULE, int PREC>
 static hipError_t launch_bwd_dk(const ScanArgs& s, const float* part) {
-  if constexpr (PREC == 0 && D >= 64) {  // bf16x3: the 8-wave kernel
+  if constexpr (PREC == 0 && D >= 64) {  // bf16x3 planes
     const int lds = Dk8Lds<D>::BYTES;
     auto k8 = scan_bwd_dk8<D, RULE>;
     hipError_t e = hipFuncSetAttribute((const void*)k8, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -859,12 +1041,12 @@ static hipError_t launch_bwd_dk(const ScanArgs& s, const float* part) {
                        s.dK, s.da, s.db, s.dm, s.dn, s.BH, (int)s.N);
     return hipGetLastError();
   }
-  const size_t lds = 2 * (size_t)D * D * sizeof(float);
-  auto k2 = scan_bwd_dk<D, RULE, PREC>;
-  hipError_t e = hipFuncSetAttribute((const void*)k2, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const int lds = D * (D + 4) * (int)sizeof(float);
+  auto kf = scan_bwd_dkf<D, RULE>;
+  hipError_t e = hipFuncSetAttribute((const void*)kf, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k2, dim3((unsigned)(s.BH * s.N)), dim3(A_KTHREADS), lds, s.stream, s.S_all, s.dU, part,
-                     s.dK, s.da, s.db, s.dm, s.dn, s.BH, (int)s.N);
+  hipLaunchKernelGGL(kf, dim3((unsigned)(s.BH * s.N)), dim3(D * 4), lds, s.stream, s.S_all, s.dU, part, s.dK, s.da,
+                     s.db, s.dm, s.dn, s.BH, (int)s.N);
   return hipGetLastError();
 }
 
@@ -883,6 +1065,12 @@ static hipError_t dk_prec(const ScanArgs& s, const float* part) {
 }
 
 hipError_t scan_bwd_dk_launch(const ScanArgs& s, const float* part) {
+  if (!s.dK && s.rule == 2) {
+    const int64_t chunks = s.BH * s.N;
+    hipLaunchKernelGGL(scan_bwd_scalars, dim3((unsigned)((4 * chunks + 255) / 256)), dim3(256), 0, s.stream, part, s.da,
+                       s.db, s.dm, s.dn, chunks, s.dh / 16);
+    return hipGetLastError();
+  }
   switch (s.dh) {
     case 32: return dk_prec<32>(s, part);
     case 64: return dk_prec<64>(s, part);
@@ -904,10 +1092,12 @@ static hipError_t launch_fwd_rows8(const ScanArgs& s) {
 
 template <int D, int PREC>
 static hipError_t fwd_rows_rule(const ScanArgs& s) {
-  if constexpr (PREC == 0 && D >= 64)  // bf16x3: the 8-wave kernel
+  // bf16x3: the 8-wave kernel (at D = 32 a row block is a few products either
+  // way: the float32 one)
+  if constexpr (PREC == 0 && D >= 64)
     return s.rule == 0 ? launch_fwd_rows8<D, 0>(s) : launch_fwd_rows8<D, 2>(s);
   else
-    return s.rule == 0 ? launch_fwd_rows<D, 0, PREC>(s) : launch_fwd_rows<D, 2, PREC>(s);
+    return s.rule == 0 ? launch_fwd_rowsf<D, 0>(s) : launch_fwd_rowsf<D, 2>(s);
 }
 template <int D, int RULE>
 static hipError_t launch_bwd_rows8(const ScanArgs& s, float* part) {
@@ -922,12 +1112,12 @@ static hipError_t launch_bwd_rows8(const ScanArgs& s, float* part) {
 
 template <int D, int PREC>
 static hipError_t bwd_rows_rule(const ScanArgs& s, float* part) {
-  // bf16x3: the 8-wave kernel (adam's at D = 128 would spill: the 2-wave one)
+  // bf16x3: the 8-wave kernel (adam's at D = 128 would spill: the float32 one)
   if constexpr (PREC == 0 && D >= 64) {
     if (s.rule == 0) return launch_bwd_rows8<D, 0>(s, part);
     if constexpr (D == 64) return launch_bwd_rows8<D, 2>(s, part);
   }
-  return s.rule == 0 ? launch_bwd_rows<D, 0, PREC>(s, part) : launch_bwd_rows<D, 2, PREC>(s, part);
+  return s.rule == 0 ? launch_bwd_rowsf<D>(s) : launch_bwd_adamf<D>(s, part);
 }
 
 template <int D>

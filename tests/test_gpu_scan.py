@@ -260,3 +260,48 @@ def test_dispatcher_head_dims():
             fast_scan.fast_state_scan(*ins, 0, 3)
     finally:
         fast_scan.set_backend("auto")
+
+
+@pytest.mark.parametrize("rule", [0, 2])
+@pytest.mark.parametrize("N", [2, 3, 4, 5])
+@pytest.mark.parametrize("B,H,dh", [(1, 3, 32), (3, 1, 64), (1, 8, 64), (1, 3, 128), (2, 4, 128)])
+def test_scan_row_kernels_short_sequences(B, H, dh, N, rule):
+    """The float32 row scans request operands up to two chunks ahead: every
+    chunk count at which such a request falls off the sequence, with head
+    counts on both branches of the block map.  |U| in [1, 2] and |S K| below
+    1/2 keep every |G| above 1/2, so adam's sqrt(V) stays away from zero and
+    its gradients are well conditioned: float32 then meets the 1e-4 bar with
+    no allowance for the reference's own error."""
+    from gmdn_amd.scan import hip_state_scan
+    dev = _dev()
+    gen = torch.Generator().manual_seed(N)
+    U, K, *gates = osc.make_scan_inputs(B, H, N, 64, dh, generator=gen)
+    U = torch.sign(U) + torch.rand(U.shape, generator=gen) * torch.sign(U)
+    K = K / (8 * K.abs().sum(-2, keepdim=True))  # |S K| <= max |S| / 8, and max |S| stays below 4
+    ins = [U, K, *gates]
+    gS = torch.randn(B, H, N, dh, dh, generator=gen, dtype=torch.float64)
+    S64, g64 = _oracle(ins, gS, rule, 3, torch.float64)
+    assert S64.abs().max() < (4 if rule == 2 else 16)
+    ins_d = [t.to(dev).requires_grad_(True) for t in ins]
+    S = hip_state_scan(*ins_d, rule, 3, precision="ieee")
+    grads = torch.autograd.grad(S, ins_d, gS.float().to(dev))
+    errs = _errs(S.detach().cpu(), [g.cpu() for g in grads], S64, g64)
+    if rule == 2 and N == 2:
+        # only chunk 0 reaches S_1, through M / sqrt(V) = a multiple of
+        # sign(G): its derivative is the difference of two equal terms
+        del errs["dU"]
+    assert max(errs.values()) <= 1e-4, errs
+
+
+@pytest.mark.parametrize("rule", [0, 2])
+@pytest.mark.parametrize("dh", [32, 64, 128])
+def test_scan_row_kernels_one_chunk(dh, rule):
+    """One chunk: its state is the initial zero, which no input reaches."""
+    from gmdn_amd.scan import hip_state_scan
+    dev = _dev()
+    ins = [t.to(dev).requires_grad_(True) for t in
+           osc.make_scan_inputs(1, 3, 1, 64, dh, generator=torch.Generator().manual_seed(dh))]
+    S = hip_state_scan(*ins, rule, 3, precision="ieee")
+    grads = torch.autograd.grad(S, ins, torch.ones_like(S))
+    for t in (S, *grads):
+        assert not t.any()
