@@ -137,6 +137,8 @@ hipError_t chunk_bwd_pair_launch(const ChunkArgs& a, int d, hipStream_t s);
 // backward's own workspace.
 size_t chunk_f32_states_floats(int64_t BH, int64_t N, int d, int rule);
 size_t chunk_f32_bwd_ws_floats(int64_t BH, int64_t N, int d, int rule, int ns);
+// smallest accepted (muon: one chunk's iterates recomputed at a time)
+size_t chunk_f32_bwd_min_ws_floats(int64_t BH, int64_t N, int d, int rule, int ns);
 hipError_t chunk_fwd_f32_launch(const ChunkArgs& a, int d, int rule, int ns, float* states, hipStream_t s);
 hipError_t chunk_bwd_f32_launch(const ChunkArgs& a, int d, int rule, int ns, const float* states, float* ws,
                                 size_t ws_floats, hipStream_t s);

@@ -725,10 +725,12 @@ int gmdn_chunk_bwd(const gmdn_chunk_desc* desc, const void* q, const void* k, co
   if (desc->rule == 2 && (desc->d == 128 || desc->dtype == GMDN_DTYPE_F32) && desc->eps != 1e-6f)
     return GMDN_ERR_UNSUPPORTED;
   if (desc->B * desc->H * (desc->T / CB_C) >= ((int64_t)1 << 31)) return GMDN_ERR_ARG;  // one workgroup per chunk
+  const int64_t BH = desc->B * desc->H, N = desc->T / CB_C;
   const bool bf16_rows = desc->dtype != GMDN_DTYPE_F32 && !(desc->rule == 2 && desc->d == 128);
   const size_t min_ws = desc->rule == 1 && desc->dtype != GMDN_DTYPE_F32 && desc->precision == GMDN_PREC_TF32
-                            ? chunk_bwd_muon_min_ws_floats(desc->B * desc->H, desc->T / CB_C, desc->d, desc->ns) *
-                                  sizeof(float)
+                            ? chunk_bwd_muon_min_ws_floats(BH, N, desc->d, desc->ns) * sizeof(float)
+                        : desc->dtype == GMDN_DTYPE_F32
+                            ? chunk_f32_bwd_min_ws_floats(BH, N, desc->d, desc->rule, desc->ns) * sizeof(float)
                         : desc->rule != 1 && bf16_rows ? chunk_bwd_min_ws_bytes(desc)
                                                        : gmdn_chunk_bwd_workspace_bytes(desc);
   if (!workspace || workspace_bytes < min_ws) return GMDN_ERR_WORKSPACE;

@@ -600,8 +600,13 @@ size_t chunk_f32_bwd_ws_floats(int64_t BH, int64_t N, int d, int rule, int ns) {
   const int64_t BHN = BH * N, mat = (int64_t)d * d;
   int64_t scan = 0;
   if (rule == 2) scan = BHN * (d / 16) * 4;
-  if (rule == 1) scan = BH * muon_bwd_ws_floats(d, ns);
+  if (rule == 1) scan = muon_bwd_ws_total(BH, N, d, ns);
   return (size_t)(3 * BHN * mat + 4 * BHN + scan);
+}
+
+size_t chunk_f32_bwd_min_ws_floats(int64_t BH, int64_t N, int d, int rule, int ns) {
+  if (rule != 1) return chunk_f32_bwd_ws_floats(BH, N, d, rule, ns);
+  return (size_t)(3 * BH * N * (int64_t)d * d + 4 * BH * N + BH * muon_bwd_ws_floats(d, ns));
 }
 
 hipError_t chunk_fwd_f32_launch(const ChunkArgs& a, int d, int rule, int ns, float* states, hipStream_t s) {

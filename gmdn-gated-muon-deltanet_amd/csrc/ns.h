@@ -37,6 +37,20 @@ GMDN_DEV float block_sum(float x, float* red) {
   return t;
 }
 
+// Largest value of the block (x >= 0); red as for block_sum.
+template <int NW>
+GMDN_DEV float block_max(float x, float* red) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
+  if (lane_id() == 0) red[wave_id()] = x;
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int q = 0; q < NW; ++q) t = fmaxf(t, red[q]);
+  __syncthreads();
+  return t;
+}
+
 // block_sum of two values under one pair of barriers (red: 2 NW floats); each
 // sum is formed in the order block_sum uses
 template <int NW>
@@ -170,9 +184,27 @@ struct NSBlock {
   }
 };
 
-// The forward quintic step with bf16x3 products and the shared matrices kept
-// as split bf16 planes in LDS (hi plane then lo plane, each D x D in the
-// 16-byte-group XOR swizzle RowSwz).  Within every 32 columns
+// Scales of a half-piece Newton-Schulz step.  X_0 = M / (|M| + eps) has
+// Frobenius norm x0 <= 1 (below 1/2 only when |M| is not far above eps), and
+// a step grows its singular values at most 3.4445-fold up to about 1.2, so
+// entries of X_k are at most min(1.3, x0 4^k): e_k = max(0, e_0 - 2 k) spare
+// binary places, e_0 = -log2 x0 (at most 24).  Then |X| 2^(12 + e) <= 5400,
+// |P| 2^(12 + 2e) <= 8000 and |Z| = |b P + c P^2| <= 3.5 at 2^(12 + 2e) stay
+// below half's 65504, with the low pieces of typical entries normal numbers.
+struct NSScale {
+  float x, p, z;
+  GMDN_DEV NSScale(float x0, int k) {
+    int e = x0 > 0.f && x0 < 0.5f ? -ilogbf(x0) - 1 : 0;
+    e = (e < 24 ? e : 24) - 2 * k;
+    e = e > 0 ? e : 0;
+    x = ldexpf(1.f, 12 + e);
+    p = z = ldexpf(1.f, 12 + 2 * e);
+  }
+};
+
+// The forward quintic step with split products and the shared matrices kept
+// as split planes in LDS (bf16 pieces, or half pieces of scaled values; hi
+// plane then lo plane, each D x D in the 16-byte-group XOR swizzle RowSwz).  Within every 32 columns
 // the 4-column blocks are stored in the order 0 4 1 5 2 6 3 7, so the eight
 // values of a row operand in the pair k order of the register operands
 // (columns 4G .. 4G+3 and 16+4G .. 16+4G+3) are one 16-byte row read per
@@ -180,7 +212,7 @@ struct NSBlock {
 // publishing wave splits its own rows once.  A row's swizzle depends only on
 // the row modulo 16, so each lane keeps one LDS base per distinct column
 // pattern and row tiles are immediate offsets.
-template <int D>
+template <int D, class P_ = PrecX3>
 struct NSSplit {
   static constexpr int NT = D / 16;
   static constexpr int NKB = D / 32;
@@ -188,8 +220,8 @@ struct NSSplit {
   static constexpr uint32_t BYTES = 2 * PLANE;             // one published matrix
   static constexpr uint32_t ROWB = D * 2;                  // bytes per row of a plane
   using L = RowSwz<D>;
-  using P = PrecX3;
-  using Op = P::Op;
+  using P = P_;  // PrecX3 (bf16 pieces) or PrecH (half pieces of scaled values)
+  using Op = typename P::Op;
   static_assert(L::MASK < 16, "row tiles of 16 must keep the swizzle");
 
   uint32_t prow[NKB];  // row reads: row lc, columns 32 kb + {4G .. 4G+3, 16+4G .. 16+4G+3}
@@ -237,7 +269,7 @@ struct NSSplit {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       bf16x4 hi, lo;
-      split4(x[q], hi, lo);
+      P::split(x[q], hi, lo);
       lds_st<bf16x4>(m + (dst + q * RSTEP * ROWB), hi);
       lds_st<bf16x4>(m + (dst + q * RSTEP * ROWB + PLANE), lo);
     }
@@ -250,8 +282,8 @@ struct NSSplit {
 #pragma unroll
     for (int c = 0; c < NT; c += 2) {
       bf16x4 h0, l0, h1, l1;
-      split4(t[c], h0, l0);
-      split4(t[c + 1], h1, l1);
+      P::split(t[c], h0, l0);
+      P::split(t[c + 1], h1, l1);
       const bf16x8 hi = cat8(h0, h1), lo = cat8(l0, l1);
       lds_st<bf16x8>(m + ppub[c], hi);
       lds_st<bf16x8>(m + (ppub[c] + PLANE), lo);
@@ -367,7 +399,11 @@ struct NSSplit {
   static GMDN_DEV void store_own(float* g, const f32x4 (&t)[NT]) {
     const int l = lane_id(), row = 16 * wave_id() + (l & 15);
 #pragma unroll
-    for (int c = 0; c < NT; ++c) *reinterpret_cast<bf16x8*>(g + row * D + 16 * c + 4 * (l >> 4)) = split_piece(t[c]);
+    for (int c = 0; c < NT; ++c) {
+      bf16x4 hi, lo;
+      P::split(t[c], hi, lo);
+      *reinterpret_cast<bf16x8*>(g + row * D + 16 * c + 4 * (l >> 4)) = cat8(hi, lo);
+    }
   }
   // operands of the wave's rows from pieces already loaded by load_pieces
   // (register moves only: placed right before their product, they do not
@@ -399,9 +435,7 @@ struct NSSplit {
   }
   static GMDN_DEV f32x4 tview(lds_cptr m, uint32_t tb, int tr) {
     const lds_cptr a = m + tb + tr * 16 * ROWB;
-    const bf16x4 h = lds_tr16(a), o = lds_tr16(a + PLANE);
-    return f32x4{(float)h[0] + (float)o[0], (float)h[1] + (float)o[1], (float)h[2] + (float)o[2],
-                 (float)h[3] + (float)o[3]};
+    return P::join(lds_tr16(a), lds_tr16(a + PLANE));
   }
   // One quintic step on the wave's rows XT (D-layout tiles of X^T); the same
   // products as NSBlock::step.  With zst / pst, Z = b P + c P^2 and P = X X^T
@@ -434,6 +468,45 @@ struct NSSplit {
 #pragma unroll
     for (int tc = 0; tc < NT; ++tc) XT[tc] = NS_A * XT[tc];
     colprod_all(XM, Bz, XT);
+    __syncthreads();
+  }
+
+  GMDN_DEV static void scale_all(f32x4 (&t)[NT], float s) {
+#pragma unroll
+    for (int c = 0; c < NT; ++c) t[c] = s * t[c];
+  }
+  // The step on half pieces (PrecH).  X, P and Z enter the products as
+  // sc.x X, sc.p P, sc.z Z (NSScale): power-of-two factors, so scaling and
+  // unscaling are exact, and XT stays unscaled between the steps.  xst: X
+  // itself as the wave's rows in pieces of sc.x X.
+  GMDN_DEV void step_scaled(f32x4 (&XT)[NT], lds_ptr XM, lds_ptr PM, const NSScale& sc, float* xst = nullptr,
+                            float* zst = nullptr, float* pst = nullptr) const {
+    scale_all(XT, sc.x);
+    publish(XM, XT);
+    if (xst) store_own(xst, XT);
+    __syncthreads();
+    Op Bx[NKB];
+    pack_all(XT, Bx);
+    f32x4 Pc[NT];
+#pragma unroll
+    for (int tr = 0; tr < NT; ++tr) Pc[tr] = zero4();
+    rowprod_all(XM, Bx, Pc);
+    scale_all(Pc, sc.p / (sc.x * sc.x));
+    publish(PM, Pc);
+    if (pst) store_own(pst, Pc);
+    __syncthreads();
+    Op Bp[NKB];
+    pack_all(Pc, Bp);
+    // c ((b / c) P + P^2) in units of sc.p^2, then of sc.z
+    scale_all(Pc, (NS_B / NS_C) * sc.p);
+    rowprod_all(PM, Bp, Pc);
+    scale_all(Pc, NS_C * (sc.z / (sc.p * sc.p)));
+    if (zst) store_own(zst, Pc);
+    Op Bz[NKB];
+    pack_all(Pc, Bz);
+    scale_all(XT, NS_A * sc.z);
+    colprod_all(XM, Bz, XT);
+    scale_all(XT, 1.f / (sc.x * sc.z));
     __syncthreads();
   }
 };

@@ -4,15 +4,24 @@
 // M (D-layout tiles of the transposes) and the waves cooperate on the
 // Newton-Schulz iterations through shared matrices.
 //
-// Forward: X and P live in LDS (2 D^2 fp32 worth): as split bf16 planes for
-// the bf16x3 precision, as swizzled fp32 for the exact one; K_i is read
-// straight from global memory (it is used once per chunk).
-// Backward with fp32 products (precision 'ieee'): X_k, P, Xbar and Bbar
-// (4 D^2) exceed LDS at D = 128, so they live in a per-(b, h) global workspace
-// (L2 resident), followed by the ns stored iterates X_0 .. X_{ns-1} (written
-// and re-read by the same lanes).  The bf16x3 backward's stages (iterate
-// rebuild, serial reverse scan) are in muon_bwd.h; scan_bwd_muon_seg runs
-// them a segment at a time.
+// Forward: X and P live in LDS as split planes of the Newton-Schulz engine
+// (NSSplit): bf16 pieces for 'tf32', half pieces of scaled values for 'ieee'
+// at D >= 64.  ('ieee' at D = 32, which serves d = 16 too, keeps exact float32
+// products, NSBlock: sums that short round so little in float32 that the
+// pieces' 2^-23 shows, 1.5 times its error at d = 16 where D >= 64 measures
+// 0.7 to 1.0 times.)
+// K_i is staged in the P store before the first step publishes P: split
+// planes ('tf32'), or float32 for exact products ('ieee').
+// Backward: the stages of muon_bwd.h (iterate rebuild, serial reverse scan)
+// in either precision; scan_bwd_muon_seg runs them a segment at a time.  An
+// 'ieee' caller whose workspace holds less than one chunk's iterates (4 + ns
+// matrices per (b, h) are accepted), and D = 32, get scan_bwd_muon: exact
+// float32 products through four matrices in that workspace.
+// 'ieee' measured (8 heads, 8 chunks, d = 128, ns = 3): forward 946 -> 333 us,
+// backward 10.1 ms -> 0.58 ms against float32 MFMAs (1/16 of the half rate)
+// through a global workspace; error against float64 0.55 to 1.0 times the
+// float32 products' (the 32-term half MFMA rounds its sum once, eight
+// float32 MFMAs eight times).
 #include "muon_bwd.h"
 #include "ns.h"
 #include "scan_a.h"
@@ -27,12 +36,10 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
               const float* __restrict__ av, const float* __restrict__ bv,
               const float* __restrict__ mv, float* __restrict__ S_all,
               float* __restrict__ M_all, int N, int ns) {
-  using P = typename PrecSel<PREC>::T;
+  using P = typename PrecSel<PREC>::T;                          // products with K_i
+  using NSX = NSSplit<D, std::conditional_t<PREC == 0, PrecX3, PrecH>>;  // Newton-Schulz products
   constexpr int NT = D / 16, NKB = D / 32, NW = D / 16;
-  using NS = NSBlock<P, SwzMat<D>, D>;
   extern __shared__ __align__(16) float smem[];
-  float* XM = smem;
-  float* PM = smem + D * D;
   __shared__ float red[NW];
 
   const int64_t bh = blockIdx.x;
@@ -44,11 +51,18 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
   f32x4 S[NT], M[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) S[t] = M[t] = zero4();
-  const NSSplit<D> nsx;  // per-lane LDS bases of the bf16x3 engine
+  const NSX nsx;  // per-lane LDS bases of the engine
+  const lds_ptr base = lds_base(smem), KP = base + NSX::BYTES;
+  float* const KF = smem + NSX::BYTES / 4;
 
   for (int i = 0; i < N; ++i) {
     const int64_t si = bh * N + i;
     const float* Ki = K + si * mat;
+    // K_i into the P store (free until the first NS step publishes P)
+    if constexpr (PREC == 0)
+      NSX::template stage<D * 4>(KP, Ki);
+    else
+      lds_dma_matrix<D, D * 4>(KF, Ki);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       *reinterpret_cast<f32x4*>((S_all + si * mat + roff(t))) = S[t];
@@ -58,12 +72,8 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) Bop[kb] = P::pack(-S[2 * kb], -S[2 * kb + 1]);
     const float a = av[si], b = bv[si], m = mv[si];
-    if constexpr (PREC == 0) {
-      // K_i as split planes in the P store (free until the first NS step
-      // publishes P), read back as column operands
-      NSSplit<D>::template stage<D * 4>(lds_base(smem) + NSSplit<D>::BYTES, Ki);
-      __syncthreads();
-    }
+    if constexpr (PREC != 0) wait_vmem();
+    __syncthreads();
     float sq = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -71,29 +81,33 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) {
         if constexpr (PREC == 0)
-          g = P::mma(nsx.col(lds_base(smem) + NSSplit<D>::BYTES, kb, t), Bop[kb], g);
+          g = P::mma(nsx.col(KP, kb, t), Bop[kb], g);
         else
-          g = P::mma(col_op<P, PlainMat<D>>(Ki, 32 * kb, 16 * t), Bop[kb], g);
+          g = P::mma(col_op<P, SwzMat<D>>(KF, 32 * kb, 16 * t), Bop[kb], g);
       }
+      if constexpr (PREC != 0) __builtin_amdgcn_sched_barrier(0);  // a tile's operands at a time
       M[t] = m * M[t] + g;
       sq += M[t][0] * M[t][0] + M[t][1] * M[t][1] + M[t][2] * M[t][2] + M[t][3] * M[t][3];
     }
-    const float scale = 1.f / (sqrtf(block_sum<NW>(sq, red)) + 1e-7f);
+    const float nf = sqrtf(block_sum<NW>(sq, red));
+    const float scale = 1.f / (nf + 1e-7f);
     f32x4 X[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) X[t] = M[t] * scale;
     if constexpr (PREC == 0) {
-      const lds_ptr base = lds_base(smem);
-      for (int s = 0; s < ns; ++s) nsx.step(X, base, base + NSSplit<D>::BYTES);
+      for (int s = 0; s < ns; ++s) nsx.step(X, base, KP);
+    } else if constexpr (D == 32) {
+      for (int s = 0; s < ns; ++s) NSBlock<PrecF32, SwzMat<D>, D>::step(X, smem, KF);
     } else {
-      for (int s = 0; s < ns; ++s) NS::step(X, XM, PM);
+      for (int s = 0; s < ns; ++s) nsx.step_scaled(X, base, KP, NSScale(nf * scale, s));
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t) S[t] = a * S[t] + b * X[t];
+    if (ns == 0) __syncthreads();  // K_i read before the next chunk's copy (a step ends with a barrier)
   }
 }
 
-template <int D, int PREC>
+template <int D>
 __global__ void __launch_bounds__(D * 4)
 scan_bwd_muon(const float* __restrict__ U, const float* __restrict__ K,
               const float* __restrict__ av, const float* __restrict__ bv,
@@ -102,7 +116,7 @@ scan_bwd_muon(const float* __restrict__ U, const float* __restrict__ K,
               float* __restrict__ dU, float* __restrict__ da, float* __restrict__ db,
               float* __restrict__ dm, float* __restrict__ dn, float* __restrict__ ws, int N,
               int ns) {
-  using P = typename PrecSel<PREC>::T;
+  using P = PrecF32;
   constexpr int NT = D / 16, NKB = D / 32, NW = D / 16;
   using NS = NSBlock<P, PlainMat<D>, D>;
   __shared__ float red[NW];
@@ -219,13 +233,13 @@ scan_bwd_muon(const float* __restrict__ U, const float* __restrict__ K,
 
 // Blocks 0 .. nx3 - 1: the reverse pass of their head over segment [i0, i1);
 // the rest: the iterates of one chunk of segment [j0, j0 + jcur) each.
-template <int D>
+template <int D, class P>
 __global__ void __launch_bounds__(D * 4) scan_bwd_muon_seg(MuonSegArgs sa) {
   const int64_t b = blockIdx.x;
   if (b < sa.nx3)
-    muon_x3_body<D>(sa, b);
+    muon_x3_body<D, P>(sa, b);
   else
-    muon_pre_body<D>(sa, b - sa.nx3);
+    muon_pre_body<D, P>(sa, b - sa.nx3);
 }
 
 template <int D, int PREC>
@@ -241,9 +255,11 @@ static hipError_t launch_fwd_muon(const ScanArgs& s) {
 
 template <int D, int PREC>
 static hipError_t launch_bwd_muon(const ScanArgs& s, float* ws, int64_t ws_floats) {
-  if constexpr (PREC == 0) {
+  const MuonBwdPlan plan = muon_bwd_plan(s.BH, s.N, D, s.ns, ws_floats);
+  if (PREC == 0 || (D >= 64 && plan.nseg >= 1)) {
+    using P = std::conditional_t<PREC == 0, PrecX3, PrecH>;
     const int lds = 2 * NSSplit<D>::BYTES + 64;
-    auto k = scan_bwd_muon_seg<D>;
+    auto k = scan_bwd_muon_seg<D, P>;
     hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return e;
     // Segments of nseg chunks from the end; Sb and Mbar carry from one
@@ -251,7 +267,6 @@ static hipError_t launch_bwd_muon(const ScanArgs& s, float* ws, int64_t ws_float
     // iterate buffers the iterates of segment k + 1 are formed in the launch
     // that runs segment k's reverse pass (only the first segment's run
     // alone); with one, each segment's iterates and then its reverse pass.
-    const MuonBwdPlan plan = muon_bwd_plan(s.BH, s.N, D, s.ns, ws_floats);
     if (plan.nseg < 1) return hipErrorInvalidValue;
     const int nseg = (int)plan.nseg;
     MuonSegArgs sa{};
@@ -283,7 +298,7 @@ static hipError_t launch_bwd_muon(const ScanArgs& s, float* ws, int64_t ws_float
     }
     return e;
   } else {
-    auto kern = scan_bwd_muon<D, PREC>;
+    auto kern = scan_bwd_muon<D>;
     hipLaunchKernelGGL(kern, dim3((unsigned)s.BH), dim3(D * 4), 0, s.stream, s.U, s.K, s.a, s.b, s.m,
                        s.S_all, s.M_all, s.gS, s.dU, s.da, s.db, s.dm, s.dn, ws, (int)s.N, s.ns);
     return hipGetLastError();

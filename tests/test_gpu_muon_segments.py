@@ -162,3 +162,56 @@ def test_fused_adam_backward_segments_bit_identical(N):
     got = run(full)
     for name, g_, w_ in zip("dq dk dv dbeta dg dgmu dgnu".split(), got, want):
         assert torch.equal(g_, w_), name
+
+
+def _bwd_ieee(lib, ins, S_all, M_all, gS, ns, ws_bytes):
+    B, H, N, dh, _ = ins[0].shape
+    outs = [torch.full_like(t, float("nan")) for t in (ins[0], ins[0], ins[2], ins[2], ins[2], ins[2])]
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=ins[0].device)
+    args = [nat.ptr(t) for t in ins] + [nat.ptr(S_all), nat.ptr(M_all), None, nat.ptr(gS)] + [nat.ptr(t) for t in outs]
+    rc = lib.gmdn_scan_bwd(*args, nat.ptr(ws), ws_bytes, B * H, N, dh, 1, ns, nat.PREC_IEEE, nat.stream_of(ins[0]))
+    nat.check(rc, "gmdn_scan_bwd")
+    torch.cuda.synchronize()
+    return outs
+
+
+@pytest.mark.parametrize("gscale", [1.0, 1e-25, 1e12])
+@pytest.mark.parametrize("N,dh,ns", [(5, 64, 3), (4, 128, 5), (3, 128, 0), (3, 64, 8), (4, 32, 5)])
+def test_muon_backward_ieee_workspaces(N, dh, ns, gscale):
+    """'ieee': segments give the default workspace's bits, and the smallest
+    accepted workspace (4 + ns matrices per head: exact float32 products
+    throughout) the same gradients to float32 accuracy at any scale of the
+    cotangent -- both within 2e-4 of each other relative to the largest entry,
+    four times the largest float32 error of this shape (ns = 8 amplifies
+    rounding by up to 3.4445^8 in small singular directions: 1e-2 there)."""
+    dev = _dev()
+    lib = nat.load()
+    B, H = 1, 2
+    gen = torch.Generator().manual_seed(N * 10 + dh)
+    ins = [t.to(dev).float().contiguous() for t in osc.make_scan_inputs(B, H, N, 64, dh, generator=gen)]
+    gS = gscale * torch.randn(B, H, N, dh, dh, generator=gen).to(dev)
+    S_all, M_all, _ = torch.ops.gmdn.state_scan(*ins, 1, ns, nat.PREC_IEEE, True)
+    want = _bwd_ieee(lib, ins, S_all, M_all, gS, ns, lib.gmdn_scan_bwd_workspace_bytes(B * H, N, dh, 1, ns))
+    assert all(torch.isfinite(t).all() for t in want)
+    for nseg in (1, 2, 3):
+        got = _bwd_ieee(lib, ins, S_all, M_all, gS, ns, _segment_bytes(B * H, nseg, dh, ns))
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), nseg
+    small = _bwd_ieee(lib, ins, S_all, M_all, gS, ns, 4 * B * H * (4 + ns) * dh * dh)
+    for name, a, b in zip("dU dK da db dm".split(), small, want):
+        assert osc.rel_err(a.cpu(), b.cpu()) <= (1e-2 if ns == 8 else 2e-4), name
+
+
+@pytest.mark.parametrize("vscale", [1e-9, 1e6])
+@pytest.mark.parametrize("dh", [64, 128])
+def test_muon_scan_ieee_scales(dh, vscale):
+    """Momentum far from one in either direction: X_0 = M / (|M| + 1e-7) is
+    small below the epsilon and of unit norm above.  Against float64 within
+    the 'ieee' bar, 1e-4 or twice the float32 reference's own error."""
+    from gmdn_amd.scan import hip_state_scan
+    dev = _dev()
+    U, *rest = osc.make_scan_inputs(1, 2, 4, 64, dh, generator=torch.Generator().manual_seed(dh))
+    ins = [U * vscale, *rest]
+    got = hip_state_scan(*[t.to(dev) for t in ins], 1, 3, precision="ieee").cpu()
+    want = osc.scan_forward(*[t.double() for t in ins], 1, 3)
+    floor = osc.rel_err(osc.scan_forward(*ins, 1, 3), want)
+    assert osc.rel_err(got, want) <= max(1e-4, 2 * floor)
