@@ -27,9 +27,17 @@
 //   dg_t = da a [g_t >= log 1e-6],  dgmu_t = (dm m + sum_{s<t} dw_s w_s [muon]) [gmu_t >= log 1e-6],
 //   dgnu_t = dn n [gnu_t >= log 1e-6]
 //
-// Every kernel runs one workgroup of four waves per (b, h, chunk) on
-// float32 tiles staged in LDS (row stride d + 4 floats); wave w owns token
-// rows 16 w .. 16 w + 15 wherever a product is local to token rows.
+// Every kernel runs one workgroup per (b, h, chunk) on float32 tiles staged
+// in LDS (row stride d + 4 floats), 16 waves at d >= 64 and 8 at d = 32: a
+// product's operand reads (LDS, and S_i, dUv_i, dKw_i from L2 in f32_tok) are
+// a dependent chain per tile, so what binds at the chunk counts of float32
+// runs is latency: each SIMD needs several waves to hide it, and operands
+// stored along the contraction are read 16 bytes at a time.  Measured (d = 128,
+// 64 chunks / 1024 chunks; d = 64, 8 chunks), four waves and 4-byte reads
+// before: f32_tok 187 -> 60 us / 993 -> 278 us; 48 -> 20 us; f32_out 32 -> 16 us
+// / 159 -> 84 us; 12.5 -> 8 us.
+// In f32_tok wave w works on token tile w % 4 and the column tiles of part
+// w / 4.
 #include "../../include/gmdn_scan.h"
 #include "chunk_b.h"
 #include "f32mm.h"
@@ -38,9 +46,7 @@
 namespace gmdn {
 namespace {
 
-constexpr int F_THREADS = 256;
-constexpr int F_WAVES = 4;
-static_assert(CB_C == 16 * F_WAVES, "one 16-token tile per wave");
+static_assert(CB_C == 64, "four 16-token tiles");
 
 struct F32Args {
   const float *q, *k, *v, *dO;
@@ -58,9 +64,12 @@ struct F32Args {
 
 template <int D>
 struct F32Lds {
+  static constexpr int WAVES = D >= 64 ? 16 : 8;
+  static constexpr int THREADS = 64 * WAVES;
+  static constexpr int PARTS = WAVES / 4;  // f32_tok: waves per token tile
   static constexpr int C = CB_C;
   static constexpr int LD = D + 4;       // float stride of a token tile row
-  static constexpr int LDC = C + 2;      // float stride of a C x C matrix row
+  static constexpr int LDC = C + 4;      // float stride of a C x C matrix row
   static constexpr int TILE = C * LD;    // floats of a token tile
   static constexpr int CC = C * LDC;     // floats of a C x C matrix
   static constexpr int SMAT = D * LD;    // floats of a d x d plane
@@ -71,7 +80,7 @@ struct F32Lds {
   static constexpr int PREP_BYTES = (2 * TILE + C) * 4;
   static constexpr int OUT_BYTES = (TILE + KV + CC + C) * 4;
   static constexpr int GS_BYTES = (3 * TILE + CC + C) * 4;
-  static constexpr int TOK_BYTES = (3 * TILE + VSLOT + (3 + F_WAVES) * C) * 4;
+  static constexpr int TOK_BYTES = (3 * TILE + VSLOT + (2 + 4 + PARTS) * C) * 4;
   static_assert(OUT_BYTES <= 160 * 1024 && GS_BYTES <= 160 * 1024 && TOK_BYTES <= 160 * 1024,
                 "float32 chunk LDS exceeds the 160 KiB of a CU");
 };
@@ -80,7 +89,7 @@ struct F32Lds {
 template <int D>
 GMDN_DEV void load_rows(float* dst, const float* src, int64_t stride) {
   constexpr int LD = D + 4, V4 = D / 4;
-  for (int e = threadIdx.x; e < CB_C * V4; e += F_THREADS) {
+  for (int e = threadIdx.x; e < CB_C * V4; e += F32Lds<D>::THREADS) {
     const int t = e / V4, c = (e % V4) * 4;
     *reinterpret_cast<f32x4*>(dst + t * LD + c) = *reinterpret_cast<const f32x4*>(src + t * stride + c);
   }
@@ -92,12 +101,11 @@ GMDN_DEV void causal_a(float* As, const float* Qs, const float* Ks, const float*
   using L = F32Lds<D>;
   constexpr int LD = L::LD;
   const int l = lane_id(), lc = l & 15, G = l >> 4;
-  for (int tile = w; tile < 16; tile += F_WAVES) {
+  for (int tile = w; tile < 16; tile += L::WAVES) {
     const int tt = tile >> 2, st = tile & 3;
     f32x4 acc = zero4();
     if (st <= tt) {
-      acc = mm16<D>([&](int r, int k) { return Qs[(16 * tt + r) * LD + k]; },
-                    [&](int k, int c) { return Ks[(16 * st + c) * LD + k]; }, acc);
+      acc = mm16<D>(row_k(Qs, LD, 16 * tt), row_k(Ks, LD, 16 * st), acc);
       const int s = 16 * st + lc;
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[j] = s <= 16 * tt + 4 * G + j ? acc[j] * rb[s] : 0.f;
@@ -111,10 +119,9 @@ template <int D>
 GMDN_DEV void qt_in_place(float* Qs, const float* As, const float* Ks, int w) {
   using L = F32Lds<D>;
   constexpr int LD = L::LD, NT = D / 16;
-  for (int tile = w; tile < 4 * NT; tile += F_WAVES) {
+  for (int tile = w; tile < 4 * NT; tile += L::WAVES) {
     const int tt = tile / NT, tc = tile % NT;
-    const f32x4 ak = mm16<CB_C>([&](int r, int k) { return As[(16 * tt + r) * L::LDC + k]; },
-                                [&](int k, int c) { return Ks[k * LD + 16 * tc + c]; }, zero4());
+    const f32x4 ak = mm16<CB_C>(row_k(As, L::LDC, 16 * tt), col_k(Ks, LD, 16 * tc), zero4());
     st_tile(Qs, LD, 16 * tt, 16 * tc, ld_tile(Qs, LD, 16 * tt, 16 * tc) - ak);
   }
 }
@@ -134,7 +141,7 @@ struct ChunkIdx {
 
 // ------------------------------------------------------------------ forward
 template <int D, int RULE>
-__global__ void __launch_bounds__(F_THREADS) f32_prep(F32Args p) {
+__global__ void __launch_bounds__(F32Lds<D>::THREADS) f32_prep(F32Args p) {
   using L = F32Lds<D>;
   constexpr int C = CB_C, LD = L::LD, NT = D / 16;
   extern __shared__ __align__(16) float sm[];
@@ -169,21 +176,20 @@ __global__ void __launch_bounds__(F_THREADS) f32_prep(F32Args p) {
   __syncthreads();
   float* Kw = p.Kw + x.si * (int64_t)D * D;
   float* Uv = p.Uv + x.si * (int64_t)D * D;
-  for (int tile = w; tile < NT * NT; tile += F_WAVES) {
+  for (int tile = w; tile < NT * NT; tile += L::WAVES) {
     const int ta = tile / NT, tb = tile % NT;
-    const f32x4 kw = mm16<C>([&](int r, int k) { return rw[k] * Ks[k * LD + 16 * ta + r]; },
-                             [&](int k, int c) { return Ks[k * LD + 16 * tb + c]; }, zero4());
-    const f32x4 uv = mm16<C>([&](int r, int k) { return rw[k] * Vs[k * LD + 16 * ta + r]; },
-                             [&](int k, int c) { return Ks[k * LD + 16 * tb + c]; }, zero4());
+    auto kcol = [&](int c, int k) { return Ks[k * LD + 16 * tb + c]; };
+    const f32x4 kw = mm16_seq<C>([&](int r, int k) { return rw[k] * Ks[k * LD + 16 * ta + r]; }, kcol, zero4());
+    const f32x4 uv = mm16_seq<C>([&](int r, int k) { return rw[k] * Vs[k * LD + 16 * ta + r]; }, kcol, zero4());
     st_tile(Kw, D, 16 * ta, 16 * tb, kw);
     st_tile(Uv, D, 16 * ta, 16 * tb, uv);
   }
 }
 
 template <int D>
-__global__ void __launch_bounds__(F_THREADS) f32_out(F32Args p) {
+__global__ void __launch_bounds__(F32Lds<D>::THREADS) f32_out(F32Args p) {
   using L = F32Lds<D>;
-  constexpr int C = CB_C, LD = L::LD, NT = D / 16, NO = 4 * NT / F_WAVES;
+  constexpr int C = CB_C, LD = L::LD, NT = D / 16, NO = 4 * NT / L::WAVES;
   extern __shared__ __align__(16) float sm[];
   float* Qs = sm;
   float* Ks = sm + L::TILE;
@@ -204,16 +210,16 @@ __global__ void __launch_bounds__(F_THREADS) f32_out(F32Args p) {
   f32x4 O[NO];
 #pragma unroll
   for (int q = 0; q < NO; ++q) {
-    const int tile = w + F_WAVES * q, tt = tile / NT, tc = tile % NT;
-    auto arow = [&](int r, int k) { return As[(16 * tt + r) * L::LDC + k]; };
-    O[q] = mm16<C>(arow, [&](int k, int c) { return Vs[k * LD + 16 * tc + c]; }, zero4());
-    const f32x4 ak = mm16<C>(arow, [&](int k, int c) { return Ks[k * LD + 16 * tc + c]; }, zero4());
+    const int tile = w + L::WAVES * q, tt = tile / NT, tc = tile % NT;
+    const auto arow = row_k(As, L::LDC, 16 * tt);
+    O[q] = mm16<C>(arow, col_k(Vs, LD, 16 * tc), zero4());
+    const f32x4 ak = mm16<C>(arow, col_k(Ks, LD, 16 * tc), zero4());
     st_tile(Qs, LD, 16 * tt, 16 * tc, ld_tile(Qs, LD, 16 * tt, 16 * tc) - ak);
   }
   __syncthreads();  // K and V are read: their slot takes S_i
   {
     const float* S = p.S + x.si * (int64_t)D * D;
-    for (int e = threadIdx.x; e < D * D / 4; e += F_THREADS) {
+    for (int e = threadIdx.x; e < D * D / 4; e += L::THREADS) {
       const int r = e / (D / 4), c = (e % (D / 4)) * 4;
       *reinterpret_cast<f32x4*>(Ss + r * LD + c) = *reinterpret_cast<const f32x4*>(S + (int64_t)r * D + c);
     }
@@ -223,10 +229,9 @@ __global__ void __launch_bounds__(F_THREADS) f32_out(F32Args p) {
   const int lc = l & 15, G = l >> 4;
 #pragma unroll
   for (int q = 0; q < NO; ++q) {
-    const int tile = w + F_WAVES * q, tt = tile / NT, tr = tile % NT;
+    const int tile = w + L::WAVES * q, tt = tile / NT, tr = tile % NT;
     // o[t][r] = sum_c Qt[t][c] S[r][c] + Ov[t][r]
-    const f32x4 acc = mm16<D>([&](int r, int k) { return Qs[(16 * tt + r) * LD + k]; },
-                              [&](int k, int c) { return Ss[(16 * tr + c) * LD + k]; }, O[q]);
+    const f32x4 acc = mm16<D>(row_k(Qs, LD, 16 * tt), row_k(Ss, LD, 16 * tr), O[q]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) og[(int64_t)(16 * tt + 4 * G + j) * p.so[2] + 16 * tr + lc] = acc[j];
   }
@@ -234,7 +239,7 @@ __global__ void __launch_bounds__(F_THREADS) f32_out(F32Args p) {
 
 // ----------------------------------------------------------------- backward
 template <int D>
-__global__ void __launch_bounds__(F_THREADS) f32_gs(F32Args p) {
+__global__ void __launch_bounds__(F32Lds<D>::THREADS) f32_gs(F32Args p) {
   using L = F32Lds<D>;
   constexpr int C = CB_C, LD = L::LD, NT = D / 16;
   extern __shared__ __align__(16) float sm[];
@@ -256,18 +261,18 @@ __global__ void __launch_bounds__(F_THREADS) f32_gs(F32Args p) {
   __syncthreads();
   // gS[r][c] = sum_t dO[t][r] Qt[t][c]
   float* gS = p.gS + x.si * (int64_t)D * D;
-  for (int tile = w; tile < NT * NT; tile += F_WAVES) {
+  for (int tile = w; tile < NT * NT; tile += L::WAVES) {
     const int tr = tile / NT, tc = tile % NT;
-    const f32x4 acc = mm16<C>([&](int r, int k) { return Os[k * LD + 16 * tr + r]; },
-                              [&](int k, int c) { return Qs[k * LD + 16 * tc + c]; }, zero4());
+    const f32x4 acc = mm16<C>(col_k(Os, LD, 16 * tr), col_k(Qs, LD, 16 * tc), zero4());
     st_tile(gS, D, 16 * tr, 16 * tc, acc);
   }
 }
 
 template <int D, int RULE>
-__global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
+__global__ void __launch_bounds__(F32Lds<D>::THREADS) f32_tok(F32Args p) {
   using L = F32Lds<D>;
-  constexpr int C = CB_C, LD = L::LD, LDC = L::LDC, NT = D / 16, NTT = C / 16;
+  constexpr int C = CB_C, LD = L::LD, LDC = L::LDC, NT = D / 16;
+  constexpr int TC = NT / L::PARTS, NS = 4 / L::PARTS;  // a wave's column tiles, and its tiles of a C x C row block
   extern __shared__ __align__(16) float sm[];
   float* Qs = sm;
   float* Os = sm + L::TILE;        // dO
@@ -278,11 +283,11 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
   float* red = Vs + L::VSLOT;
   float* rb = red;                 // beta
   float* rw = red + C;             // token weights w
-  float* rdw = red + 2 * C;        // dL/dw
-  float* pdb = red + 3 * C;        // [wave][s]: sum over the wave's t of dA[t,s] (q_t . k_s)
+  float* pdb = red + 2 * C;        // [token tile][s]: sum over the tile's t of dA[t,s] (q_t . k_s)
+  float* rdw = red + 6 * C;        // [part][t]: dL/dw, summed over the part's columns
   const ChunkIdx x(p);
   const int w = wave_id(), l = lane_id(), lc = l & 15, G = l >> 4;
-  const int tt = w;  // this wave's token tile
+  const int tt = w & 3, part = w >> 2;  // this wave's token tile and part
   load_rows<D>(Qs, p.q + x.bb * p.sq[0] + x.hh * p.sq[1] + x.t0 * p.sq[2], p.sq[2]);
   load_rows<D>(Os, p.dO + x.bb * p.so[0] + x.hh * p.so[1] + x.t0 * p.so[2], p.so[2]);
   load_rows<D>(Ks, p.k + x.bb * p.sk[0] + x.hh * p.sk[1] + x.t0 * p.sk[2], p.sk[2]);
@@ -308,44 +313,48 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
   const float* S = p.S + x.si * mat;
   const float* dUv = p.dUv + x.si * mat;
   const float* dKw = p.dKw + x.si * mat;
-  auto own = [&](const float* X) { return [=](int r, int k) { return X[(16 * tt + r) * LD + k]; }; };
+  auto own = [&](const float* X) { return row_k(X, LD, 16 * tt); };
 
   // ---- phase A, rows of tile tt: Z = V dUv (dK's w-term so far), E = V - K S^T, dQt = dO S,
   // the raw Q K^T tiles; dw accumulates k_t . (V dUv)_t
-  f32x4 Z[NT], E[NT], dqt[NT], qk[NTT];
+  f32x4 Z[TC], E[TC], dqt[TC], qk[NS];
   float dwj[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int tc = 0; tc < NT; ++tc) {
-    Z[tc] = mm16<D>(own(Vs), [&](int k, int c) { return dUv[k * D + 16 * tc + c]; }, zero4());
-    const f32x4 ks = mm16<D>(own(Ks), [&](int k, int c) { return S[(16 * tc + c) * D + k]; }, zero4());
-    dqt[tc] = mm16<D>(own(Os), [&](int k, int c) { return S[k * D + 16 * tc + c]; }, zero4());
+  for (int u = 0; u < TC; ++u) {
+    const int tc = part * TC + u;
+    Z[u] = mm16<D>(own(Vs), col_k(dUv, D, 16 * tc), zero4());
+    const f32x4 ks = mm16<D>(own(Ks), row_k(S, D, 16 * tc), zero4());
+    dqt[u] = mm16<D>(own(Os), col_k(S, D, 16 * tc), zero4());
     const f32x4 kt = ld_tile(Ks, LD, 16 * tt, 16 * tc);
-    E[tc] = ld_tile(Vs, LD, 16 * tt, 16 * tc) - ks;
+    E[u] = ld_tile(Vs, LD, 16 * tt, 16 * tc) - ks;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dwj[j] += Z[tc][j] * kt[j];
+    for (int j = 0; j < 4; ++j) dwj[j] += Z[u][j] * kt[j];
   }
 #pragma unroll
-  for (int st = 0; st < NTT; ++st)
-    qk[st] = st <= tt ? mm16<D>(own(Qs), [&](int k, int c) { return Ks[(16 * st + c) * LD + k]; }, zero4())
-                      : zero4();
+  for (int u = 0; u < NS; ++u) {
+    const int st = part + L::PARTS * u;
+    qk[u] = st <= tt ? mm16<D>(own(Qs), row_k(Ks, LD, 16 * st), zero4())
+                     : zero4();
+  }
   __syncthreads();  // every wave has read its V rows: E takes their place
 #pragma unroll
-  for (int tc = 0; tc < NT; ++tc) st_tile(Vs, LD, 16 * tt, 16 * tc, E[tc]);
+  for (int u = 0; u < TC; ++u) st_tile(Vs, LD, 16 * tt, 16 * (part * TC + u), E[u]);
   __syncthreads();
 
   // ---- dA = tril(dO E^T) for rows of tile tt; dbeta's (q_t . k_s) term
-  f32x4 dA[NTT];
+  f32x4 dA[NS];
 #pragma unroll
-  for (int st = 0; st < NTT; ++st) {
-    dA[st] = zero4();
+  for (int u = 0; u < NS; ++u) {
+    const int st = part + L::PARTS * u;
+    dA[u] = zero4();
     float pb = 0.f;
     if (st <= tt) {
-      dA[st] = mm16<D>(own(Os), [&](int k, int c) { return Vs[(16 * st + c) * LD + k]; }, zero4());
+      dA[u] = mm16<D>(own(Os), row_k(Vs, LD, 16 * st), zero4());
       const int s = 16 * st + lc;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        if (s > 16 * tt + 4 * G + j) dA[st][j] = 0.f;
-        pb += dA[st][j] * qk[st][j];
+        if (s > 16 * tt + 4 * G + j) dA[u][j] = 0.f;
+        pb += dA[u][j] * qk[u][j];
       }
     }
     pb = group_sum(pb);
@@ -353,14 +362,15 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
   }
   __syncthreads();  // E is read: A and dA diag(beta) take its place
 #pragma unroll
-  for (int st = 0; st < NTT; ++st) {
+  for (int u = 0; u < NS; ++u) {
+    const int st = part + L::PARTS * u;
     const float bs = rb[16 * st + lc];
     f32x4 a = zero4(), ab = zero4();
     if (st <= tt) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        a[j] = 16 * st + lc <= 16 * tt + 4 * G + j ? qk[st][j] * bs : 0.f;
-        ab[j] = dA[st][j] * bs;
+        a[j] = 16 * st + lc <= 16 * tt + 4 * G + j ? qk[u][j] * bs : 0.f;
+        ab[j] = dA[u][j] * bs;
       }
     }
     st_tile(As, LDC, 16 * tt, 16 * st, a);
@@ -370,29 +380,30 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
 
   // ---- dQ = dQt + (dA diag(beta)) K; Z += K (dKw + dKw^T); Y3 = K dUv^T
   float* dqg = p.dq + x.bb * p.sq[0] + x.hh * p.sq[1] + x.t0 * p.sq[2];
-  f32x4 Y3[NT];
+  f32x4 Y3[TC];
 #pragma unroll
-  for (int tc = 0; tc < NT; ++tc) {
-    const f32x4 dq = mm16<C>([&](int r, int k) { return Abs[(16 * tt + r) * LDC + k]; },
-                             [&](int k, int c) { return Ks[k * LD + 16 * tc + c]; }, dqt[tc]);
+  for (int u = 0; u < TC; ++u) {
+    const int tc = part * TC + u;
+    const f32x4 dq = mm16<C>(row_k(Abs, LDC, 16 * tt), col_k(Ks, LD, 16 * tc), dqt[u]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) dqg[(int64_t)(16 * tt + 4 * G + j) * p.sq[2] + 16 * tc + lc] = dq[j];
-    const f32x4 y2 = mm16<D>(own(Ks), [&](int k, int c) { return dKw[k * D + 16 * tc + c] + dKw[(16 * tc + c) * D + k]; },
-                             zero4());
+    const auto kwc = col_k(dKw, D, 16 * tc);
+    const auto kwr = row_k(dKw, D, 16 * tc);
+    const f32x4 y2 = mm16<D>(own(Ks), [&](int i, int k) { return kwc(i, k) + kwr(i, k); }, zero4());
     const f32x4 kt = ld_tile(Ks, LD, 16 * tt, 16 * tc);
 #pragma unroll
     for (int j = 0; j < 4; ++j) dwj[j] += 0.5f * y2[j] * kt[j];  // k^T dKw k = k^T (dKw + dKw^T) k / 2
-    Z[tc] += y2;
-    Y3[tc] = mm16<D>(own(Ks), [&](int k, int c) { return dUv[(16 * tc + c) * D + k]; }, zero4());
+    Z[u] += y2;
+    Y3[u] = mm16<D>(own(Ks), row_k(dUv, D, 16 * tc), zero4());
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float s = row16_sum(dwj[j]);
-    if (lc == 0) rdw[16 * tt + 4 * G + j] = s;
+    if (lc == 0) rdw[part * C + 16 * tt + 4 * G + j] = s;
   }
   __syncthreads();  // K is read: dQt takes its place
 #pragma unroll
-  for (int tc = 0; tc < NT; ++tc) st_tile(Ks, LD, 16 * tt, 16 * tc, dqt[tc]);
+  for (int u = 0; u < TC; ++u) st_tile(Ks, LD, 16 * tt, 16 * (part * TC + u), dqt[u]);
   __syncthreads();
 
   // ---- phase B, rows s of tile tt: dK = -A^T dQt + (dA diag(beta))^T Q + diag(w) Z,
@@ -403,19 +414,18 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) wr[j] = rw[16 * tt + 4 * G + j];
 #pragma unroll
-  for (int tc = 0; tc < NT; ++tc) {
+  for (int u = 0; u < TC; ++u) {
+    const int tc = part * TC + u;
     f32x4 dk, dv;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      dk[j] = wr[j] * Z[tc][j];
-      dv[j] = wr[j] * Y3[tc][j];
+      dk[j] = wr[j] * Z[u][j];
+      dv[j] = wr[j] * Y3[u][j];
     }
-    dk = mm16<C>([&](int r, int k) { return Abs[k * LDC + 16 * tt + r]; },
-                 [&](int k, int c) { return Qs[k * LD + 16 * tc + c]; }, dk);
-    dk = mm16<C>([&](int r, int k) { return -As[k * LDC + 16 * tt + r]; },
-                 [&](int k, int c) { return Ks[k * LD + 16 * tc + c]; }, dk);
-    dv = mm16<C>([&](int r, int k) { return As[k * LDC + 16 * tt + r]; },
-                 [&](int k, int c) { return Os[k * LD + 16 * tc + c]; }, dv);
+    const auto at = col_k(As, LDC, 16 * tt);
+    dk = mm16<C>(col_k(Abs, LDC, 16 * tt), col_k(Qs, LD, 16 * tc), dk);
+    dk = mm16<C>([&](int i, int k) { return -at(i, k); }, col_k(Ks, LD, 16 * tc), dk);
+    dv = mm16<C>(at, col_k(Os, LD, 16 * tc), dv);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int64_t t = 16 * tt + 4 * G + j;
@@ -431,8 +441,11 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
     const float da = p.dsc[x.si], db = p.dsc[BHN + x.si];
     float dbeta = db * (1.f / C);  // b = mean(beta)
 #pragma unroll
-    for (int q = 0; q < F_WAVES; ++q) dbeta += pdb[q * C + l];
-    if constexpr (RULE == 0) dbeta += rdw[l];  // w = beta
+    for (int q = 0; q < 4; ++q) dbeta += pdb[q * C + l];
+    float dw = 0.f;
+#pragma unroll
+    for (int q = 0; q < L::PARTS; ++q) dw += rdw[q * C + l];
+    if constexpr (RULE == 0) dbeta += dw;  // w = beta
     p.dbeta[o] = dbeta;
     const float a = expf(wave_sum(fmaxf(gg, LOG_FLOOR)));
     p.dg[o] = gg >= LOG_FLOOR ? da * a : 0.f;
@@ -442,7 +455,7 @@ __global__ void __launch_bounds__(F_THREADS) f32_tok(F32Args p) {
       float dl = dm * m;
       if constexpr (RULE == 1) {
         // w_s = exp(sum_{u > s} log mu_u): d w_s / d log mu_t = w_s for s < t
-        const float y = rdw[l] * rw[l];
+        const float y = dw * rw[l];
         dl += wave_incl_scan(y) - y;
       }
       p.dgmu[o] = gm >= LOG_FLOOR ? dl : 0.f;
@@ -477,11 +490,11 @@ F32Args f32_args(const ChunkArgs& a) {
   return f;
 }
 
-template <class K>
+template <int D, class K>
 hipError_t launch(K kern, int bytes, int64_t grid, const F32Args& f, hipStream_t s) {
   hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(F_THREADS), bytes, s, f);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(F32Lds<D>::THREADS), bytes, s, f);
   return hipGetLastError();
 }
 
@@ -499,9 +512,9 @@ hipError_t fwd_d(const ChunkArgs& a, int rule, int ns, float* states, hipStream_
   f.Uv = f.Kw + BHN * mat;
   f.abmn = f.Uv + BHN * mat;
   f.S = S;
-  hipError_t e = rule == 0   ? launch(f32_prep<D, 0>, L::PREP_BYTES, grid, f, s)
-                 : rule == 1 ? launch(f32_prep<D, 1>, L::PREP_BYTES, grid, f, s)
-                             : launch(f32_prep<D, 2>, L::PREP_BYTES, grid, f, s);
+  hipError_t e = rule == 0   ? launch<D>(f32_prep<D, 0>, L::PREP_BYTES, grid, f, s)
+                 : rule == 1 ? launch<D>(f32_prep<D, 1>, L::PREP_BYTES, grid, f, s)
+                             : launch<D>(f32_prep<D, 2>, L::PREP_BYTES, grid, f, s);
   if (e != hipSuccess) return e;
   ScanArgs sa{};
   sa.U = f.Uv;
@@ -522,7 +535,7 @@ hipError_t fwd_d(const ChunkArgs& a, int rule, int ns, float* states, hipStream_
   sa.stream = s;
   e = rule == 1 ? scan_fwd_muon_launch(sa) : scan_fwd_rows_launch(sa);
   if (e != hipSuccess) return e;
-  return launch(f32_out<D>, L::OUT_BYTES, grid, f, s);
+  return launch<D>(f32_out<D>, L::OUT_BYTES, grid, f, s);
 }
 
 template <int D>
@@ -544,7 +557,7 @@ hipError_t bwd_d(const ChunkArgs& a, int rule, int ns, const float* states, floa
   float* dsc = ws + 3 * BHN * mat;
   float* part = dsc + 4 * BHN;
   const int64_t part_floats = (int64_t)ws_floats - (3 * BHN * mat + 4 * BHN);
-  hipError_t e = launch(f32_gs<D>, L::GS_BYTES, grid, f, s);
+  hipError_t e = launch<D>(f32_gs<D>, L::GS_BYTES, grid, f, s);
   if (e != hipSuccess) return e;
   ScanArgs sa{};
   sa.U = Uv;
@@ -583,9 +596,9 @@ hipError_t bwd_d(const ChunkArgs& a, int rule, int ns, const float* states, floa
   f.dg = a.dg;
   f.dgmu = a.dgmu;
   f.dgnu = a.dgnu;
-  return rule == 0   ? launch(f32_tok<D, 0>, L::TOK_BYTES, grid, f, s)
-         : rule == 1 ? launch(f32_tok<D, 1>, L::TOK_BYTES, grid, f, s)
-                     : launch(f32_tok<D, 2>, L::TOK_BYTES, grid, f, s);
+  return rule == 0   ? launch<D>(f32_tok<D, 0>, L::TOK_BYTES, grid, f, s)
+         : rule == 1 ? launch<D>(f32_tok<D, 1>, L::TOK_BYTES, grid, f, s)
+                     : launch<D>(f32_tok<D, 2>, L::TOK_BYTES, grid, f, s);
 }
 
 }  // namespace

@@ -9,15 +9,42 @@
 
 namespace gmdn {
 
-// acc += sum_k A(r, k) B(k, c) over a 16 x 16 tile, k = 0 .. K-1 in steps
-// of 4; a(r, k) / b(k, c) return the lane's operand element for tile row r /
-// tile column c.
+// acc += sum_k A(r, k) B(k, c) over a 16 x 16 tile, k = 0 .. K-1.  The
+// contraction runs in the order k = 16 t + 4 G + e (step e of block t, lane
+// group G): a(i, k) / b(i, k) return the lane's operand elements k .. k + 3 of
+// tile row / column i, so that an operand stored along k is one 16-byte read
+// for four products.
 template <int K, class FA, class FB>
 GMDN_DEV f32x4 mm16(FA a, FB b, f32x4 acc) {
   const int l = lane_id(), i = l & 15, G = l >> 4;
-#pragma unroll 4
-  for (int k = 0; k < K; k += 4) acc = mfma_f32(a(i, k + G), b(k + G, i), acc);
+#pragma unroll
+  for (int k = 0; k < K; k += 16) {
+    const f32x4 x = a(i, k + 4 * G), y = b(i, k + 4 * G);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = mfma_f32(x[e], y[e], acc);
+  }
   return acc;
+}
+// The same with the contraction in natural order (lane group G takes 4 s + G
+// in step s) and scalar operands a(i, k), b(i, k): for operands stored down k.
+template <int K, class FA, class FB>
+GMDN_DEV f32x4 mm16_seq(FA a, FB b, f32x4 acc) {
+  const int l = lane_id(), i = l & 15, G = l >> 4;
+#pragma unroll 8
+  for (int k = 0; k < K; k += 4) acc = mfma_f32(a(i, k + G), b(i, k + G), acc);
+  return acc;
+}
+// Operands of mm16 from a row-major float matrix (row stride ld): tile rows
+// (columns) are the matrix's rows r0 .. (k along them, 16-byte aligned), or
+// its columns c0 .. (k down them).
+GMDN_DEV auto row_k(const float* X, int ld, int r0) {
+  return [=](int i, int k) { return *reinterpret_cast<const f32x4*>(X + (r0 + i) * ld + k); };
+}
+GMDN_DEV auto col_k(const float* X, int ld, int c0) {
+  return [=](int i, int k) {
+    const float* x = X + k * ld + c0 + i;
+    return f32x4{x[0], x[ld], x[2 * ld], x[3 * ld]};
+  };
 }
 
 // D-layout tile -> row-major float matrix X (row stride ld) at (r0, c0)
