@@ -51,7 +51,7 @@
 namespace gmdn {
 namespace {
 
-constexpr int WY_THREADS = 256;
+constexpr int WY_THREADS = 512;
 
 // Per-token gate quantities of the chunk (wave 0, lane = token): beta, gamma,
 // beta gamma, kd = gamma_C / gamma and log gamma (the prefix sums of the
@@ -142,7 +142,8 @@ GMDN_DEV void tri_inverse(const float* As, float* Ts, float* Xw_all) {
 //   P  = T^T diag(kd) K, tiles [s][c], scaled by beta_s / beta gamma_s:
 //   U_A = V^T (diag(beta) P),  K_A = K^T (diag(beta gamma) P)
 // (the same algebra, with diag(beta) moved onto P.)
-constexpr int WYP_THREADS = 512;
+template <int D>
+constexpr int WYP_THREADS = D == 128 ? 1024 : 512;
 
 template <int D>
 struct WyPrepLds {
@@ -173,10 +174,13 @@ GMDN_DEV void causal_tile(int idx, int& tt, int& st) {
 // Rows x W floats (row stride ld) -> split planes BSwz<W>.
 template <int W, int ROWS, int NTHR>
 struct SplitRows {
-  static constexpr int PER = ROWS * (W / 8) / NTHR;
-  static_assert(ROWS * (W / 8) % NTHR == 0, "whole 8-column groups per thread");
+  static constexpr int GROUPS = ROWS * (W / 8);  // 8-column groups
+  static constexpr int PER = (GROUPS + NTHR - 1) / NTHR;
+  static_assert(GROUPS % NTHR == 0 || PER == 1, "whole groups per thread, or one for the first threads");
   f32x4 x[PER][2];
+  static GMDN_DEV bool mine() { return GROUPS >= NTHR || (int)threadIdx.x < GROUPS; }
   GMDN_DEV void load(const float* src, int64_t ld) {
+    if (!mine()) return;
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int e = threadIdx.x + q * NTHR, r = e / (W / 8), c = (e % (W / 8)) * 8;
@@ -186,6 +190,7 @@ struct SplitRows {
   }
   // zero the entries above the diagonal (square matrices)
   GMDN_DEV void lower() {
+    if (!mine()) return;
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int e = threadIdx.x + q * NTHR, r = e / (W / 8), c = (e % (W / 8)) * 8;
@@ -198,6 +203,7 @@ struct SplitRows {
   }
   GMDN_DEV void store(bf16* hi, bf16* lo) const {
     using LW = BSwz<W>;
+    if (!mine()) return;
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int e = threadIdx.x + q * NTHR, r = e / (W / 8), c = (e % (W / 8)) * 8;
@@ -234,7 +240,7 @@ struct TokRows {
 };
 
 template <int D>
-__global__ void __launch_bounds__(WYP_THREADS)
+__global__ void __launch_bounds__(WYP_THREADS<D>)
 wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __restrict__ Qt,
         float* __restrict__ Ov, float* __restrict__ aout) {
   using L = WyPrepLds<D>;
@@ -269,7 +275,7 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
   const bf16* kg = p.k + bb * p.sk[0] + hh * p.sk[1] + t0 * p.sk[2];
   const bf16* vg = p.v + bb * p.sv[0] + hh * p.sv[1] + t0 * p.sv[2];
   {
-    TokRows<D, WYP_THREADS> tk, tq, tv;
+    TokRows<D, WYP_THREADS<D>> tk, tq, tv;
     tk.load(kg, p.sk[2]);
     tq.load(qg, p.sq[2]);
     tv.load(vg, p.sv[2]);
@@ -277,8 +283,8 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
     tq.store(Qb);
     tv.store(Vb);
   }
-  for (int e = threadIdx.x; e < C * LDC / 4; e += WYP_THREADS) reinterpret_cast<f32x4*>(Ts)[e] = zero4();
-  for (int e = threadIdx.x; e < 2 * L::CP / 16; e += WYP_THREADS) reinterpret_cast<f32x4*>(Mh)[e] = zero4();
+  for (int e = threadIdx.x; e < C * LDC / 4; e += WYP_THREADS<D>) reinterpret_cast<f32x4*>(Ts)[e] = zero4();
+  for (int e = threadIdx.x; e < 2 * L::CP / 16; e += WYP_THREADS<D>) reinterpret_cast<f32x4*>(Mh)[e] = zero4();
   if (w == 0) {
     const float g_ = wy_gates(p.beta, p.g, bh * p.T + t0 + l, bet, gam, bg, kd, lgam);
     if (l == 63) aout[bh * p.N + i] = g_;
@@ -287,7 +293,7 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
 
   // ---- A's causal tiles (float32, for the substitution) and M's (split
   //      planes): jobs 0-9 and 10-19 over the waves
-  for (int job = w; job < 20; job += WYP_THREADS / 64) {
+  for (int job = w; job < 20; job += WYP_THREADS<D> / 64) {
     int tt, st;
     causal_tile(job % 10, tt, st);
     if (job < 10) {
@@ -324,8 +330,8 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
   __syncthreads();
   tri_inverse<LDC>(As, Ts, reinterpret_cast<float*>(smem + L::X0));
 
-  // ---- split planes of T and diag(kd) T (one 8-column group per thread)
-  {
+  // ---- split planes of T and diag(kd) T (an 8-column group for each of the first 512 threads)
+  if (threadIdx.x < 512) {
     const int r = threadIdx.x >> 3, c = (threadIdx.x & 7) * 8;
     const f32x4 x0 = *reinterpret_cast<const f32x4*>(Ts + r * LDC + c);
     const f32x4 x1 = *reinterpret_cast<const f32x4*>(Ts + r * LDC + c + 4);
@@ -343,10 +349,12 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
   __syncthreads();
 
   const int64_t tokbase = (bh * p.T + t0) * (int64_t)D;
-  // ---- Qt (waves 0-3) or Ov (waves 4-7) of token tile tt
+  // ---- Qt (waves 0-3, 8-11) or Ov (waves 4-7, 12-15) of token tile tt
   {
-    const bool ov = w >= 4;
+    const bool ov = (w >> 2) & 1;
     const int tt = w & 3;
+    constexpr int TPP = NT / (WYP_THREADS<D> / 512);  // column tiles of a wave
+    const int tc0 = (w >> 3) * TPP;
     // (M T)^T[u][t] = sum_s T[s][u] M[t][s], causal (u <= t)
     f32x4 mt[4];
 #pragma unroll
@@ -367,7 +375,7 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
     const bf16* Bt = ov ? Vb : Kb;
     float* out = (ov ? Ov : Qt) + tokbase;
 #pragma unroll 2
-    for (int tc = 0; tc < NT; ++tc) {
+    for (int tc = tc0; tc < tc0 + TPP; ++tc) {
       f32x4 acc = mma<2, 1>(a0, Op<1>{{b_col<LT>(Bt, 0, 16 * tc)}}, zero4());
       if (tt >= 2) acc = mma<2, 1>(a1, Op<1>{{b_col<LT>(Bt, 32, 16 * tc)}}, acc);
       const int c = 16 * tc + lc;
@@ -381,7 +389,7 @@ wy_prep(ChunkArgs p, float* __restrict__ UA, float* __restrict__ KA, float* __re
 
   // ---- P column tile ct, then U_A and K_A columns ct over the wave's row tiles
   {
-    constexpr int WPC = (WYP_THREADS / 64) / NT;  // waves per column tile
+    constexpr int WPC = (WYP_THREADS<D> / 64) / NT;  // waves per column tile
     const int ct = w % NT, part = w / NT;
     f32x4 pt[4];
 #pragma unroll
@@ -434,13 +442,14 @@ wy_out(ChunkArgs p, const float* __restrict__ Qt, const float* __restrict__ Ov, 
   const int64_t bb = bh / p.H, hh = bh % p.H, t0 = (int64_t)i * C;
   const int w = wave_id(), l = lane_id(), lc = l & 15, G = l >> 4;
   const int64_t tokbase = (bh * p.T + t0) * (int64_t)D;
+  const int tt = w & 3, h = w >> 2;  // token tile, half of the rows of S
   const float* S = Sst + (bh * p.N + i) * (int64_t)D * D;
   SplitRows<D, D, WY_THREADS> sr;
   sr.load(S, D);
   // lane (t, G) of k-block kb: Qt[16 w + t][32 kb + 8G .. +7]
   Op<2> qa[NKB];
   {
-    const float* qr = Qt + tokbase + (int64_t)(16 * w + lc) * D + 8 * G;
+    const float* qr = Qt + tokbase + (int64_t)(16 * tt + lc) * D + 8 * G;
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
       bf16x4 h0, o0, h1, o1;
@@ -453,7 +462,7 @@ wy_out(ChunkArgs p, const float* __restrict__ Qt, const float* __restrict__ Ov, 
   __syncthreads();
   bf16* og = p.o + bb * p.so[0] + hh * p.so[1] + t0 * p.so[2];
 #pragma unroll 2
-  for (int rt = 0; rt < NT; ++rt) {
+  for (int rt = h * NT / 2; rt < (h + 1) * NT / 2; ++rt) {
     // tile [t][r] = sum_c Qt[t][c] S[r][c]
     f32x4 acc = zero4();
 #pragma unroll
@@ -462,7 +471,7 @@ wy_out(ChunkArgs p, const float* __restrict__ Qt, const float* __restrict__ Ov, 
     const int r = 16 * rt + lc;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int t = 16 * w + 4 * G + j;
+      const int t = 16 * tt + 4 * G + j;
       og[t * p.so[2] + r] = (bf16)(acc[j] + Ov[tokbase + (int64_t)t * D + r]);
     }
   }
@@ -472,7 +481,7 @@ wy_out(ChunkArgs p, const float* __restrict__ Qt, const float* __restrict__ Ov, 
 // Chunk-parallel kernels of 8 waves; intermediates of one chunk pass
 // through the workspace.  Split-bf16 products as in the forward; S_i and Sb
 // are staged in LDS as split planes (rows r, BSwz), one of them per kernel.
-// Wave w takes token tile tt = w % 4 and the feature half h = w / 4 of
+// Wave w takes token tile tt = w % 4 and the feature part h = w / 4 of
 // every C x d result.
 //   wy_gs  gS = dO^T Qt
 //   wy_ka  (S_i)  A, T (to the workspace); W, U; X = U - W S^T;
@@ -483,7 +492,7 @@ wy_out(ChunkArgs p, const float* __restrict__ Qt, const float* __restrict__ Ov, 
 //                 dT = dX Z^T (the lower tiles; with dW = -dX S, dW (diag(beta gamma) K)^T
 //                 = -dX (diag(beta gamma) K S^T)^T)
 //   wy_kc2        dA = strict_lower(-T^T dT T^T); the A and M terms of dq, dk; the gates
-// Per-token partial sums (one slot per feature half) go to the chunk's
+// Per-token partial sums (one slot per feature part) go to the chunk's
 // `tokp` record and are added in a fixed order: the gradients are bitwise
 // reproducible.
 struct WyBwd {
@@ -497,11 +506,16 @@ struct WyBwd {
   bf16 *dq, *dk, *dv;
   float *dbeta, *dg;
 };
-// tokp record: [dgamma from q: 2 C][dkd: 2 C][beta-side of U: 2 C][beta gamma-side of W: 2 C][<Sb, S_i>]
-constexpr int TOKP = 8 * CB_C + 4;
-constexpr int TP_GQ = 0, TP_KD = 2 * CB_C, TP_SB = 4 * CB_C, TP_SBG = 6 * CB_C, TP_DA = 8 * CB_C;
+// tokp record, one slot of C per feature part: [dgamma from q: 4 C][dkd: 4 C][beta-side of U: 4 C]
+// [beta gamma-side of W: 4 C][<Sb, S_i>]
+constexpr int TOKP = 16 * CB_C + 4;
+constexpr int TP_GQ = 0, TP_KD = 4 * CB_C, TP_SB = 8 * CB_C, TP_SBG = 12 * CB_C, TP_DA = 16 * CB_C;
 
-constexpr int WYB_THREADS = 512;
+template <int D>
+constexpr int WYB_THREADS = D == 128 ? 1024 : 512;
+// feature parts of a C x d result: waves per token tile
+template <int D>
+constexpr int WYB_PARTS = WYB_THREADS<D> / 256;
 
 // split operand from a float row in global memory: lane (i, G) takes
 // X[r0 + i][k0 + 8G .. +7] (natural k order)
@@ -592,11 +606,11 @@ struct WyKaLds {
 };
 
 template <int D>
-__global__ void __launch_bounds__(WYB_THREADS) wy_ka(ChunkArgs p, WyBwd b) {
+__global__ void __launch_bounds__(WYB_THREADS<D>) wy_ka(ChunkArgs p, WyBwd b) {
   using L = WyKaLds<D>;
   using LT = BSwz<D>;
   using LP = BSwz<CB_C>;
-  constexpr int C = CB_C, LDC = L::LDC, NT = D / 16, NKB = D / 32, NH = NT / 2;
+  constexpr int C = CB_C, LDC = L::LDC, NT = D / 16, NKB = D / 32, NH = NT / WYB_PARTS<D>;
   extern __shared__ __align__(16) char smem[];
   bf16* Kb = reinterpret_cast<bf16*>(smem + L::K0);
   bf16* Vb = reinterpret_cast<bf16*>(smem + L::V0);
@@ -621,9 +635,9 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_ka(ChunkArgs p, WyBwd b) {
   const bf16* qg = p.q + bb * p.sq[0] + hh * p.sq[1] + t0 * p.sq[2];
 
   // S_i's loads stay in flight through A and T (its planes replace them in region R)
-  SplitRows<D, D, WYB_THREADS> sr;
+  SplitRows<D, D, WYB_THREADS<D>> sr;
   {
-    TokRows<D, WYB_THREADS> tk, tv, to;
+    TokRows<D, WYB_THREADS<D>> tk, tv, to;
     tk.load(p.k + bb * p.sk[0] + hh * p.sk[1] + t0 * p.sk[2], p.sk[2]);
     tv.load(p.v + bb * p.sv[0] + hh * p.sv[1] + t0 * p.sv[2], p.sv[2]);
     to.load(b.dO + bb * p.so[0] + hh * p.so[1] + t0 * p.so[2], p.so[2]);
@@ -632,11 +646,11 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_ka(ChunkArgs p, WyBwd b) {
     tv.store(Vb);
     to.store(Ob);
   }
-  for (int e = threadIdx.x; e < C * LDC / 4; e += WYB_THREADS) reinterpret_cast<f32x4*>(Ts)[e] = zero4();
+  for (int e = threadIdx.x; e < C * LDC / 4; e += WYB_THREADS<D>) reinterpret_cast<f32x4*>(Ts)[e] = zero4();
   if (w == 0) wy_gates(p.beta, p.g, bh * p.T + t0 + l, bet, gam, bg, kd, lgam);
   __syncthreads();
   // ---- A's causal tiles, T
-  for (int job = w; job < 10; job += WYB_THREADS / 64) {
+  for (int job = w; job < 10; job += WYB_THREADS<D> / 64) {
     int tt, st;
     causal_tile(job, tt, st);
     f32x4 acc = zero4();
@@ -653,7 +667,7 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_ka(ChunkArgs p, WyBwd b) {
   }
   __syncthreads();
   tri_inverse<LDC>(As, Ts, Ts + C * LDC);
-  {
+  if (threadIdx.x < 512) {
     // T's split planes, and T itself for the later kernels
     const int r = threadIdx.x >> 3, c = (threadIdx.x & 7) * 8;
     const f32x4 x0 = *reinterpret_cast<const f32x4*>(Ts + r * LDC + c);
@@ -687,10 +701,12 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_ka(ChunkArgs p, WyBwd b) {
 #pragma unroll
   for (int kp = 0; kp < NKB; ++kp) {
     f32x4 a0 = zero4(), a1 = zero4();
-    for (int kb = 0; kb <= kbt; ++kb) {
-      a0 = mma<1, 2>(Op<1>{{col8<LT>(Kb, 32 * kb, 32 * kp)}}, tg[kb], a0);
-      a1 = mma<1, 2>(Op<1>{{col8<LT>(Kb, 32 * kb, 32 * kp + 16)}}, tg[kb], a1);
-    }
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      if (kb <= kbt) {
+        a0 = mma<1, 2>(Op<1>{{col8<LT>(Kb, 32 * kb, 32 * kp)}}, tg[kb], a0);
+        a1 = mma<1, 2>(Op<1>{{col8<LT>(Kb, 32 * kb, 32 * kp + 16)}}, tg[kb], a1);
+      }
     wn[kp] = pack_tiles<2>(-a0, -a1);
   }
 #pragma unroll 1
@@ -698,7 +714,9 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_ka(ChunkArgs p, WyBwd b) {
     const int rt = h * NH + q;
     // X = U - W S^T, U[t][r] = sum_s beta_s T[t][s] V[s][r]
     f32x4 x = zero4();
-    for (int kb = 0; kb <= kbt; ++kb) x = mma<2, 1>(tb[kb], Op<1>{{col8<LT>(Vb, 32 * kb, 16 * rt)}}, x);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      if (kb <= kbt) x = mma<2, 1>(tb[kb], Op<1>{{col8<LT>(Vb, 32 * kb, 16 * rt)}}, x);
 #pragma unroll
     for (int kp = 0; kp < NKB; ++kp) x = mma<2, 2>(wn[kp], prow_p<LT>(Sh, Sl, 16 * rt, 32 * kp), x);
     st_tile(b.X + tokbase, D, 16 * tt, 16 * rt, x);
@@ -746,16 +764,16 @@ struct WyKbLds {
   static constexpr int K0 = 0, Q0 = TB, O0 = 2 * TB;
   static constexpr int SH0 = 3 * TB, SL0 = SH0 + 2 * D * D, MH0 = SL0 + 2 * D * D, ML0 = MH0 + CP;
   static constexpr int G0 = ML0 + CP, DA0 = G0 + 5 * C * 4;
-  static constexpr int BYTES = DA0 + 8 * 4;
+  static constexpr int BYTES = DA0 + 16 * 4;
   static_assert(BYTES <= 160 * 1024, "WY backward LDS exceeds the 160 KiB of a CU");
 };
 
 template <int D>
-__global__ void __launch_bounds__(WYB_THREADS) wy_kb(ChunkArgs p, WyBwd b) {
+__global__ void __launch_bounds__(WYB_THREADS<D>) wy_kb(ChunkArgs p, WyBwd b) {
   using L = WyKbLds<D>;
   using LT = BSwz<D>;
   using LP = BSwz<CB_C>;
-  constexpr int C = CB_C, NT = D / 16, NKB = D / 32, NH = NT / 2;
+  constexpr int C = CB_C, NT = D / 16, NKB = D / 32, NH = NT / WYB_PARTS<D>;
   extern __shared__ __align__(16) char smem[];
   bf16* Kb = reinterpret_cast<bf16*>(smem + L::K0);
   bf16* Qb = reinterpret_cast<bf16*>(smem + L::Q0);
@@ -779,8 +797,8 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kb(ChunkArgs p, WyBwd b) {
 
   {
     // Sb's planes, and <Sb, S_i> from the same pieces of both
-    TokRows<D, WYB_THREADS> tk, tq, to;
-    SplitRows<D, D, WYB_THREADS> sb, sx;
+    TokRows<D, WYB_THREADS<D>> tk, tq, to;
+    SplitRows<D, D, WYB_THREADS<D>> sb, sx;
     tk.load(p.k + bb * p.sk[0] + hh * p.sk[1] + t0 * p.sk[2], p.sk[2]);
     tq.load(p.q + bb * p.sq[0] + hh * p.sq[1] + t0 * p.sq[2], p.sq[2]);
     to.load(b.dO + bb * p.so[0] + hh * p.so[1] + t0 * p.so[2], p.so[2]);
@@ -796,11 +814,11 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kb(ChunkArgs p, WyBwd b) {
     acc = wave_sum(acc);
     if (l == 0) dap[w] = acc;
   }
-  for (int e = threadIdx.x; e < 2 * L::CP / 16; e += WYB_THREADS) reinterpret_cast<f32x4*>(Mh)[e] = zero4();
+  for (int e = threadIdx.x; e < 2 * L::CP / 16; e += WYB_THREADS<D>) reinterpret_cast<f32x4*>(Mh)[e] = zero4();
   if (w == 0) wy_gates(p.beta, p.g, bh * p.T + t0 + l, bet, gam, bg, kd, lgam);
   __syncthreads();
   // ---- M's causal tiles (split planes, rows t) and dM = lower_incl(dO X^T) (to the workspace)
-  for (int job = w; job < 20; job += WYB_THREADS / 64) {
+  for (int job = w; job < 20; job += WYB_THREADS<D> / 64) {
     int tt, st;
     causal_tile(job % 10, tt, st);
     if (job < 10) {
@@ -872,8 +890,12 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kb(ChunkArgs p, WyBwd b) {
     const float s = row16_sum(dkd[j]);
     if (lc == 0) tp[TP_KD + h * C + 16 * tt + 4 * G + j] = s;
   }
-  if (threadIdx.x == 0)
-    tp[TP_DA] = ((dap[0] + dap[1]) + (dap[2] + dap[3])) + ((dap[4] + dap[5]) + (dap[6] + dap[7]));
+  if (threadIdx.x == 0) {
+    float s = 0.f;
+#pragma unroll
+    for (int q = 0; q < WYB_THREADS<D> / 64; ++q) s += dap[q];
+    tp[TP_DA] = s;
+  }
 }
 
 template <int D>
@@ -886,11 +908,11 @@ struct WyKc1Lds {
 };
 
 template <int D>
-__global__ void __launch_bounds__(WYB_THREADS) wy_kc1(ChunkArgs p, WyBwd b) {
+__global__ void __launch_bounds__(WYB_THREADS<D>) wy_kc1(ChunkArgs p, WyBwd b) {
   using L = WyKc1Lds<D>;
   using LT = BSwz<D>;
   using LP = BSwz<CB_C>;
-  constexpr int C = CB_C, NT = D / 16, NKB = D / 32, NH = NT / 2;
+  constexpr int C = CB_C, NT = D / 16, NKB = D / 32, NH = NT / WYB_PARTS<D>;
   extern __shared__ __align__(16) char smem[];
   bf16* Sh = reinterpret_cast<bf16*>(smem + L::SH0);
   bf16* Sl = reinterpret_cast<bf16*>(smem + L::SL0);
@@ -913,9 +935,9 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc1(ChunkArgs p, WyBwd b) {
   const bf16* vg = p.v + bb * p.sv[0] + hh * p.sv[1] + t0 * p.sv[2];
 
   {
-    SplitRows<D, D, WYB_THREADS> ss;
-    SplitRows<C, C, WYB_THREADS> st;
-    SplitRows<D, C, WYB_THREADS> sx;
+    SplitRows<D, D, WYB_THREADS<D>> ss;
+    SplitRows<C, C, WYB_THREADS<D>> st;
+    SplitRows<D, C, WYB_THREADS<D>> sx;
     ss.load(b.S_all + si * (int64_t)D * D, D);
     st.load(b.T + si * C * C, C);
     sx.load(b.dX + tokbase, D);
@@ -978,7 +1000,7 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc1(ChunkArgs p, WyBwd b) {
     }
   }
   // dT = dX Z^T, the causal tiles (the strictly upper part of dT does not reach dA)
-  for (int job = w; job < 10; job += WYB_THREADS / 64) {
+  for (int job = w; job < 10; job += WYB_THREADS<D> / 64) {
     int at, st;
     causal_tile(job, at, st);
     f32x4 acc = zero4();
@@ -1003,11 +1025,11 @@ struct WyKc2Lds {
 };
 
 template <int D>
-__global__ void __launch_bounds__(WYB_THREADS) wy_kc2(ChunkArgs p, WyBwd b) {
+__global__ void __launch_bounds__(WYB_THREADS<D>) wy_kc2(ChunkArgs p, WyBwd b) {
   using L = WyKc2Lds<D>;
   using LT = BSwz<D>;
   using LP = BSwz<CB_C>;
-  constexpr int C = CB_C, NT = D / 16, NKB = D / 32, NH = NT / 2, CP = L::CP / 2;  // CP: bf16 per plane
+  constexpr int C = CB_C, NT = D / 16, NKB = D / 32, NH = NT / WYB_PARTS<D>, CP = L::CP / 2;  // CP: bf16 per plane
   extern __shared__ __align__(16) char smem[];
   bf16* Qb = reinterpret_cast<bf16*>(smem + L::Q0);
   bf16* Kb = reinterpret_cast<bf16*>(smem + L::K0);
@@ -1037,8 +1059,8 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc2(ChunkArgs p, WyBwd b) {
   const int64_t tokbase = (bh * p.T + t0) * (int64_t)D;
   {
     // dT's planes with its strictly upper part (not written) as zeros; H and DG^T zeroed
-    TokRows<D, WYB_THREADS> tq, tk;
-    SplitRows<C, C, WYB_THREADS> st, sd;
+    TokRows<D, WYB_THREADS<D>> tq, tk;
+    SplitRows<C, C, WYB_THREADS<D>> st, sd;
     tq.load(p.q + bb * p.sq[0] + hh * p.sq[1] + t0 * p.sq[2], p.sq[2]);
     tk.load(p.k + bb * p.sk[0] + hh * p.sk[1] + t0 * p.sk[2], p.sk[2]);
     st.load(b.T + si * C * C, C);
@@ -1049,7 +1071,7 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc2(ChunkArgs p, WyBwd b) {
     sd.lower();
     sd.store(Dh, Dl);
   }
-  for (int e = threadIdx.x; e < 4 * L::CP / 16; e += WYB_THREADS) reinterpret_cast<f32x4*>(Hh)[e] = zero4();
+  for (int e = threadIdx.x; e < 4 * L::CP / 16; e += WYB_THREADS<D>) reinterpret_cast<f32x4*>(Hh)[e] = zero4();
   float graw = 0.f;
   if (w == 0) {
     graw = p.g[bh * p.T + t0 + l];
@@ -1057,7 +1079,7 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc2(ChunkArgs p, WyBwd b) {
   }
   __syncthreads();
   // ---- Y = dT T^T as planes of rows t: tiles Y^T[u][t] = sum_s T[u][s] dT[t][s], stored transposed
-  for (int tile = w; tile < 16; tile += WYB_THREADS / 64) {
+  for (int tile = w; tile < 16; tile += WYB_THREADS<D> / 64) {
     const int ut = tile >> 2, tt = tile & 3;
     f32x4 acc = zero4();
 #pragma unroll
@@ -1071,7 +1093,7 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc2(ChunkArgs p, WyBwd b) {
   __syncthreads();
   // ---- causal tiles [t][s]: dA = strict_lower(-T^T Y), G_A = dA beta_t Gamma, DG = dM Gamma,
   //      E = dGamma * Gamma = (dA beta_t (K K^T) + dM (Q K^T)) Gamma, the A term of dbeta
-  for (int job = w; job < 10; job += WYB_THREADS / 64) {
+  for (int job = w; job < 10; job += WYB_THREADS<D> / 64) {
     int tt, st;
     causal_tile(job, tt, st);
     f32x4 ta = zero4(), kk = zero4(), qk = zero4();
@@ -1148,11 +1170,17 @@ __global__ void __launch_bounds__(WYB_THREADS) wy_kc2(ChunkArgs p, WyBwd b) {
   // ---- gate gradients (wave 0, lane = token)
   if (w == 0) {
     const float* tp = b.tokp + si * TOKP;
-    const float sbg = tp[TP_SBG + l] + tp[TP_SBG + C + l];
-    const float dgm = (tp[TP_GQ + l] + tp[TP_GQ + C + l]) + bet[l] * sbg;  // dL/dgamma_t
-    const float dkdv = tp[TP_KD + l] + tp[TP_KD + C + l];                   // dL/dkd_t
-    const float dbu = (tp[TP_SB + l] + tp[TP_SB + C + l]) + gam[l] * sbg;   // dL/dbeta_t from U and W
-    const float dgC = tp[TP_DA];                                            // dL/dgamma_C = <Sb, S_i>
+    auto parts = [&](int slot) {
+      float s = 0.f;
+#pragma unroll
+      for (int q = 0; q < WYB_PARTS<D>; ++q) s += tp[slot + q * C + l];
+      return s;
+    };
+    const float sbg = parts(TP_SBG);
+    const float dgm = parts(TP_GQ) + bet[l] * sbg;  // dL/dgamma_t
+    const float dkdv = parts(TP_KD);                 // dL/dkd_t
+    const float dbu = parts(TP_SB) + gam[l] * sbg;   // dL/dbeta_t from U and W
+    const float dgC = tp[TP_DA];                     // dL/dgamma_C = <Sb, S_i>
     // row and column sums of E over the causal tiles of this token, in a fixed order
     const int tl = l >> 4, lr = l & 15;
     float rowE = 0.f, bsum = 0.f, colE = 0.f;
@@ -1214,7 +1242,7 @@ hipError_t launch_wy(const ChunkArgs& a, float* ws, hipStream_t s) {
   hipError_t e = hipFuncSetAttribute((const void*)kp, hipFuncAttributeMaxDynamicSharedMemorySize, lp);
   if (e == hipSuccess) e = hipFuncSetAttribute((const void*)ko, hipFuncAttributeMaxDynamicSharedMemorySize, lo);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kp, dim3((unsigned)chunks), dim3(WYP_THREADS), lp, s, a, c.UA, c.KA, c.Qt, c.Ov, c.av);
+  hipLaunchKernelGGL(kp, dim3((unsigned)chunks), dim3(WYP_THREADS<D>), lp, s, a, c.UA, c.KA, c.Qt, c.Ov, c.av);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   ScanArgs sa{};
   sa.U = c.UA;
@@ -1291,10 +1319,10 @@ hipError_t launch_wy_bwd(const ChunkArgs& a, float* ckpt, const void* dO, void* 
   sa.precision = GMDN_PREC_TF32;
   sa.stream = s;
   if ((e = scan_bwd_rows_launch(sa, nullptr)) != hipSuccess) return e;
-  if ((e = launch_k(wy_ka<D>, WYB_THREADS, WyKaLds<D>::BYTES, chunks, s, a, b)) != hipSuccess) return e;
-  if ((e = launch_k(wy_kb<D>, WYB_THREADS, WyKbLds<D>::BYTES, chunks, s, a, b)) != hipSuccess) return e;
-  if ((e = launch_k(wy_kc1<D>, WYB_THREADS, WyKc1Lds<D>::BYTES, chunks, s, a, b)) != hipSuccess) return e;
-  return launch_k(wy_kc2<D>, WYB_THREADS, WyKc2Lds<D>::BYTES, chunks, s, a, b);
+  if ((e = launch_k(wy_ka<D>, WYB_THREADS<D>, WyKaLds<D>::BYTES, chunks, s, a, b)) != hipSuccess) return e;
+  if ((e = launch_k(wy_kb<D>, WYB_THREADS<D>, WyKbLds<D>::BYTES, chunks, s, a, b)) != hipSuccess) return e;
+  if ((e = launch_k(wy_kc1<D>, WYB_THREADS<D>, WyKc1Lds<D>::BYTES, chunks, s, a, b)) != hipSuccess) return e;
+  return launch_k(wy_kc2<D>, WYB_THREADS<D>, WyKc2Lds<D>::BYTES, chunks, s, a, b);
 }
 
 }  // namespace
