@@ -14,6 +14,7 @@ import threading
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libgmdn_scan.so")
+OPS_PATH = os.path.join(HERE, "libgmdn_ops.so")  # the torch operators over it (csrc/torch_ops.cpp)
 
 GMDN_OK = 0
 PREC_TF32 = 0
@@ -23,6 +24,7 @@ DTYPE_F32 = 1
 
 _lock = threading.Lock()
 _lib = None
+_ops = None
 
 c_f32p = ctypes.c_void_p
 c_i64 = ctypes.c_int64
@@ -75,25 +77,37 @@ SIGNATURES = {
 
 
 def load():
-    """Load (once) and return the native library; raise if it is not built."""
-    global _lib
+    """Load (once) the native library and the torch operators over it, and
+    return the former; raise if they are not built."""
+    global _lib, _ops
     if _lib is not None:
         return _lib
     with _lock:
         if _lib is not None:
             return _lib
-        if not os.path.exists(LIB_PATH):
-            raise RuntimeError(
-                f"gmdn native library not found at {LIB_PATH}; build it with "
-                "`python -m gmdn_amd.build` (or __graft_entry__.build())")
-        import torch  # noqa: F401  -- make torch's HIP runtime the one we bind to
+        for path in (LIB_PATH, OPS_PATH):
+            if not os.path.exists(path):
+                raise RuntimeError(
+                    f"gmdn native library not found at {path}; build it with "
+                    "`python -m gmdn_amd.build` (or __graft_entry__.build())")
+        import torch  # make torch's HIP runtime the one we bind to
         lib = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_GLOBAL)
+        torch.ops.load_library(OPS_PATH)
+        ops_lib = ctypes.CDLL(OPS_PATH)
+        ops_lib.gmdn_ops_set_precision.argtypes = [c_i64]
+        ops_lib.gmdn_ops_set_precision.restype = None
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        _lib = lib
+        _lib, _ops = lib, ops_lib
     return _lib
+
+
+def set_default_precision(code: int) -> None:
+    """The product precision (PREC_*) that the muon core's backward reads."""
+    if available():
+        _ops.gmdn_ops_set_precision(code)
 
 
 def available() -> bool:

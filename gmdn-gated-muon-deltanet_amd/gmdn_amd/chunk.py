@@ -54,7 +54,8 @@ import math
 
 import torch
 
-from . import ops  # noqa: F401  -- registers torch.ops.gmdn.*
+from . import _native as nat
+from . import ops  # registers torch.ops.gmdn.*
 
 RULES = {"delta": 0, "muon": 1, "adam": 2}
 CHUNK = 64
@@ -96,6 +97,8 @@ def _rule_id(rule) -> int:
 def _check(q, k, v, beta, g, gmu, gnu, rule, chunk=CHUNK):
     if not q.is_cuda:
         raise RuntimeError("chunk_scan needs GPU tensors")
+    if not ops.REGISTERED:
+        nat.load()
     if q.dim() != 4 or k.shape != q.shape or v.shape != q.shape:
         raise RuntimeError(f"q, k, v must be (B, H, T, d) of equal shape, got {tuple(q.shape)}, "
                            f"{tuple(k.shape)}, {tuple(v.shape)}")

@@ -40,6 +40,7 @@ def set_precision(name: str) -> None:
     if name not in ("tf32", "ieee"):
         raise ValueError(f"precision must be 'tf32' or 'ieee', got {name!r}")
     _state["precision"] = name
+    nat.set_default_precision(_prec_code())
 
 
 def get_precision() -> str:

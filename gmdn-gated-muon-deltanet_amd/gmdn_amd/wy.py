@@ -35,91 +35,10 @@ import math
 import torch
 
 from . import _native as nat
-from . import ops  # noqa: F401  -- registers torch.ops.gmdn.*
+from . import ops  # registers torch.ops.gmdn.*
 
 CHUNK = 64
 LOG_FLOOR = math.log(1e-6)
-
-
-def _ckpt_numel(q):
-    desc = ops.chunk_desc(q, q, q, q, 0, 0, 1e-6)
-    return max(nat.load().gmdn_wy_fwd_workspace_bytes(desc) // 4, 4)
-
-
-@torch.library.custom_op("gmdn::wy_fwd", mutates_args=(), device_types="cuda")
-def wy_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, g: torch.Tensor,
-           record: bool) -> tuple[torch.Tensor, torch.Tensor]:
-    lib = nat.load()
-    ops._check_tokens(q, k, v)
-    qc, kc, vc = ops._tok(q), ops._tok(k), ops._tok(v)
-    bc, gc = ops._gate(beta), ops._gate(g)
-    o = torch.empty_strided(q.shape, ops._kernel_strides(q), dtype=q.dtype, device=q.device)
-    desc = ops.chunk_desc(qc, kc, vc, o, 0, 0, 1e-6)
-    # the forward's workspace is the backward's checkpoint
-    ws = torch.empty(_ckpt_numel(q), dtype=torch.float32, device=q.device)
-    with torch.cuda.device(q.device):
-        rc = lib.gmdn_wy_fwd(desc, nat.ptr(qc), nat.ptr(kc), nat.ptr(vc), nat.ptr(bc), nat.ptr(gc), nat.ptr(o),
-                             nat.ptr(ws), ws.numel() * 4, nat.stream_of(q))
-    nat.check(rc, "gmdn_wy_fwd")
-    return o, (ws if record else ops._empty(q))
-
-
-@wy_fwd.register_fake
-def _wy_fwd_fake(q, k, v, beta, g, record):
-    o = q.new_empty_strided(q.shape, ops._kernel_strides(q))
-    return o, (q.new_empty((_ckpt_numel(q),), dtype=torch.float32) if record else ops._empty(q))
-
-
-@torch.library.custom_op("gmdn::wy_bwd", mutates_args=(), device_types="cuda")
-def wy_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, g: torch.Tensor,
-           ckpt: torch.Tensor, dO: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor,
-                                                          torch.Tensor]:
-    lib = nat.load()
-    ops._check_tokens(q, k, v)
-    qc, kc, vc = ops._tok(q, dense=True), ops._tok(k, dense=True), ops._tok(v, dense=True)
-    bc, gc = ops._gate(beta), ops._gate(g)
-    dOc = ops._tok(dO.to(q.dtype))
-    dq, dk, dv = (torch.empty_strided(t.shape, t.stride(), dtype=t.dtype, device=t.device) for t in (qc, kc, vc))
-    dbeta, dg = torch.empty_like(bc), torch.empty_like(gc)
-    desc = ops.chunk_desc(qc, kc, vc, dOc, 0, 0, 1e-6)
-    ws = torch.empty(max(lib.gmdn_wy_bwd_workspace_bytes(desc), 16), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
-        rc = lib.gmdn_wy_bwd(desc, nat.ptr(qc), nat.ptr(kc), nat.ptr(vc), nat.ptr(bc), nat.ptr(gc), nat.ptr(ckpt),
-                             nat.ptr(dOc), nat.ptr(dq), nat.ptr(dk), nat.ptr(dv), nat.ptr(dbeta), nat.ptr(dg),
-                             nat.ptr(ws), ws.numel(), nat.stream_of(q))
-    nat.check(rc, "gmdn_wy_bwd")
-    dq, dk, dv = (ops._as_strided_like(d_, t) for d_, t in ((dq, q), (dk, k), (dv, v)))
-    return dq, dk, dv, dbeta, dg
-
-
-@wy_bwd.register_fake
-def _wy_bwd_fake(q, k, v, beta, g, ckpt, dO):
-    dq, dk, dv = (t.new_empty_strided(t.shape, ops._kernel_strides(t)) for t in (q, k, v))
-    return (dq, dk, dv, beta.new_empty(beta.shape, dtype=torch.float32),
-            g.new_empty(g.shape, dtype=torch.float32))
-
-
-def _wy_setup(ctx, inputs, output):
-    q, k, v, beta, g, record = inputs
-    o, ckpt = output
-    ctx.mark_non_differentiable(ckpt)
-    ctx.set_materialize_grads(False)
-    ctx.save_for_backward(q, k, v, beta, g, ckpt)
-    ctx.record = record
-
-
-def _wy_backward(ctx, dO, dckpt):
-    q, k, v, beta, g, ckpt = ctx.saved_tensors
-    if not ctx.record:
-        raise RuntimeError("gmdn::wy_fwd ran without its checkpoint (grad mode was off at the call); "
-                           "it has no backward")
-    if dO is None:
-        dO = torch.zeros_like(q)
-    dq, dk, dv, dbeta, dg = torch.ops.gmdn.wy_bwd(q, k, v, beta, g, ckpt, dO)
-    return dq, dk, dv, dbeta.to(beta.dtype), dg.to(g.dtype), None
-
-
-wy_fwd.register_autograd(_wy_backward, setup_context=_wy_setup)
 
 
 def wy_chunk_terms(q, k, v, beta, g):
@@ -155,6 +74,8 @@ def wy_scan(q, k, v, beta, g):
     """o of the token-exact gated delta rule; see the module docstring."""
     if not q.is_cuda:
         raise RuntimeError("wy_scan needs GPU tensors")
+    if not ops.REGISTERED:
+        nat.load()
     if q.dim() != 4 or k.shape != q.shape or v.shape != q.shape:
         raise RuntimeError(f"q, k, v must be (B, H, T, d) of equal shape, got {tuple(q.shape)}")
     B, H, T, d = q.shape
