@@ -4,7 +4,8 @@
 //
 // One wave owns 512 channels of the (B, T, 3 D) projection output -- 8
 // consecutive channels per lane, so a row is one 16-byte (bf16) load per
-// lane -- over a run of 64 tokens.  The conv's K input rows per output sit
+// lane -- over a run of 64 tokens (forward: fewer where the chip is not
+// filled, front_run).  The conv's K input rows per output sit
 // in a register window that slides one token per step, so every row of y is
 // read once; a head's dh channels are dh / 8 consecutive lanes, and its norm
 // is a shuffle reduction within them.  The backward recomputes the forward
@@ -154,11 +155,11 @@ struct Lane {
 template <typename T, int DH>
 __global__ void __launch_bounds__(64 * FT_WAVES)
 front_fwd(const T* __restrict__ y, const float* __restrict__ w, const float* __restrict__ bias,
-          T* __restrict__ q, T* __restrict__ k, T* __restrict__ v, int T_, int D, int K) {
+          T* __restrict__ q, T* __restrict__ k, T* __restrict__ v, int T_, int D, int K, int run) {
   const int C3 = 3 * D;
-  const int ntiles = (T_ + FT_TOK - 1) / FT_TOK;
+  const int ntiles = (T_ + run - 1) / run;
   const int64_t b = blockIdx.x / ntiles;
-  const int t0 = (int)(blockIdx.x % ntiles) * FT_TOK;
+  const int t0 = (int)(blockIdx.x % ntiles) * run;
   const Lane ln(blockIdx.y * FT_WAVES + (threadIdx.x >> 6), C3, D, K, w, bias);
   T* dst = (ln.part == 0 ? q : ln.part == 1 ? k : v) + b * T_ * (int64_t)D + ln.cc;
   const T* yb = y + b * T_ * (int64_t)C3 + ln.c0;
@@ -175,7 +176,7 @@ front_fwd(const T* __restrict__ y, const float* __restrict__ w, const float* __r
       for (int j = 0; j < FT_LC; ++j) win[s][j] = 0.f;
     }
   }
-  const int t1 = min(t0 + FT_TOK, T_);
+  const int t1 = min(t0 + run, T_);
   for (int tg = t0; tg < t1; tg += FT_GF) {
     // the group's rows in flight together, then the tokens in order
     Raw8<T> rows[FT_GF];
@@ -354,14 +355,26 @@ int check_front(const void* y, const float* w, const float* bias, int64_t B, int
   return GMDN_OK;
 }
 
+// Tokens per wave of the forward.  A wave's run is a serial chain of row
+// groups (one memory latency each), so short runs are faster until the chip
+// has about four waves a CU; past that the three halo rows each run re-reads
+// only cost.  Measured (bf16, D = 1024, 64 -> rule): B1 T1024 27 -> 7.6 us,
+// B1 T64 25 -> 7.0 us; B8 T2048 keeps 64 (48 us).
+int front_run(int64_t B, int64_t T_, int nchunks) {
+  int run = FT_TOK;
+  while (run > FT_GF && B * ((T_ + run - 1) / run) * nchunks < 1024) run /= 2;
+  return run;
+}
+
 template <typename T, int DH>
 hipError_t launch_fwd(const void* y, const float* w, const float* bias, void* q, void* k, void* v, int64_t B,
                       int64_t T_, int32_t D, int32_t K, hipStream_t st) {
-  const int ntiles = (int)((T_ + FT_TOK - 1) / FT_TOK);
   const int nchunks = (3 * D + FT_WC - 1) / FT_WC;
+  const int run = front_run(B, T_, nchunks);
+  const int ntiles = (int)((T_ + run - 1) / run);
   const dim3 grid((unsigned)(B * ntiles), (unsigned)((nchunks + FT_WAVES - 1) / FT_WAVES));
   hipLaunchKernelGGL((front_fwd<T, DH>), grid, dim3(64 * FT_WAVES), 0, st, static_cast<const T*>(y), w, bias,
-                     static_cast<T*>(q), static_cast<T*>(k), static_cast<T*>(v), (int)T_, D, K);
+                     static_cast<T*>(q), static_cast<T*>(k), static_cast<T*>(v), (int)T_, D, K, run);
   return hipGetLastError();
 }
 

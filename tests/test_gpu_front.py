@@ -73,3 +73,20 @@ def test_front_opcheck():
     torch.library.opcheck(torch.ops.gmdn.front_fwd.default, (y, w, b, 64),
                           test_utils=("test_schema", "test_autograd_registration", "test_faketensor",
                                       "test_aot_dispatch_static"))
+
+
+@pytest.mark.parametrize("B,T,D", [(1, 7, 128), (1, 9, 128), (2, 131, 256), (1, 2047, 128), (40, 257, 512)])
+def test_front_forward_run_edges(B, T, D):
+    """The forward's tokens per wave (8 to 64) follow the size: every token's
+    sums are the same whatever run it falls in, so each row equals the same
+    row of a call on the tokens it can see (its own and the three before)."""
+    dev = _dev()
+    gen = torch.Generator().manual_seed(T)
+    y = torch.randn(B, T, 3 * D, generator=gen).to(dev, torch.bfloat16)
+    w, b = torch.randn(3 * D, 1, 4, generator=gen).to(dev), torch.randn(3 * D, generator=gen).to(dev)
+    full = torch.ops.gmdn.front_fwd(y, w, b, 64)
+    for t in {0, 3, 7, 8, T // 2, T - 1} & set(range(T)):
+        lo = max(t - 3, 0)
+        part = torch.ops.gmdn.front_fwd(y[:, lo:t + 1].contiguous(), w, b, 64)
+        for x, p in zip(full, part):
+            assert torch.equal(x[:, t], p[:, -1]), t
