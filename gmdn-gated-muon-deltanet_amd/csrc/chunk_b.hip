@@ -501,6 +501,12 @@ hipError_t chunk_fwd_launch(const ChunkArgs& a, int d, int rule, hipStream_t s) 
   // row-owned state waves: the delta rule, and adam at d = 64 (at d = 128
   // adam's three state tiles per row block exceed that kernel's registers)
   if (rule == 2 && d == 64) return chunk_fwd_adam16_launch(a, d, s);
+  // Up to one 16-row workgroup per CU (256) the chain's latency decides and four
+  // waves a row block are faster: 1.31x to 1.54x at B H d / 16 = 256 and below
+  // (T = 4096).  Past that they queue (one workgroup fills a CU's LDS at d = 128)
+  // and the 32-row kernel is faster: 1.4x at 384 and at 512, 1.25x at d = 64 and
+  // 512.
+  if (rule == 0 && a.B * a.H * (d / 16) <= 256) return chunk_fwd_delta16_launch(a, d, s);
   if (rule == 0) return chunk_fwd_rows_launch(a, d, rule, s);
   return launch_fwd<128, 2>(a, s);
 }

@@ -41,7 +41,7 @@
 //
 // Splitting each row block's state work over two waves (a mid-chunk barrier
 // exchanging the halves of E) measured slower: the output waves became the
-// chain.
+// chain.  Where CUs would be idle, chunk_fwd_delta16 runs instead.
 #include "../../include/gmdn_scan.h"
 #include "chunk_b.h"
 

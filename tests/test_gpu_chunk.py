@@ -70,6 +70,45 @@ def test_delta_multi_head_batch():
     assert err <= TOL
 
 
+@pytest.mark.parametrize("d,B,H,T", [
+    (128, 1, 1, 64), (128, 1, 3, 128), (128, 1, 8, 192), (128, 2, 3, 320), (128, 1, 1, 4224),
+    (128, 2, 16, 128), (128, 1, 33, 128),
+    (64, 1, 1, 64), (64, 1, 5, 128), (64, 1, 8, 192), (64, 1, 3, 320), (64, 1, 2, 4224),
+    (64, 4, 16, 128), (64, 1, 65, 128)])
+def test_delta_few_heads(d, B, H, T):
+    """The 16-row kernel's edges: every remainder of its four-stage ring (1, 2,
+    3 and 5 chunks), 66 chunks (a second block of chunk decays), heads that do
+    and do not spread over the XCDs, and both sides of the 256-workgroup line.
+    The output's own rounding is half an ulp of the largest |o| (2.1e-2 of rms at
+    33 heads), so the bound is on the excess over it: S, E and A are held as 16-bit
+    pairs (2^-17 each), two of them in each product and |o| <= 8 rms, with a factor
+    8 for the chunks a state comes through: 8 * 2 * 8 * 2^-17 = 1e-3."""
+    _, _, excess = _forward(Workload("t", "delta", B, H, T, d), seed=5)
+    assert excess <= 1e-3
+
+
+@pytest.mark.parametrize("d,T", [(128, 192), (128, 256), (64, 192), (64, 320)])
+def test_delta_few_heads_checkpoint(d, T):
+    """The 16-row kernel's checkpoint against the 32-row kernel's (the same
+    head in a launch past the 256-workgroup line).  Both hold hi + lo bfloat16
+    pieces, 16 significant bits: a state differs by a rounding of the pieces
+    (2^-17) per chunk it came through, in relation to the largest state."""
+    dev = _dev()
+    n = 4096 // d + 8
+    inp = make_inputs(Workload("t", "delta", 1, n, T, d), seed=7, with_grad_out=False)
+    a = [inp[k].to(dev) for k in ("q", "k", "v", "beta", "g")]
+    o_all, st_all = torch.ops.gmdn.chunk_fwd(*a, None, None, 0, 3, 1e-6, True)
+    o, st = torch.ops.gmdn.chunk_fwd(*(t[:, :2].contiguous() for t in a), None, None, 0, 3, 1e-6, True)
+
+    def val(t):  # units of four hi and four lo pieces
+        x = t.flatten().view(torch.bfloat16).double().reshape(-1, 2, 4)
+        return x.sum(1)
+
+    x, y = val(st), val(st_all.flatten()[:st.numel()])
+    assert (x - y).abs().max() <= 2.0**-17 * 2 * (T // 64) * y.abs().max()
+    assert ((o.double() - o_all[:, :2].double()).abs().max() / o.double().pow(2).mean().sqrt()) <= TOL
+
+
 def test_gated_delta_full_size():
     """The headline workload B=4, H=16, T=4096, d=128."""
     err, _, _ = _forward(Workload("gated_delta_b4_h16_t4096_d128", "delta", 4, 16, 4096, 128))
