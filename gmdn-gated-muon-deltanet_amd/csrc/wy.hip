@@ -19,7 +19,7 @@
 // and the output is o = Qt S^T + Ov with
 //     Qt = diag(gamma) Q - (M T diag(beta gamma)) K,  Ov = (M T diag(beta)) V.
 //
-// Forward: wy_prep (one workgroup of 8 waves per (b, h, chunk)) forms a, U_A,
+// Forward: wy_prep (one workgroup per (b, h, chunk)) forms a, U_A,
 // K_A, Qt and Ov: bf16 q, k, v enter the products exactly, float32
 // intermediates as split hi + lo bf16 operands; T by blocked forward
 // substitution in float32.  The drop-in delta scan kernels carry S
@@ -30,7 +30,7 @@
 //   wy_gs     gS_i = dL/dS_i through o = dO^T Qt                 (chunk-parallel)
 //   the drop-in delta scan's reverse kernel (split-bf16) on (U_A, K_A, a, S_all,
 //             gS): its dU_i is Sb = dL/dS_{i+1}, the state cotangent after chunk i
-//   wy_tok1 / wy_tok2: the VJP of the chunk algebra in the X-form above, per
+//   wy_ka, wy_kb, wy_kc1, wy_kc2: the VJP of the chunk algebra in the X-form above, per
 //             chunk from S_i and Sb (chunk-parallel):
 //     dX  = M^T dO + diag(kd) K Sb^T,  dQt~ = dO S_i,  dM = lower_incl(dO X^T),
 //     dK~ = X Sb,  dW = -dX S_i,  dgamma_C = <Sb, S_i>,
@@ -40,9 +40,8 @@
 //     then A, M, gamma, kd and Gamma back to q, k, v, beta and the log-gates
 //     (Gamma's exponent differences give dgc_t as row minus column sums of
 //     dGamma * Gamma; dg_u = sum_{t >= u} dgc_t where g_u is above its floor).
-//   wy_tok1 runs up to dT (dv final; partial dq, dk; T, dT, dM and per-token
-//   gate partials to the workspace), wy_tok2 the rest (dA, the A and M terms,
-//   the gate gradients).
+//   Each of the four stages one state tile (S_i or Sb) in LDS; what they hand
+//   on goes through the workspace.
 #include "../../include/gmdn_scan.h"
 #include "chunk_b.h"
 #include "f32mm.h"
@@ -128,7 +127,7 @@ GMDN_DEV void tri_inverse(const float* As, float* Ts, float* Xw_all) {
 }
 
 // ------------------------------------------------------------------ forward
-// wy_prep: one workgroup of 8 waves per (b, h, chunk).  q, k, v stay bf16 in
+// wy_prep: one workgroup of WYP_THREADS per (b, h, chunk).  q, k, v stay bf16 in
 // LDS (row swizzle BSwz) and enter the products exactly; A, T, M and the
 // decays are float32, and every float32 operand of a product is split into
 // hi + lo bf16 (three MFMAs for two split operands, two for one: about
@@ -478,10 +477,10 @@ wy_out(ChunkArgs p, const float* __restrict__ Qt, const float* __restrict__ Ov, 
 }
 
 // ----------------------------------------------------------------- backward
-// Chunk-parallel kernels of 8 waves; intermediates of one chunk pass
+// Chunk-parallel kernels of WYB_THREADS (wy_gs, wy_out: 8 waves); intermediates of one chunk pass
 // through the workspace.  Split-bf16 products as in the forward; S_i and Sb
 // are staged in LDS as split planes (rows r, BSwz), one of them per kernel.
-// Wave w takes token tile tt = w % 4 and the feature part h = w / 4 of
+// Wave w takes token tile tt = w % 4 and the feature part h = w / 4 (of WYB_PARTS) of
 // every C x d result.
 //   wy_gs  gS = dO^T Qt
 //   wy_ka  (S_i)  A, T (to the workspace); W, U; X = U - W S^T;
