@@ -16,9 +16,8 @@
 // (B H D / 16 workgroups, the D/16 of one (b, h) on one XCD).  Two barriers a
 // chunk; interval i runs from barrier i to barrier i + 1.
 //  * State waves 0-3: wave q owns token tile q of E and D/64 column tiles of
-//    the state (D = 128: k-block q, whose pieces it multiplies from its
-//    registers; D = 64: half of k-block q / 2).  E's tile from the published
-//    pieces of Sf = -S, -beta E published | mid-chunk barrier | Sf <- a Sf +
+//    the state (D = 128: k-block q; D = 64: half of k-block q / 2).  E's tile
+//    from the published pieces of Sf = -S, -beta E published | mid-chunk barrier | Sf <- a Sf +
 //    K^T (-beta E) on its columns, its pieces published | barrier.
 //  * Output waves 4-7 (token tiles 0, 1, 3, 2): A^T = K Q^T, packed | mid-chunk
 //    barrier | -o^T = Sf Q^T + (-beta E)^T A^T, stored.  Q rows come straight
@@ -31,10 +30,14 @@
 //
 // What bounds it: LDS reads (~150 KB a chunk at d = 128, ~1200 cycles at 128
 // B/clk) behind two latency chains; 1950 cycles a chunk in all.  So operands
-// that do not depend on the state are read in the half that reads less, each
-// half's reads are all issued before its first product, and no product chain
-// is longer than NKB.  K rows from global memory for the state waves cost more
+// that do not depend on the state are read in the half that reads less, and each
+// half's reads are all issued before its first product.  K rows from global memory for the state waves cost more
 // than the LDS they save (1.3x the time: 64-byte row pieces, 16 lines a load).
+//
+// Every sum (the decay's too) runs in chunk_fwd_rows' order, so that a head's
+// bits do not depend on how many heads the call has.  Two and four shorter
+// chains in place of the 8 and 14 dependent products gained nothing: 103.4
+// against 103.6 us at B 1, H 8, T 8128, d 128.
 //
 // Measured against chunk_fwd_rows (bf16, one launch, infer / with checkpoint):
 // B 1, H 8, T 8128, d 128: 158 -> 104 us / 166 -> 108 us; B 2, H 16, T 4096,
@@ -146,13 +149,19 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
       const int c = 64 * J + l;
       if (cw != 0 || c >= N) return;
       const float* x = p.g + bh * p.T + (int64_t)c * CB_C;
-      float s = 0.f;
+      // wave_sum's order: quads, quads 0 + 3 and 2 + 1 of each 16, then the rows of 16
+      float row[CB_C / 16];
 #pragma unroll
-      for (int k = 0; k < CB_C / 4; ++k) {
-        const f32x4 u = *reinterpret_cast<const f32x4*>(x + 4 * k);
-        s += (fmaxf(u[0], LOG_FLOOR) + fmaxf(u[1], LOG_FLOOR)) + (fmaxf(u[2], LOG_FLOOR) + fmaxf(u[3], LOG_FLOOR));
+      for (int r = 0; r < CB_C / 16; ++r) {
+        float q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const f32x4 u = *reinterpret_cast<const f32x4*>(x + 16 * r + 4 * k);
+          q[k] = (fmaxf(u[0], LOG_FLOOR) + fmaxf(u[1], LOG_FLOOR)) + (fmaxf(u[2], LOG_FLOOR) + fmaxf(u[3], LOG_FLOOR));
+        }
+        row[r] = (q[0] + q[3]) + (q[2] + q[1]);
       }
-      lds_st<float>(L0 + (L::SC0 + (J & 1) * 256 + 4 * l), expf(s));
+      lds_st<float>(L0 + (L::SC0 + (J & 1) * 256 + 4 * l), expf((row[0] + row[1]) + (row[2] + row[3])));
     };
     // the even chunks' checkpoint rows from the staging: lane L = 64 cw + l
     // stores units f = 128 k + L (row f / (D/4), columns 4 u4 .. 4 u4 + 3)
@@ -224,12 +233,12 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
     for (int c = 0; c < CT; ++c)
       ckw[c] = L0 + (L::CK0 + lc * (D / 4) * 16 + 16 * ((8 * kb0 + 2 * G + u0 + c) ^ lc));
 
-    bf16x4 hi[CT], lo[CT];  // the pieces of Sf: at CT = 2 k-block kb0's operand as they stand
-    f32x4 Sf[CT];           // -S, lane (r, G): columns 32 kb0 + 8G + 4 (u0 + c) + j of row r
+    f32x4 Sf[CT];  // -S, lane (r, G): columns 32 kb0 + 8G + 4 (u0 + c) + j of row r
 #pragma unroll
     for (int c = 0; c < CT; ++c) Sf[c] = zero4();
     auto publish_s = [&](int i) {
       const uint32_t par = (uint32_t)(i & 1) * L::SPB;
+      bf16x4 hi[CT], lo[CT];
 #pragma unroll
       for (int c = 0; c < CT; ++c) split4(Sf[c], hi[c], lo[c]);
       if constexpr (CT == 2) {
@@ -244,16 +253,11 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
         for (int c = 0; c < CT; ++c) lds_st<bf16x8>(ckw[c], neg8(cat8(hi[c], lo[c])));
       }
     };
-    // E's operands of a chunk that do not depend on the state; k-blocks kb0,
-    // kb0 + 1, .. (mod NKB)
+    // E's operands of a chunk that do not depend on the state
     lds_cptr rowq[NKB];
-    uint32_t spo[NKB];
 #pragma unroll
-    for (int n = 0; n < NKB; ++n) {
-      const int kb = (kb0 + n) % NKB;
-      rowq[n] = opaque16(L0 + (L::K0 + q * 16 * ROWB + swz_off<LQ>(lc, 32 * kb + 8 * G)));
-      spo[n] = kb * 2048;
-    }
+    for (int kb = 0; kb < NKB; ++kb)
+      rowq[kb] = opaque16(L0 + (L::K0 + q * 16 * ROWB + swz_off<LQ>(lc, 32 * kb + 8 * G)));
     struct Ops {
       bf16x8 Kr[NKB];
       bf16x4 vb;
@@ -263,7 +267,7 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
       constexpr int STG = decltype(stg_tag)::value;
       Ops o;
 #pragma unroll
-      for (int n = 0; n < NKB; ++n) o.Kr[n] = lds_ld<bf16x8>(rowq[n] + STG * L::TILE);
+      for (int kb = 0; kb < NKB; ++kb) o.Kr[kb] = lds_ld<bf16x8>(rowq[kb] + STG * L::TILE);
       o.vb = lds_tr16(vp + STG * L::VT);
       o.bt = lds_ld<f32x4>(bp + STG * L::GT);
       return o;
@@ -275,19 +279,13 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
 
     auto state_chunk = [&](auto stg_tag, int i) {
       constexpr int STG = decltype(stg_tag)::value;
-      // E = V + K Sf^T, token tile q, from every wave's Sf_i pieces (at CT = 2
-      // the wave's own k-block is in its registers)
+      // E = V + K Sf^T, token tile q, from every wave's Sf_i pieces
       const uint32_t so = (uint32_t)(i & 1) * L::SPB;
       bf16x8 Sr[NKB][2];
-      if constexpr (CT == 2) {
-        Sr[0][0] = cat8(hi[0], hi[1]);
-        Sr[0][1] = cat8(lo[0], lo[1]);
-      }
 #pragma unroll
-      for (int n = CT == 2 ? 1 : 0; n < NKB; ++n)
+      for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-        for (int pc = 0; pc < 2; ++pc)
-          Sr[n][pc] = lds_ld<bf16x8>(spr + (so + pc * 1024 + spo[n]));
+        for (int pc = 0; pc < 2; ++pc) Sr[kb][pc] = lds_ld<bf16x8>(spr + (so + kb * 2048 + pc * 1024));
       const float a = lds_ld<float>(L0 + (L::SC0 + ((i >> 6) & 1) * 256 + (i & 63) * 4));
       // the update's K^T operands and chunk i + 1's operands of E (landed since
       // barrier i), read under E's products
@@ -301,14 +299,11 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
       Ops nxt;
       if (i + 1 < N) nxt = load_ops(std::integral_constant<int, (STG + 1) % FE_RING>{});
       __builtin_amdgcn_sched_barrier(0);
-      // the pieces' sums in two chains
-      f32x4 E = zero4(), El = zero4();
+      f32x4 E = f32x4{(float)cur.vb[0], (float)cur.vb[1], (float)cur.vb[2], (float)cur.vb[3]};
 #pragma unroll
-      for (int n = 0; n < NKB; ++n) {
-        E = mfma(cur.Kr[n], Sr[n][0], E);
-        El = mfma(cur.Kr[n], Sr[n][1], El);
-      }
-      E = (f32x4{(float)cur.vb[0], (float)cur.vb[1], (float)cur.vb[2], (float)cur.vb[3]} + E) + El;
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int pc = 0; pc < 2; ++pc) E = mfma(cur.Kr[kb], Sr[kb][pc], E);
 #pragma unroll
       for (int c = 0; c < CT; ++c) Sf[c] = a * Sf[c];
       const uint32_t eo = (uint32_t)(i & 1) * L::EPB;
@@ -397,35 +392,33 @@ __global__ void __launch_bounds__(FE_THREADS) chunk_fwd_delta16(ChunkArgs p) {
       for (int kt = 0; kt < NKT; ++kt) Ap[kt] = pack_tiles<2>(At[2 * kt], At[2 * kt + 1]);
       __builtin_amdgcn_sched_barrier(0);  // A is packed before the barrier
       __syncthreads();  // the mid-chunk barrier of chunk i: -beta E published
-      // -o^T = Sf Q^T + (-beta E)^T A^T, in four chains
+      // -o^T = Sf Q^T + (-beta E)^T A^T
       const uint32_t eo = (uint32_t)(i & 1) * L::EPB, sbo = (uint32_t)(i & 1) * L::SPB;
-      bf16x8 We[2][2];
-#pragma unroll
-      for (int kt = 0; kt < NKT; ++kt)
-#pragma unroll
-        for (int pc = 0; pc < 2; ++pc) We[kt][pc] = lds_ld<bf16x8>(epr + eo + kt * 2048 + pc * 1024);
       bf16x8 Sr[NKB][2];
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int pc = 0; pc < 2; ++pc) Sr[kb][pc] = lds_ld<bf16x8>(spr + sbo + kb * 2048 + pc * 1024);
-      __builtin_amdgcn_sched_barrier(0);
-      f32x4 O[2], P[2];
+      bf16x8 We[2][2];
 #pragma unroll
-      for (int x = 0; x < 2; ++x) O[x] = P[x] = zero4();
+      for (int kt = 0; kt < NKT; ++kt)
+#pragma unroll
+        for (int pc = 0; pc < 2; ++pc) We[kt][pc] = lds_ld<bf16x8>(epr + eo + kt * 2048 + pc * 1024);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4 O = zero4();
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-        for (int pc = 0; pc < 2; ++pc) O[pc] = mfma(Sr[kb][pc], Qr[kb], O[pc]);
+        for (int pc = 0; pc < 2; ++pc) O = mfma(Sr[kb][pc], Qr[kb], O);
       load_q(i + 2, Qr);
       __builtin_amdgcn_sched_barrier(0);
       // (hi, hi), (hi, lo), (lo, hi) of each operand pair
 #pragma unroll
-      for (int pc = 0; pc < 3; ++pc)
+      for (int kt = 0; kt < NKT; ++kt)
 #pragma unroll
-        for (int kt = 0; kt < NKT; ++kt) P[kt] = mfma(We[kt][pc == 2 ? 1 : 0], Ap[kt].v[pc == 1 ? 1 : 0], P[kt]);
+        for (int pc = 0; pc < 3; ++pc) O = mfma(We[kt][pc == 2 ? 1 : 0], Ap[kt].v[pc == 1 ? 1 : 0], O);
       // lane (t, G): token 16 TT + t, state rows 4G ..
-      *reinterpret_cast<bf16x4*>(og + ((int64_t)i * CB_C + 16 * TT + lc) * p.so[2]) = to_bf16x4(-((O[0] + P[0]) + (O[1] + P[1])));
+      *reinterpret_cast<bf16x4*>(og + ((int64_t)i * CB_C + 16 * TT + lc) * p.so[2]) = to_bf16x4(-O);
       __syncthreads();  // barrier i + 1
     };
     // the chunks of a ring turn without branches between them: the compiler

@@ -87,26 +87,19 @@ def test_delta_few_heads(d, B, H, T):
     assert excess <= 1e-3
 
 
-@pytest.mark.parametrize("d,T", [(128, 192), (128, 256), (64, 192), (64, 320)])
+@pytest.mark.parametrize("d,T", [(128, 192), (128, 256), (128, 4224), (64, 192), (64, 320), (64, 4224)])
 def test_delta_few_heads_checkpoint(d, T):
-    """The 16-row kernel's checkpoint against the 32-row kernel's (the same
-    head in a launch past the 256-workgroup line).  Both hold hi + lo bfloat16
-    pieces, 16 significant bits: a state differs by a rounding of the pieces
-    (2^-17) per chunk it came through, in relation to the largest state."""
+    """The 16-row kernel's output and checkpoint are the 32-row kernel's bits
+    (the same head in a launch past the 256-workgroup line): the number of
+    heads in a call does not reach a head's result."""
     dev = _dev()
     n = 4096 // d + 8
     inp = make_inputs(Workload("t", "delta", 1, n, T, d), seed=7, with_grad_out=False)
     a = [inp[k].to(dev) for k in ("q", "k", "v", "beta", "g")]
     o_all, st_all = torch.ops.gmdn.chunk_fwd(*a, None, None, 0, 3, 1e-6, True)
     o, st = torch.ops.gmdn.chunk_fwd(*(t[:, :2].contiguous() for t in a), None, None, 0, 3, 1e-6, True)
-
-    def val(t):  # units of four hi and four lo pieces
-        x = t.flatten().view(torch.bfloat16).double().reshape(-1, 2, 4)
-        return x.sum(1)
-
-    x, y = val(st), val(st_all.flatten()[:st.numel()])
-    assert (x - y).abs().max() <= 2.0**-17 * 2 * (T // 64) * y.abs().max()
-    assert ((o.double() - o_all[:, :2].double()).abs().max() / o.double().pow(2).mean().sqrt()) <= TOL
+    assert torch.equal(o, o_all[:, :2])
+    assert torch.equal(st.flatten().view(torch.int32), st_all.flatten()[:st.numel()].view(torch.int32))
 
 
 def test_gated_delta_full_size():
