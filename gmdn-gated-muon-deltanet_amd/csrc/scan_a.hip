@@ -118,21 +118,15 @@ scan_fwd_rowsf(const float* __restrict__ U, const float* __restrict__ K,
     }
     *reinterpret_cast<f32x4*>(x + rl * LD + 16 * w + 4 * G) = -S;
     __syncthreads();
-    f32x4 g0 = c.u, g1 = zero4();
+    f32x4 g = c.u;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const f32x4 s = *reinterpret_cast<const f32x4*>(x + rl * LD + 16 * t + 4 * G);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (t & 1)
-          g1 = mfma_f32(c.k[t][e], s[e], g1);
-        else
-          g0 = mfma_f32(c.k[t][e], s[e], g0);
-      }
+      for (int e = 0; e < 4; ++e) g = mfma_f32(c.k[t][e], s[e], g);
     }
     const float a = c.a, b = c.b, m = c.m, n = c.n;
     if (i + 2 < N) load(c, i + 2);
-    const f32x4 g = g0 + g1;
     if constexpr (RULE == 0) {
       S = a * S + g;
     } else {
@@ -361,19 +355,13 @@ scan_bwd_rowsf(const float* __restrict__ K, const float* __restrict__ av, const 
     *reinterpret_cast<f32x4*>(x + rl * LD + 16 * w + 4 * G) = -Sb;
     *reinterpret_cast<f32x4*>(dU + base + i * mat + to) = Sb;
     __syncthreads();
-    f32x4 a0 = c.a * Sb + c.gs, a1 = zero4();
+    Sb = c.a * Sb + c.gs;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const f32x4 gb = *reinterpret_cast<const f32x4*>(x + rl * LD + 16 * t + 4 * G);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (t & 1)
-          a1 = mfma_f32(c.k[t][e], gb[e], a1);
-        else
-          a0 = mfma_f32(c.k[t][e], gb[e], a0);
-      }
+      for (int e = 0; e < 4; ++e) Sb = mfma_f32(c.k[t][e], gb[e], Sb);
     }
-    Sb = a0 + a1;
     if (i >= 2) load(c, i - 2);
   };
   Chunk c0, c1;
@@ -393,7 +381,7 @@ scan_bwd_rowsf(const float* __restrict__ K, const float* __restrict__ av, const 
 // update) in step i and by columns (G) in step i + 1, both from one LDS copy
 // (LDS-DMA, two buffers); S_{i-1}'s rows, which every wave reads whole, go
 // through a second exchange like -Gb's.  Per step:
-//   moment VJP of chunk i; -Gb, S_{i-1} and the partial sums to LDS | barrier
+//   moment VJP of chunk i; -Gb, -S_{i-1} and the partial sums to LDS | barrier
 //   Sb^T <- a Sb^T + gS^T - K_i Gb^T                                | barrier
 //   request K_{i-2} into K_i's buffer, and chunk i-2's tiles
 //   G_{i-1}^T = U^T - K_{i-1}^T S_{i-1}^T
@@ -410,7 +398,7 @@ template <int D>
 struct AdamfLds {
   static constexpr int K = 0;                           // two D x D float32 buffers (SwzMat)
   static constexpr int XG = 2 * D * D;                  // -Gb rows
-  static constexpr int XS = XG + RowsfLds<D>::X;        // S rows
+  static constexpr int XS = XG + RowsfLds<D>::X;        // -S rows
   static constexpr int RED = XS + RowsfLds<D>::X;       // [wave][4] partial sums
   static constexpr int BYTES = (RED + D / 16 * 4) * 4;
   static_assert(BYTES <= 160 * 1024, "adam reverse scan LDS exceeds the 160 KiB of a CU");
@@ -461,22 +449,17 @@ scan_bwd_adamf(const float* __restrict__ U, const float* __restrict__ K,
     c.n = nv[sc];
   };
   f32x4 Sb = zero4(), Mb = zero4(), Vb = zero4();
-  // u - K^T S^T of the chunk whose S rows are in the exchange, K_j at kl
-  auto form_g = [&](const f32x4& u, const float* kl) {
-    f32x4 g0 = zero4(), g1 = zero4();
+  // g - K^T S^T of the chunk whose -S rows are in the exchange, K_j at kl
+  auto form_g = [&](f32x4 g, const float* kl) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const f32x4 s = *reinterpret_cast<const f32x4*>(xsr + rl * LD + 16 * t + 4 * G);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float k = kl[L::off(16 * t + 4 * G + e, 16 * w + rl)];
-        if (t & 1)
-          g1 = mfma_f32(k, s[e], g1);
-        else
-          g0 = mfma_f32(k, s[e], g0);
+        g = mfma_f32(kl[L::off(16 * t + 4 * G + e, 16 * w + rl)], s[e], g);
       }
     }
-    return u - (g0 + g1);
+    return g;
   };
 
   // Step i: `c` holds chunk i's pieces, `p` chunk i-1's, g is G_i.  Buffers:
@@ -509,7 +492,7 @@ scan_bwd_adamf(const float* __restrict__ U, const float* __restrict__ K,
     if (l < 4) red[4 * w + l] = l == 0 ? s0[0] : l == 1 ? s0[1] : l == 2 ? s1[0] : s1[1];
     *reinterpret_cast<f32x4*>(dU + base + i * mat + to) = Gb;
     __syncthreads();  // -Gb and the partial sums published; S_i's rows read
-    *reinterpret_cast<f32x4*>(xsr + xo) = p.si;
+    *reinterpret_cast<f32x4*>(xsr + xo) = -p.si;
     if (w == 0 && l < 4) {
       float t = 0.f;
 #pragma unroll
@@ -517,20 +500,14 @@ scan_bwd_adamf(const float* __restrict__ U, const float* __restrict__ K,
       part[((bh * N + i) * NT + blk) * 4 + l] = t;
     }
     const float* kl = smem + R::K + (i & 1) * D * D;
-    f32x4 a0 = c.a * Sb + c.gs, a1 = zero4();
+    Sb = c.a * Sb + c.gs;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const f32x4 k = *reinterpret_cast<const f32x4*>(kl + L::off(16 * w + rl, 16 * t + 4 * G));
       const f32x4 gb = *reinterpret_cast<const f32x4*>(xg + rl * LD + 16 * t + 4 * G);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (t & 1)
-          a1 = mfma_f32(k[e], gb[e], a1);
-        else
-          a0 = mfma_f32(k[e], gb[e], a0);
-      }
+      for (int e = 0; e < 4; ++e) Sb = mfma_f32(k[e], gb[e], Sb);
     }
-    Sb = a0 + a1;
     if (i == 0) return;
     wait_vmem();      // K_{i-1} landed
     __syncthreads();  // K_{i-1} and S_{i-1}'s rows published; K_i, -Gb and the sums read
@@ -545,7 +522,7 @@ scan_bwd_adamf(const float* __restrict__ U, const float* __restrict__ K,
   lds_dma_matrix<D, D * 4>(smem + R::K + ((N - 1) & 1) * D * D, Kb + (N - 1) * mat);
   load(c0, N - 1);
   load(c1, N > 1 ? N - 2 : 0);
-  *reinterpret_cast<f32x4*>(xsr + xo) = c0.si;
+  *reinterpret_cast<f32x4*>(xsr + xo) = -c0.si;
   wait_vmem();
   __syncthreads();
   if (N > 1) lds_dma_matrix<D, D * 4>(smem + R::K + ((N - 2) & 1) * D * D, Kb + (N - 2) * mat);
@@ -834,19 +811,16 @@ scan_bwd_dkf(const float* __restrict__ S_all, const float* __restrict__ dU,
 #pragma unroll 2
   for (int tc = 0; tc < NT; ++tc) {
     const float* const gp = smem + 4 * G * LD + 16 * tc + rl;
-    f32x4 a0 = zero4(), a1 = zero4();
+    f32x4 acc = zero4();
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float gv = gp[(16 * t + e) * LD];
-        if (t & 1)
-          a1 = mfma_f32(gv, s[t][e], a1);
-        else
-          a0 = mfma_f32(gv, s[t][e], a0);
+        acc = mfma_f32(gv, s[t][e], acc);
         if constexpr (RULE == 0) dot += tc == w ? gv * s[t][e] : 0.f;  // da_i = <Gb_i, S_i>
       }
-    *reinterpret_cast<f32x4*>(out + 16 * tc) = -(a0 + a1);
+    *reinterpret_cast<f32x4*>(out + 16 * tc) = -acc;
   }
   if constexpr (RULE == 0) {
     dot = wave_sum(dot);
