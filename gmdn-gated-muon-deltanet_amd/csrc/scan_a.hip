@@ -470,22 +470,25 @@ scan_bwd_adamf(const float* __restrict__ U, const float* __restrict__ K,
     float pda = 0.f, pdb = 0.f, pdm = 0.f, pdn = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      // the moments contracted as in the forward, and nothing across steps
+      // (of two unrolled steps the compiler would fuse one's Mb, Vb only)
+#pragma clang fp contract(off)
       const float gg = g[j];
-      const float Mi = c.m * c.mp[j] + (1.f - c.m) * gg;
-      const float Vi = c.n * c.vp[j] + (1.f - c.n) * gg * gg;
+      const float Mi = fmaf(c.m, c.mp[j], (1.f - c.m) * gg);
+      const float Vi = fmaf(c.n, c.vp[j], (1.f - c.n) * gg * gg);
       const float root = sqrtf(Vi);
       const float den = root + 1e-6f;
       const float sb = Sb[j];
-      pda += sb * c.si[j];
-      pdb += sb * (Mi / den);
+      pda = fmaf(sb, c.si[j], pda);
+      pdb = fmaf(sb, Mi / den, pdb);
       const float ub = c.b * sb;
       const float Mtot = Mb[j] + ub / den;
       const float Vtot = Vb[j] - ub * Mi / (den * den) / (2.f * fmaxf(root, 1e-12f));
-      pdm += Mtot * (c.mp[j] - gg);
-      pdn += Vtot * (c.vp[j] - gg * gg);
+      pdm = fmaf(Mtot, c.mp[j] - gg, pdm);
+      pdn = fmaf(Vtot, fmaf(-gg, gg, c.vp[j]), pdn);
       Mb[j] = c.m * Mtot;
       Vb[j] = c.n * Vtot;
-      Gb[j] = (1.f - c.m) * Mtot + (1.f - c.n) * 2.f * gg * Vtot;
+      Gb[j] = fmaf(1.f - c.m, Mtot, (1.f - c.n) * 2.f * gg * Vtot);
     }
     *reinterpret_cast<f32x4*>(xg + xo) = -Gb;
     const f32x2 s0 = wave_sum2(pda, pdb), s1 = wave_sum2(pdm, pdn);

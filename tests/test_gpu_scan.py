@@ -22,6 +22,7 @@ zeros (the reference's Triton backward leaves them uninitialised).
 import pytest
 import torch
 
+from gmdn_amd import _native as nat
 from oracle import scan as osc
 
 pytestmark = pytest.mark.gpu
@@ -305,3 +306,33 @@ def test_scan_row_kernels_one_chunk(dh, rule):
     grads = torch.autograd.grad(S, ins, torch.ones_like(S))
     for t in (S, *grads):
         assert not t.any()
+
+
+@pytest.mark.parametrize("rule", [0, 2])
+@pytest.mark.parametrize("dh", [32, 64, 128])
+def test_scan_row_kernels_step_parity(dh, rule):
+    """The row scans take two chunks a loop turn: a chunk's results are the
+    same bits in either place of the turn.  Behind a chunk of zeros, and before
+    a chunk with no cotangent, every state, moment and gradient is as without
+    it."""
+    dev = _dev()
+    B, H, N = 1, 3, 4
+    gen = torch.Generator().manual_seed(dh)
+    U, K, *gates = [t.float() for t in osc.make_scan_inputs(B, H, N, 64, dh, generator=gen)]
+    gS = torch.randn(B, H, N, dh, dh, generator=gen)
+
+    def run(front, back):
+        def pad(t, x):
+            shape = (B, H, 1) + tuple(t.shape[3:])
+            parts = [torch.full(shape, x)] * front + [t] + [torch.full(shape, x)] * back
+            return torch.cat(parts, 2).to(dev)
+        ins = [pad(U, 0.), pad(K, 0.)] + [pad(t, 0.5) for t in gates]
+        S, M, V = torch.ops.gmdn.state_scan(*ins, rule, 3, nat.PREC_IEEE, True)
+        grads = torch.ops.gmdn.state_scan_bwd(*ins, S, M, V, pad(gS, 0.), rule, 3, nat.PREC_IEEE)
+        n = 4 if rule == 2 else 1  # delta reads a only
+        return [t[:, :, front:front + N] for t in (S, *grads[:2 + n])]
+
+    want = run(0, 0)
+    for front, back in ((1, 0), (0, 1), (1, 1)):
+        for i, (x, y) in enumerate(zip(run(front, back), want)):
+            assert torch.equal(x, y), (front, back, i)
