@@ -21,6 +21,7 @@
 #include <array>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
@@ -606,4 +607,10 @@ TORCH_LIBRARY_IMPL(gmdn, Autograd, m) {
   m.impl("front_fwd", front_fwd_ad);
   m.impl("gates_fwd", gates_fwd_ad);
   m.impl("head_norm_fwd", head_norm_fwd_ad);
+  // The backward operators have no derivative: differentiating a gradient
+  // taken with create_graph=True raises (unregistered, it would only warn and
+  // drop the operator's terms).
+  for (const char* name : {"state_scan_bwd", "chunk_bwd", "chunk_bwd_muon", "wy_bwd", "front_bwd", "gates_bwd",
+                           "head_norm_bwd"})
+    m.impl(name, torch::autograd::autogradNotImplementedFallback());
 }

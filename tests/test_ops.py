@@ -104,3 +104,48 @@ def test_front_fake_shapes():
         assert all(tuple(t.shape) == (2, 100, 256) and t.dtype == torch.bfloat16 for t in (q, k, v))
         dy, dw, db = torch.ops.gmdn.front_bwd(y, w, b, q, k, v, 128)
         assert dy.shape == y.shape and dw.shape == w.shape and db.shape == b.shape
+
+
+def _meta_ops():
+    """(name, call, differentiable inputs) of every forward operator, on meta tensors."""
+    def t(*shape, dtype=torch.float32):
+        return torch.empty(*shape, device="meta", dtype=dtype, requires_grad=True)
+
+    U, K, a, b, m, n = t(1, 2, 3, 64, 64), t(1, 2, 3, 64, 64), *(t(1, 2, 3) for _ in range(4))
+    q, k, v = (t(1, 2, 128, 64, dtype=torch.bfloat16) for _ in range(3))
+    beta, g, mu, nu = (t(1, 2, 128) for _ in range(4))
+    y, w, bias, hw = t(2, 70, 384), t(384, 1, 4), t(384), t(64)
+    op = torch.ops.gmdn
+    for r in range(3):
+        yield f"state_scan-{r}", lambda *x, r=r: op.state_scan(*x, r, 3, 0, True), (U, K, a, b, m, n)
+    yield "chunk_fwd-delta", lambda *x: op.chunk_fwd(*x, None, None, 0, 3, 1e-6, True), (q, k, v, beta, g)
+    yield "chunk_fwd-muon", lambda *x: op.chunk_fwd(*x, None, 1, 3, 1e-6, True), (q, k, v, beta, g, mu)
+    yield "chunk_fwd-adam", lambda *x: op.chunk_fwd(*x, 2, 3, 1e-6, True), (q, k, v, beta, g, mu, nu)
+    yield "wy_fwd", lambda *x: op.wy_fwd(*x, True), (q, k, v, beta, g)
+    yield "front_fwd", lambda *x: op.front_fwd(*x, 64), (y, w, bias)
+    yield "gates_fwd", lambda x: op.gates_fwd(x, 128, 3), (y,)
+    yield "head_norm_fwd", lambda *x: op.head_norm_fwd(*x, 1e-6), (q, hw)
+
+
+@pytest.mark.parametrize("name", [x[0] for x in _meta_ops()])
+def test_second_derivative_raises(name):
+    """A gradient taken with create_graph=True is usable, and differentiating
+    it again raises: the backward operators have no derivative of their own,
+    and must not drop out of the graph."""
+    _, call, xs = next(x for x in _meta_ops() if x[0] == name)
+    out = call(*xs)
+    out = out[0] if isinstance(out, tuple) else out
+    grads = torch.autograd.grad(out.float().square().sum(), xs, create_graph=True)
+    assert all(g.requires_grad for g in grads)
+    for g in grads:
+        with pytest.raises(RuntimeError, match="not implemented|no autograd formula"):
+            torch.autograd.grad(g.float().square().sum(), xs, retain_graph=True, allow_unused=True)
+
+
+def test_hip_scan_second_derivative_raises(monkeypatch):
+    from gmdn_amd import scan
+    monkeypatch.setattr(scan, "_check_inputs", lambda *x: None)  # (it wants GPU tensors)
+    _, _, xs = next(_meta_ops())
+    grads = torch.autograd.grad(scan.HipScan.apply(*xs, 1, 3).square().sum(), xs[:2], create_graph=True)
+    with pytest.raises(RuntimeError, match="not implemented|no autograd formula"):
+        torch.autograd.grad(grads[0].square().sum(), xs, allow_unused=True)
