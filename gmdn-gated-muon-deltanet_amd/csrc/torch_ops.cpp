@@ -28,6 +28,8 @@
 #include <atomic>
 #include <optional>
 #include <tuple>
+#include <type_traits>
+#include <vector>
 
 namespace {
 
@@ -358,7 +360,16 @@ template <class F>
 auto op(const char* name) {
   return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
 }
-#define GMDN_OP(fn) ([]() -> const auto& { static const auto h = op<decltype(fn)>("gmdn::" #fn); return h; }())
+// A kernel's signature with symbolic integers: a traced size reaches the
+// schema unspecialised, and only the kernels themselves see plain integers.
+template <class F>
+struct Symbolic;
+template <class R, class... A>
+struct Symbolic<R(A...)> {
+  using T = R(std::conditional_t<std::is_same_v<A, int64_t>, c10::SymInt, A>...);
+};
+#define GMDN_OP(fn) \
+  ([]() -> const auto& { static const auto h = op<Symbolic<decltype(fn)>::T>("gmdn::" #fn); return h; }())
 
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
   if (!at::GradMode::is_enabled()) return false;
@@ -371,7 +382,7 @@ OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor()
 
 struct StateScan : torch::autograd::Function<StateScan> {
   static variable_list forward(AutogradContext* ctx, const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b,
-                               const Tensor& m, const Tensor& n, int64_t rule, int64_t ns, int64_t precision,
+                               const Tensor& m, const Tensor& n, c10::SymInt rule, c10::SymInt ns, c10::SymInt precision,
                                bool save) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [S, M, V] = GMDN_OP(state_scan).call(U, K, a, b, m, n, rule, ns, precision, save);
@@ -390,14 +401,14 @@ struct StateScan : torch::autograd::Function<StateScan> {
     const Tensor gS = grads[0].defined() ? grads[0] : at::zeros_like(s[6]);
     auto [dU, dK, da, db, dm, dn] = GMDN_OP(state_scan_bwd)
                                         .call(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], gS,
-                                              ctx->saved_data["rule"].toInt(), ctx->saved_data["ns"].toInt(),
-                                              ctx->saved_data["precision"].toInt());
+                                              ctx->saved_data["rule"].toSymInt(), ctx->saved_data["ns"].toSymInt(),
+                                              ctx->saved_data["precision"].toSymInt());
     return {dU, dK, da, db, dm, dn, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 std::tuple<Tensor, Tensor, Tensor> state_scan_ad(const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b,
-                                                 const Tensor& m, const Tensor& n, int64_t rule, int64_t ns,
-                                                 int64_t precision, bool save) {
+                                                 const Tensor& m, const Tensor& n, c10::SymInt rule, c10::SymInt ns,
+                                                 c10::SymInt precision, bool save) {
   if (!wants_grad({&U, &K, &a, &b, &m, &n})) {
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(state_scan).call(U, K, a, b, m, n, rule, ns, precision, save);
@@ -409,7 +420,7 @@ std::tuple<Tensor, Tensor, Tensor> state_scan_ad(const Tensor& U, const Tensor& 
 struct ChunkFwd : torch::autograd::Function<ChunkFwd> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
                                const Tensor& beta, const Tensor& g, const OptTensor& gmu, const OptTensor& gnu,
-                               int64_t rule, int64_t ns, double eps, bool record) {
+                               c10::SymInt rule, c10::SymInt ns, double eps, bool record) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [o, states] = GMDN_OP(chunk_fwd).call(q, k, v, beta, g, gmu, gnu, rule, ns, eps, record);
     ctx->mark_non_differentiable({states});  // a saved intermediate, as above
@@ -427,7 +438,7 @@ struct ChunkFwd : torch::autograd::Function<ChunkFwd> {
                 "(grad mode was off at the call); it has no backward");
     const auto s = ctx->get_saved_variables();
     const Tensor dO = grads[0].defined() ? grads[0] : at::zeros_like(s[0]);
-    const int64_t rule = ctx->saved_data["rule"].toInt(), ns = ctx->saved_data["ns"].toInt();
+    const c10::SymInt rule = ctx->saved_data["rule"].toSymInt(), ns = ctx->saved_data["ns"].toSymInt();
     const Tensor none;
     if (rule == 1) {
       auto [dq, dk, dv, db, dg, dm] =
@@ -441,8 +452,8 @@ struct ChunkFwd : torch::autograd::Function<ChunkFwd> {
   }
 };
 std::tuple<Tensor, Tensor> chunk_fwd_ad(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& beta,
-                                        const Tensor& g, const OptTensor& gmu, const OptTensor& gnu, int64_t rule,
-                                        int64_t ns, double eps, bool record) {
+                                        const Tensor& g, const OptTensor& gmu, const OptTensor& gnu, c10::SymInt rule,
+                                        c10::SymInt ns, double eps, bool record) {
   const Tensor m = opt(gmu), n = opt(gnu);
   if (!wants_grad({&q, &k, &v, &beta, &g, &m, &n})) {
     at::AutoDispatchBelowADInplaceOrView below;
@@ -484,7 +495,7 @@ std::tuple<Tensor, Tensor> wy_fwd_ad(const Tensor& q, const Tensor& k, const Ten
 
 struct FrontFwd : torch::autograd::Function<FrontFwd> {
   static variable_list forward(AutogradContext* ctx, const Tensor& y, const Tensor& weight, const Tensor& bias,
-                               int64_t dh) {
+                               c10::SymInt dh) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [q, k, v] = GMDN_OP(front_fwd).call(y, weight, bias, dh);
     ctx->save_for_backward({y, weight, bias});
@@ -494,12 +505,12 @@ struct FrontFwd : torch::autograd::Function<FrontFwd> {
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const auto s = ctx->get_saved_variables();
     auto [dy, dw, db] =
-        GMDN_OP(front_bwd).call(s[0], s[1], s[2], g[0], g[1], g[2], ctx->saved_data["dh"].toInt());
+        GMDN_OP(front_bwd).call(s[0], s[1], s[2], g[0], g[1], g[2], ctx->saved_data["dh"].toSymInt());
     return {dy, dw, db, Tensor()};
   }
 };
 std::tuple<Tensor, Tensor, Tensor> front_fwd_ad(const Tensor& y, const Tensor& weight, const Tensor& bias,
-                                                int64_t dh) {
+                                                c10::SymInt dh) {
   if (!wants_grad({&y, &weight, &bias})) {
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(front_fwd).call(y, weight, bias, dh);
@@ -509,7 +520,7 @@ std::tuple<Tensor, Tensor, Tensor> front_fwd_ad(const Tensor& y, const Tensor& w
 }
 
 struct GatesFwd : torch::autograd::Function<GatesFwd> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& y, int64_t heads, int64_t n_gates) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& y, c10::SymInt heads, c10::SymInt n_gates) {
     at::AutoDispatchBelowADInplaceOrView below;
     ctx->save_for_backward({y});
     ctx->saved_data["heads"] = heads;
@@ -518,11 +529,11 @@ struct GatesFwd : torch::autograd::Function<GatesFwd> {
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const auto s = ctx->get_saved_variables();
-    return {GMDN_OP(gates_bwd).call(s[0], g[0], ctx->saved_data["heads"].toInt(), ctx->saved_data["n_gates"].toInt()),
+    return {GMDN_OP(gates_bwd).call(s[0], g[0], ctx->saved_data["heads"].toSymInt(), ctx->saved_data["n_gates"].toSymInt()),
             Tensor(), Tensor()};
   }
 };
-Tensor gates_fwd_ad(const Tensor& y, int64_t heads, int64_t n_gates) {
+Tensor gates_fwd_ad(const Tensor& y, c10::SymInt heads, c10::SymInt n_gates) {
   if (!wants_grad({&y})) {
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(gates_fwd).call(y, heads, n_gates);
@@ -562,26 +573,28 @@ extern "C" __attribute__((visibility("default"))) void gmdn_ops_set_precision(in
 }
 
 TORCH_LIBRARY_FRAGMENT(gmdn, m) {
-  m.def("state_scan(Tensor U, Tensor K, Tensor a, Tensor b, Tensor m, Tensor n, int rule, int ns, int precision, "
-        "bool save_moments) -> (Tensor, Tensor, Tensor)");
+  const std::vector<at::Tag> PT2{at::Tag::pt2_compliant_tag};
+  m.def("state_scan(Tensor U, Tensor K, Tensor a, Tensor b, Tensor m, Tensor n, SymInt rule, SymInt ns, "
+        "SymInt precision, bool save_moments) -> (Tensor, Tensor, Tensor)", PT2);
   m.def("state_scan_bwd(Tensor U, Tensor K, Tensor a, Tensor b, Tensor m, Tensor n, Tensor S_all, Tensor M_all, "
-        "Tensor V_all, Tensor gS, int rule, int ns, int precision) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
-  m.def("chunk_fwd(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, Tensor? gmu, Tensor? gnu, int rule, int ns, "
-        "float eps, bool record) -> (Tensor, Tensor)");
+        "Tensor V_all, Tensor gS, SymInt rule, SymInt ns, SymInt precision) -> "
+        "(Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)", PT2);
+  m.def("chunk_fwd(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, Tensor? gmu, Tensor? gnu, SymInt rule, "
+        "SymInt ns, float eps, bool record) -> (Tensor, Tensor)", PT2);
   m.def("chunk_bwd(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, Tensor? gmu, Tensor? gnu, Tensor states, "
-        "Tensor dO, int rule, int ns, float eps) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
+        "Tensor dO, SymInt rule, SymInt ns, float eps) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)", PT2);
   m.def("chunk_bwd_muon(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, Tensor gmu, Tensor states, Tensor dO, "
-        "int ns, int precision) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
-  m.def("wy_fwd(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, bool record) -> (Tensor, Tensor)");
+        "SymInt ns, SymInt precision) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)", PT2);
+  m.def("wy_fwd(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, bool record) -> (Tensor, Tensor)", PT2);
   m.def("wy_bwd(Tensor q, Tensor k, Tensor v, Tensor beta, Tensor g, Tensor ckpt, Tensor dO) -> "
-        "(Tensor, Tensor, Tensor, Tensor, Tensor)");
-  m.def("front_fwd(Tensor y, Tensor weight, Tensor bias, int dh) -> (Tensor, Tensor, Tensor)");
-  m.def("front_bwd(Tensor y, Tensor weight, Tensor bias, Tensor dq, Tensor dk, Tensor dv, int dh) -> "
-        "(Tensor, Tensor, Tensor)");
-  m.def("gates_fwd(Tensor y, int heads, int n_gates) -> Tensor");
-  m.def("gates_bwd(Tensor y, Tensor dout, int heads, int n_gates) -> Tensor");
-  m.def("head_norm_fwd(Tensor x, Tensor weight, float eps) -> (Tensor, Tensor)");
-  m.def("head_norm_bwd(Tensor x, Tensor weight, Tensor rstd, Tensor dout) -> (Tensor, Tensor)");
+        "(Tensor, Tensor, Tensor, Tensor, Tensor)", PT2);
+  m.def("front_fwd(Tensor y, Tensor weight, Tensor bias, SymInt dh) -> (Tensor, Tensor, Tensor)", PT2);
+  m.def("front_bwd(Tensor y, Tensor weight, Tensor bias, Tensor dq, Tensor dk, Tensor dv, SymInt dh) -> "
+        "(Tensor, Tensor, Tensor)", PT2);
+  m.def("gates_fwd(Tensor y, SymInt heads, SymInt n_gates) -> Tensor", PT2);
+  m.def("gates_bwd(Tensor y, Tensor dout, SymInt heads, SymInt n_gates) -> Tensor", PT2);
+  m.def("head_norm_fwd(Tensor x, Tensor weight, float eps) -> (Tensor, Tensor)", PT2);
+  m.def("head_norm_bwd(Tensor x, Tensor weight, Tensor rstd, Tensor dout) -> (Tensor, Tensor)", PT2);
 }
 
 TORCH_LIBRARY_IMPL(gmdn, CUDA, m) {

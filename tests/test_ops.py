@@ -149,3 +149,28 @@ def test_hip_scan_second_derivative_raises(monkeypatch):
     grads = torch.autograd.grad(scan.HipScan.apply(*xs, 1, 3).square().sum(), xs[:2], create_graph=True)
     with pytest.raises(RuntimeError, match="not implemented|no autograd formula"):
         torch.autograd.grad(grads[0].square().sum(), xs, allow_unused=True)
+
+
+def test_operator_schemas():
+    """Integers are symbolic and every operator is marked safe for torch.compile
+    (only_allow_pt2_compliant_ops refuses the others)."""
+    for name in OPS + ("wy_fwd", "wy_bwd", "gates_fwd", "gates_bwd", "head_norm_fwd", "head_norm_bwd"):
+        op = getattr(torch.ops.gmdn, name).default
+        assert torch.Tag.pt2_compliant_tag in op.tags, name
+        assert ", int " not in str(op._schema), name
+
+
+def test_traced_sizes_stay_symbolic():
+    """A size of a traced input reaches the operators, and the backward's,
+    without being specialised to a number."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    def step(y):
+        y = y.detach().requires_grad_()
+        out = torch.ops.gmdn.gates_fwd(y, y.shape[2] // 3, 3)
+        return torch.autograd.grad(out.sum(), y)
+
+    gm = make_fx(step, tracing_mode="symbolic")(torch.empty(2, 70, 24, device="meta"))
+    nodes = {str(n.target): n for n in gm.graph.nodes if "gmdn" in str(n.target)}
+    assert isinstance(nodes["gmdn.gates_fwd.default"].args[1], torch.fx.Node)
+    assert isinstance(nodes["gmdn.gates_bwd.default"].args[2], torch.fx.Node)
