@@ -11,7 +11,10 @@
 // The autograd kernels sit at the Autograd dispatch key as torch's own
 // autograd functions (saved tensors go through SavedVariable, so saved-tensor
 // hooks apply), and call the operators through the dispatcher, so tracing,
-// fake tensors and functionalisation see the same operators as before.
+// fake tensors and functionalisation see the same operators as before.  Each
+// function's outputs are the differentiable ones only: what the forward saves
+// (moments, checkpoints, 1 / rms) reaches the caller through a pointer, since
+// compiled autograd takes no function with non-differentiable outputs.
 #include "../../include/gmdn_front.h"
 #include "../../include/gmdn_scan.h"
 #include "../../include/gmdn_tail.h"
@@ -381,20 +384,19 @@ Tensor opt(const OptTensor& t) { return t ? *t : Tensor(); }
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); }
 
 struct StateScan : torch::autograd::Function<StateScan> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b,
-                               const Tensor& m, const Tensor& n, c10::SymInt rule, c10::SymInt ns, c10::SymInt precision,
-                               bool save) {
+  static constexpr bool is_traceable = true;
+  static Tensor forward(AutogradContext* ctx, const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b,
+                        const Tensor& m, const Tensor& n, c10::SymInt rule, c10::SymInt ns, c10::SymInt precision,
+                        bool save, std::pair<Tensor, Tensor>* moments) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [S, M, V] = GMDN_OP(state_scan).call(U, K, a, b, m, n, rule, ns, precision, save);
-    // the moment stacks are saved intermediates: no cotangent is formed for
-    // them (materialised zeros would cost a d x d memset per chunk)
-    ctx->mark_non_differentiable({M, V});
+    *moments = {M, V};
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({U, K, a, b, m, n, S, M, V});
     ctx->saved_data["rule"] = rule;
     ctx->saved_data["ns"] = ns;
     ctx->saved_data["precision"] = precision;
-    return {S, M, V};
+    return S;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     const auto s = ctx->get_saved_variables();
@@ -403,7 +405,7 @@ struct StateScan : torch::autograd::Function<StateScan> {
                                         .call(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], gS,
                                               ctx->saved_data["rule"].toSymInt(), ctx->saved_data["ns"].toSymInt(),
                                               ctx->saved_data["precision"].toSymInt());
-    return {dU, dK, da, db, dm, dn, Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dU, dK, da, db, dm, dn, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 std::tuple<Tensor, Tensor, Tensor> state_scan_ad(const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b,
@@ -413,24 +415,28 @@ std::tuple<Tensor, Tensor, Tensor> state_scan_ad(const Tensor& U, const Tensor& 
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(state_scan).call(U, K, a, b, m, n, rule, ns, precision, save);
   }
-  auto r = StateScan::apply(U, K, a, b, m, n, rule, ns, precision, save);
-  return {r[0], r[1], r[2]};
+  std::pair<Tensor, Tensor> moments;
+  Tensor S = StateScan::apply(U, K, a, b, m, n, rule, ns, precision, save, &moments);
+  return {S, moments.first, moments.second};
 }
 
 struct ChunkFwd : torch::autograd::Function<ChunkFwd> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
-                               const Tensor& beta, const Tensor& g, const OptTensor& gmu, const OptTensor& gnu,
-                               c10::SymInt rule, c10::SymInt ns, double eps, bool record) {
+  static constexpr bool is_traceable = true;
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& beta,
+                        const Tensor& g, const OptTensor& gmu, const OptTensor& gnu, c10::SymInt rule, c10::SymInt ns,
+                        double eps, bool record, Tensor* checkpoint) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [o, states] = GMDN_OP(chunk_fwd).call(q, k, v, beta, g, gmu, gnu, rule, ns, eps, record);
-    ctx->mark_non_differentiable({states});  // a saved intermediate, as above
+    *checkpoint = states;
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({q, k, v, beta, g, opt(gmu), opt(gnu), states});
     ctx->saved_data["rule"] = rule;
     ctx->saved_data["ns"] = ns;
     ctx->saved_data["eps"] = eps;
     ctx->saved_data["record"] = record;
-    return {o, states};
+    // a compiled backward is kept for its saved data: another setting, another trace
+    ctx->saved_data["ieee"] = default_precision.load() == GMDN_PREC_IEEE;
+    return o;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     TORCH_CHECK(ctx->saved_data["record"].toBool(),
@@ -443,12 +449,12 @@ struct ChunkFwd : torch::autograd::Function<ChunkFwd> {
     if (rule == 1) {
       auto [dq, dk, dv, db, dg, dm] =
           GMDN_OP(chunk_bwd_muon).call(s[0], s[1], s[2], s[3], s[4], s[5], s[7], dO, ns, default_precision.load());
-      return {dq, dk, dv, db, dg, dm, none, none, none, none, none};
+      return {dq, dk, dv, db, dg, dm, none, none, none, none, none, none};
     }
     auto [dq, dk, dv, db, dg, dm, dn] = GMDN_OP(chunk_bwd)
                                             .call(s[0], s[1], s[2], s[3], s[4], opt(s[5]), opt(s[6]), s[7], dO, rule, ns,
                                                   ctx->saved_data["eps"].toDouble());
-    return {dq, dk, dv, db, dg, s[5].defined() ? dm : none, s[6].defined() ? dn : none, none, none, none, none};
+    return {dq, dk, dv, db, dg, s[5].defined() ? dm : none, s[6].defined() ? dn : none, none, none, none, none, none};
   }
 };
 std::tuple<Tensor, Tensor> chunk_fwd_ad(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& beta,
@@ -459,20 +465,21 @@ std::tuple<Tensor, Tensor> chunk_fwd_ad(const Tensor& q, const Tensor& k, const 
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(chunk_fwd).call(q, k, v, beta, g, gmu, gnu, rule, ns, eps, record);
   }
-  auto r = ChunkFwd::apply(q, k, v, beta, g, gmu, gnu, rule, ns, eps, record);
-  return {r[0], r[1]};
+  Tensor states, o = ChunkFwd::apply(q, k, v, beta, g, gmu, gnu, rule, ns, eps, record, &states);
+  return {o, states};
 }
 
 struct WyFwd : torch::autograd::Function<WyFwd> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
-                               const Tensor& beta, const Tensor& g, bool record) {
+  static constexpr bool is_traceable = true;
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& beta,
+                        const Tensor& g, bool record, Tensor* checkpoint) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [o, ckpt] = GMDN_OP(wy_fwd).call(q, k, v, beta, g, record);
-    ctx->mark_non_differentiable({ckpt});
+    *checkpoint = ckpt;
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({q, k, v, beta, g, ckpt});
     ctx->saved_data["record"] = record;
-    return {o, ckpt};
+    return o;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     TORCH_CHECK(ctx->saved_data["record"].toBool(),
@@ -480,7 +487,7 @@ struct WyFwd : torch::autograd::Function<WyFwd> {
     const auto s = ctx->get_saved_variables();
     const Tensor dO = grads[0].defined() ? grads[0] : at::zeros_like(s[0]);
     auto [dq, dk, dv, db, dg] = GMDN_OP(wy_bwd).call(s[0], s[1], s[2], s[3], s[4], s[5], dO);
-    return {dq, dk, dv, db.to(s[3].scalar_type()), dg.to(s[4].scalar_type()), Tensor()};
+    return {dq, dk, dv, db.to(s[3].scalar_type()), dg.to(s[4].scalar_type()), Tensor(), Tensor()};
   }
 };
 std::tuple<Tensor, Tensor> wy_fwd_ad(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& beta,
@@ -489,11 +496,12 @@ std::tuple<Tensor, Tensor> wy_fwd_ad(const Tensor& q, const Tensor& k, const Ten
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(wy_fwd).call(q, k, v, beta, g, record);
   }
-  auto r = WyFwd::apply(q, k, v, beta, g, record);
-  return {r[0], r[1]};
+  Tensor ckpt, o = WyFwd::apply(q, k, v, beta, g, record, &ckpt);
+  return {o, ckpt};
 }
 
 struct FrontFwd : torch::autograd::Function<FrontFwd> {
+  static constexpr bool is_traceable = true;
   static variable_list forward(AutogradContext* ctx, const Tensor& y, const Tensor& weight, const Tensor& bias,
                                c10::SymInt dh) {
     at::AutoDispatchBelowADInplaceOrView below;
@@ -520,6 +528,7 @@ std::tuple<Tensor, Tensor, Tensor> front_fwd_ad(const Tensor& y, const Tensor& w
 }
 
 struct GatesFwd : torch::autograd::Function<GatesFwd> {
+  static constexpr bool is_traceable = true;
   static Tensor forward(AutogradContext* ctx, const Tensor& y, c10::SymInt heads, c10::SymInt n_gates) {
     at::AutoDispatchBelowADInplaceOrView below;
     ctx->save_for_backward({y});
@@ -542,19 +551,20 @@ Tensor gates_fwd_ad(const Tensor& y, c10::SymInt heads, c10::SymInt n_gates) {
 }
 
 struct HeadNorm : torch::autograd::Function<HeadNorm> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, double eps) {
+  static constexpr bool is_traceable = true;
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, double eps, Tensor* rms) {
     at::AutoDispatchBelowADInplaceOrView below;
     auto [out, rstd] = GMDN_OP(head_norm_fwd).call(x, weight, eps);
-    ctx->mark_non_differentiable({rstd});
+    *rms = rstd;
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({x, weight, rstd});
-    return {out, rstd};
+    return out;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor()};
+    if (!g[0].defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
     const auto s = ctx->get_saved_variables();
     auto [dx, dw] = GMDN_OP(head_norm_bwd).call(s[0], s[1], s[2], g[0]);
-    return {dx, dw, Tensor()};
+    return {dx, dw, Tensor(), Tensor()};
   }
 };
 std::tuple<Tensor, Tensor> head_norm_fwd_ad(const Tensor& x, const Tensor& weight, double eps) {
@@ -562,8 +572,8 @@ std::tuple<Tensor, Tensor> head_norm_fwd_ad(const Tensor& x, const Tensor& weigh
     at::AutoDispatchBelowADInplaceOrView below;
     return GMDN_OP(head_norm_fwd).call(x, weight, eps);
   }
-  auto r = HeadNorm::apply(x, weight, eps);
-  return {r[0], r[1]};
+  Tensor rstd, out = HeadNorm::apply(x, weight, eps, &rstd);
+  return {out, rstd};
 }
 
 }  // namespace

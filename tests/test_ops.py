@@ -174,3 +174,39 @@ def test_traced_sizes_stay_symbolic():
     nodes = {str(n.target): n for n in gm.graph.nodes if "gmdn" in str(n.target)}
     assert isinstance(nodes["gmdn.gates_fwd.default"].args[1], torch.fx.Node)
     assert isinstance(nodes["gmdn.gates_bwd.default"].args[2], torch.fx.Node)
+
+
+@pytest.mark.parametrize("name", [x[0] for x in _meta_ops()])
+def test_compiled_autograd_traces_the_backward(name):
+    """torch's compiled autograd takes every operator's autograd function, and
+    traces again when the product precision has changed."""
+    from gmdn_amd import scan
+    from torch._dynamo import compiled_autograd
+
+    _, call, xs = next(x for x in _meta_ops() if x[0] == name)
+    traces = []
+
+    def compiler(gm):
+        traces.append(gm)
+        return torch.compile(gm, backend=lambda m, _: m.forward, fullgraph=True)
+
+    def step():
+        for t in xs:
+            t.grad = None
+        out = call(*xs)
+        with compiled_autograd._enable(compiler):
+            (out[0] if isinstance(out, tuple) else out).float().sum().backward()
+        assert all(t.grad.shape == t.shape for t in xs)
+
+    torch._dynamo.reset()
+    compiled_autograd.reset()
+    step()
+    step()
+    assert len(traces) == 1
+    if name.startswith("chunk_fwd"):
+        try:
+            scan.set_precision("ieee")
+            step()
+        finally:
+            scan.set_precision("tf32")
+        assert len(traces) == 2
