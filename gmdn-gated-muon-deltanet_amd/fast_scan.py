@@ -12,7 +12,7 @@ mirrors reference ``fast_scan.py``:
   ``set_precision('tf32' | 'ieee')`` (reference :47-56); 'triton' is kept as
   the name of the native (HIP) backend so existing ``--scan triton`` flags
   work, and 'hip' is accepted as an alias.
-* ``HAS_TRITON`` -- True when the native library is loadable (the flag
+* ``HAS_TRITON`` -- True when the native libraries are loadable (the flag
   callers test before requesting the kernel backend, reference :36-41).
 * ``_TritonScan`` -- the autograd op, here the HIP one (reference :334-396).
 * ``scan_eager``, ``manual_backward``, ``_msign_sq``, ``_msign_vjp``,
@@ -230,13 +230,13 @@ def fast_state_scan(U, K, a, b, m, n, rule: int, ns: int) -> torch.Tensor:
     """
     if _BACKEND == "eager":
         return scan_eager(U, K, a, b, m, n, rule, ns)
-    if U.is_cuda and not HAS_NATIVE:
-        raise RuntimeError("GPU tensors need the native gmdn kernels, but libgmdn_scan.so "
-                           "is not built; build it or set_backend('eager') explicitly")
+    if U.is_cuda and not (HAS_NATIVE or _native.available()):
+        raise RuntimeError("GPU tensors need the native gmdn kernels (libgmdn_scan.so, libgmdn_ops.so), which did not "
+                           "load; build them or set_backend('eager') explicitly") from _native.load_error()
     if U.is_cuda and U.shape[-1] in SUPPORTED_DH:
         return hip_state_scan(U, K, a, b, m, n, rule, ns)
     if _BACKEND == "triton":
-        raise RuntimeError("native backend requested but unavailable (needs GPU tensors, libgmdn_scan.so "
+        raise RuntimeError("native backend requested but unavailable (needs GPU tensors, the native libraries "
                            f"and a head dim in {SUPPORTED_DH}; got dh={U.shape[-1]}, "
                            f"device {U.device})")
     return scan_eager(U, K, a, b, m, n, rule, ns)

@@ -1,7 +1,8 @@
 """ctypes binding of ``libgmdn_scan.so`` (the C ABI declared in include/gmdn_scan.h,
 include/gmdn_front.h, include/gmdn_tail.h and include/gmdn_msign.h).
 
-The library is built in-tree by ``gmdn_amd.build`` and loaded after torch, so
+The libraries (it, and ``libgmdn_ops.so`` with the torch operators over it) are
+built in-tree by ``gmdn_amd.build`` and loaded after torch, so
 its HIP runtime dependency (soname ``libamdhip64.so.7``) binds to the runtime
 torch already loaded.  There is no fallback: if the library is missing or a
 call returns an error code, a ``RuntimeError`` is raised.
@@ -25,6 +26,8 @@ DTYPE_F32 = 1
 _lock = threading.Lock()
 _lib = None
 _ops = None
+_precision = PREC_TF32  # what the muon core's backward reads, pushed on loading
+_on_load = []           # called once, when the libraries have loaded
 
 c_f32p = ctypes.c_void_p
 c_i64 = ctypes.c_int64
@@ -96,26 +99,48 @@ def load():
         ops_lib = ctypes.CDLL(OPS_PATH)
         ops_lib.gmdn_ops_set_precision.argtypes = [c_i64]
         ops_lib.gmdn_ops_set_precision.restype = None
+        ops_lib.gmdn_ops_set_precision(_precision)
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        while _on_load:
+            _on_load[0]()
+            del _on_load[0]
         _lib, _ops = lib, ops_lib
     return _lib
 
 
+def when_loaded(fn) -> None:
+    """Call ``fn`` once the libraries are loaded: now, or at the end of the
+    ``load`` that succeeds."""
+    with _lock:
+        if _lib is None:
+            _on_load.append(fn)
+            return
+    fn()
+
+
 def set_default_precision(code: int) -> None:
     """The product precision (PREC_*) that the muon core's backward reads."""
-    if available():
-        _ops.gmdn_ops_set_precision(code)
+    global _precision
+    with _lock:
+        _precision = code
+        if _ops is not None:
+            _ops.gmdn_ops_set_precision(code)
+
+
+def load_error() -> Exception | None:
+    """What ``load`` raises, or None when the libraries are loaded."""
+    try:
+        load()
+    except (RuntimeError, OSError) as e:
+        return e
+    return None
 
 
 def available() -> bool:
-    try:
-        load()
-        return True
-    except (RuntimeError, OSError):
-        return False
+    return load_error() is None
 
 
 def check(rc: int, what: str) -> None:

@@ -54,7 +54,6 @@ import math
 
 import torch
 
-from . import _native as nat
 from . import ops  # registers torch.ops.gmdn.*
 
 RULES = {"delta": 0, "muon": 1, "adam": 2}
@@ -97,8 +96,7 @@ def _rule_id(rule) -> int:
 def _check(q, k, v, beta, g, gmu, gnu, rule, chunk=CHUNK):
     if not q.is_cuda:
         raise RuntimeError("chunk_scan needs GPU tensors")
-    if not ops.REGISTERED:
-        nat.load()
+    ops.ensure()
     if q.dim() != 4 or k.shape != q.shape or v.shape != q.shape:
         raise RuntimeError(f"q, k, v must be (B, H, T, d) of equal shape, got {tuple(q.shape)}, "
                            f"{tuple(k.shape)}, {tuple(v.shape)}")

@@ -27,7 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops  # noqa: F401  -- registers torch.ops.gmdn.*
+from . import ops  # registers torch.ops.gmdn.*
 from .chunk import chunk_scan
 
 
@@ -64,6 +64,7 @@ class FastWeightMixer(nn.Module):
     def front_end(self, x: torch.Tensor):
         """q, k, v (B, H, T, dh) views and the gate streams (B, H, T): beta and
         the log gates clamped at log 1e-6 (train_ablation.py:124-134, 155, 170-175)."""
+        ops.ensure()
         B, T, D = x.shape
         H, dh = self.h, self.dh
         # conv, SiLU and the q / k norms in one HIP kernel per direction

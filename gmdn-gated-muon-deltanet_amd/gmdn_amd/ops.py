@@ -177,11 +177,14 @@ def _head_norm_bwd_fake(x, weight, rstd, dout):
     return torch.empty_like(x, memory_format=torch.contiguous_format), weight.new_empty(weight.shape)
 
 
-# (without the native libraries the operators do not exist: the entry points
-# raise what _native.load raises)
-REGISTERED = nat.available()
-if REGISTERED:
-    for _name, _fake in (
+# Set by _register_fakes.  Without the native libraries the operators do not
+# exist: every entry point calls ensure(), which raises what _native.load raises.
+REGISTERED = False
+
+
+def _register_fakes():
+    global REGISTERED
+    for name, fake in (
             ("state_scan", _state_scan_fake),
             ("state_scan_bwd", _state_scan_bwd_fake),
             ("chunk_fwd", _chunk_fwd_fake),
@@ -196,7 +199,19 @@ if REGISTERED:
             ("head_norm_fwd", _head_norm_fwd_fake),
             ("head_norm_bwd", _head_norm_bwd_fake),
     ):
-        torch.library.register_fake(f"gmdn::{_name}", _fake)
+        torch.library.register_fake(f"gmdn::{name}", fake)
+    REGISTERED = True
+
+
+nat.when_loaded(_register_fakes)
+nat.available()
+
+
+def ensure() -> None:
+    """Load the operators if they are not registered yet (the libraries may
+    have been built after this module's import)."""
+    if not REGISTERED:
+        nat.load()
 
 
 def _dtype_code(t: Tensor) -> int:

@@ -15,7 +15,7 @@ from __future__ import annotations
 import torch
 
 from . import _native as nat
-from . import ops  # noqa: F401  -- registers torch.ops.gmdn.*
+from . import ops  # registers torch.ops.gmdn.*
 
 KERNEL_DH = (32, 64, 128)       # head dims the kernels are built for
 SUPPORTED_DH = (16,) + KERNEL_DH  # 16: zero-padded to 32 on the way in
@@ -71,6 +71,7 @@ def _effective_prec(rule: int, save: bool, prec: int) -> int:
 def _check_inputs(U, K, a, b, m, n, rule, ns):
     if not (U.is_cuda and K.is_cuda):
         raise RuntimeError("HIP scan needs GPU tensors")
+    ops.ensure()
     if U.dim() != 5 or U.shape[-1] != U.shape[-2] or K.shape != U.shape:
         raise RuntimeError(f"U and K must be (B, H, N, dh, dh) with equal shapes, got {tuple(U.shape)}, {tuple(K.shape)}")
     dh = U.shape[-1]

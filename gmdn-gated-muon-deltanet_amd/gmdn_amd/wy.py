@@ -34,7 +34,6 @@ import math
 
 import torch
 
-from . import _native as nat
 from . import ops  # registers torch.ops.gmdn.*
 
 CHUNK = 64
@@ -74,8 +73,7 @@ def wy_scan(q, k, v, beta, g):
     """o of the token-exact gated delta rule; see the module docstring."""
     if not q.is_cuda:
         raise RuntimeError("wy_scan needs GPU tensors")
-    if not ops.REGISTERED:
-        nat.load()
+    ops.ensure()
     if q.dim() != 4 or k.shape != q.shape or v.shape != q.shape:
         raise RuntimeError(f"q, k, v must be (B, H, T, d) of equal shape, got {tuple(q.shape)}")
     B, H, T, d = q.shape
