@@ -58,6 +58,10 @@ Tensor bytes_of(const Tensor& like, size_t n) {
   return at::empty({(int64_t)n}, like.options().dtype(at::kByte));
 }
 
+void check_rank(const Tensor& t, int64_t rank, const char* what) {
+  TORCH_CHECK(t.dim() == rank, what, " must have ", rank, " dimensions, got shape ", t.sizes());
+}
+
 // ------------------------------------------------------------ token streams
 void check_tokens(const Tensor& q, const Tensor& k, const Tensor& v) {
   for (const Tensor* t : {&q, &k, &v}) {
@@ -146,6 +150,7 @@ gmdn_chunk_desc chunk_desc(const Tensor& q, const Tensor& k, const Tensor& v, co
 std::tuple<Tensor, Tensor, Tensor> state_scan(const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b,
                                               const Tensor& m, const Tensor& n, int64_t rule, int64_t ns,
                                               int64_t precision, bool save_moments) {
+  check_rank(U, 5, "U");
   const c10::DeviceGuard g(U.device());
   Tensor S = at::empty_like(U);
   Tensor M = rule != 0 && save_moments ? at::empty_like(U) : none_of(U);
@@ -159,6 +164,7 @@ std::tuple<Tensor, Tensor, Tensor> state_scan(const Tensor& U, const Tensor& K, 
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> state_scan_bwd(
     const Tensor& U, const Tensor& K, const Tensor& a, const Tensor& b, const Tensor& m, const Tensor& n,
     const Tensor& S, const Tensor& M, const Tensor& V, const Tensor& gS_, int64_t rule, int64_t ns, int64_t precision) {
+  check_rank(U, 5, "U");
   const c10::DeviceGuard g(U.device());
   Tensor gS = gS_.to(at::kFloat).contiguous();
   Tensor dU = at::empty_like(U), dK = at::empty_like(K);
@@ -287,6 +293,7 @@ int32_t dtype_code(const Tensor& t) {
 }
 
 std::tuple<Tensor, Tensor, Tensor> front_fwd(const Tensor& y, const Tensor& weight, const Tensor& bias, int64_t dh) {
+  check_rank(y, 3, "y");
   const c10::DeviceGuard guard(y.device());
   const int64_t B = y.size(0), T = y.size(1), C3 = y.size(2), D = C3 / 3, K = weight.size(-1);
   Tensor yc = y.contiguous(), w = weight.reshape({C3, K}).to(at::kFloat).contiguous(),
@@ -300,6 +307,7 @@ std::tuple<Tensor, Tensor, Tensor> front_fwd(const Tensor& y, const Tensor& weig
 }
 std::tuple<Tensor, Tensor, Tensor> front_bwd(const Tensor& y, const Tensor& weight, const Tensor& bias,
                                              const Tensor& dq, const Tensor& dk, const Tensor& dv, int64_t dh) {
+  check_rank(y, 3, "y");
   const c10::DeviceGuard guard(y.device());
   const int64_t B = y.size(0), T = y.size(1), C3 = y.size(2), D = C3 / 3, K = weight.size(-1);
   Tensor yc = y.contiguous(), w = weight.reshape({C3, K}).to(at::kFloat).contiguous(),
@@ -317,6 +325,7 @@ std::tuple<Tensor, Tensor, Tensor> front_bwd(const Tensor& y, const Tensor& weig
 }
 
 Tensor gates_fwd(const Tensor& y, int64_t heads, int64_t n_gates) {
+  check_rank(y, 3, "y");
   const c10::DeviceGuard guard(y.device());
   Tensor yc = y.contiguous(), out = f32_empty(y, {n_gates, y.size(0), heads, y.size(1)});
   check(gmdn_gates_fwd(yc.data_ptr(), fp(out), y.size(0), y.size(1), (int32_t)heads, (int32_t)n_gates, dtype_code(yc),
@@ -325,6 +334,7 @@ Tensor gates_fwd(const Tensor& y, int64_t heads, int64_t n_gates) {
   return out;
 }
 Tensor gates_bwd(const Tensor& y, const Tensor& dout, int64_t heads, int64_t n_gates) {
+  check_rank(y, 3, "y");
   const c10::DeviceGuard guard(y.device());
   Tensor yc = y.contiguous(), dc = dout.to(at::kFloat).contiguous(), dy = at::empty_like(yc);
   check(gmdn_gates_bwd(yc.data_ptr(), fp(dc), dy.data_ptr(), y.size(0), y.size(1), (int32_t)heads, (int32_t)n_gates,
@@ -347,6 +357,7 @@ std::tuple<Tensor, Tensor> head_norm_bwd(const Tensor& x, const Tensor& weight, 
                                          const Tensor& dout) {
   const c10::DeviceGuard guard(x.device());
   const int64_t d = x.size(-1);
+  TORCH_CHECK(d > 0, "head_norm_bwd: rows of x are empty, shape ", x.sizes());
   Tensor xc = x.contiguous(), wc = weight.contiguous(), rc = rstd.contiguous();
   const int64_t rows = xc.numel() / d;
   Tensor dc = dout.to(x.scalar_type()).contiguous(), dx = at::empty_like(xc), dw = f32_empty(x, {d});

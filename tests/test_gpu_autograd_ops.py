@@ -78,3 +78,30 @@ def test_unrecorded_forward_has_no_backward():
     with pytest.raises(RuntimeError, match="failed with code"):
         torch.ops.gmdn.chunk_fwd(*[t.detach()[..., :50, :] if t.dim() == 4 else t.detach() for t in xs], None, None, 0,
                                  3, 1e-6, False)
+
+
+def test_wrong_ranks_are_refused():
+    """An operator that takes its sizes from a tensor's leading dimensions
+    refuses any other rank before it launches; a head norm of empty rows is an
+    error, not a division by zero."""
+    dev = _dev()
+    op = torch.ops.gmdn
+    U, g = torch.zeros(1, 2, 3, 64, 64, device=dev), torch.zeros(1, 2, 3, device=dev)
+    for x in (U[0], U[None]):
+        with pytest.raises(RuntimeError, match="5 dimensions"):
+            op.state_scan(x, x, g, g, g, g, 0, 3, 0, False)
+        with pytest.raises(RuntimeError, match="5 dimensions"):
+            op.state_scan_bwd(x, x, g, g, g, g, x, x, x, x, 0, 3, 0)
+    y, w, b = torch.zeros(2, 70, 384, device=dev), torch.zeros(384, 1, 4, device=dev), torch.zeros(384, device=dev)
+    for x in (y[0], y[None]):
+        with pytest.raises(RuntimeError, match="3 dimensions"):
+            op.front_fwd(x, w, b, 64)
+        with pytest.raises(RuntimeError, match="3 dimensions"):
+            op.front_bwd(x, w, b, y, y, y, 64)
+        with pytest.raises(RuntimeError, match="3 dimensions"):
+            op.gates_fwd(x, 128, 3)
+        with pytest.raises(RuntimeError, match="3 dimensions"):
+            op.gates_bwd(x, x, 128, 3)
+    e = torch.zeros(4, 0, device=dev)
+    with pytest.raises(RuntimeError, match="empty"):
+        op.head_norm_bwd(e, torch.zeros(0, device=dev), torch.zeros(4, device=dev), e)
