@@ -1,4 +1,4 @@
-// The split-precision muon reverse scan's stages as device functions over one
+// The muon reverse scan's stages as device functions over one
 // workgroup each (reference fast_scan.py:107-131 and :158-166), shared by the
 // drop-in scan's backward (scan_muon.hip) and the fused mixer core's muon
 // backward (chunk_bwd.hip), which launch them side by side with their other
@@ -11,12 +11,9 @@
 
 namespace gmdn {
 
-// The backward in two stages on the NSSplit engine (two LDS slots of one
-// split matrix each, A and B).  P = PrecX3 ('tf32'): bf16x3 products
-// throughout.  P = PrecH ('ieee'): half-piece products on scaled values in
-// the Newton-Schulz steps and their VJP, whose operands are bounded (X_k, P_k,
-// Z_k by NSScale; the cotangent by its norm, below), and exact float32
-// products with K_i (float32 copy in B), whose operands are the caller's.
+// The backward in two stages on an engine NSX of block-cooperative products:
+// NSSplit ('tf32', bf16x3) or NSFull ('ieee', exact float32)
+// (two LDS slots of one split matrix each, A and B).
 //
 // muon_pre_body, one workgroup per (b, h, chunk): the forward iterates do
 // not depend on the cotangent, so they are rebuilt for every chunk at once
@@ -86,7 +83,7 @@ struct MuonSegArgs {
 };
 
 // The iterates of chunk j0 + blk % jcur of head blk / jcur.
-template <int D, class P = PrecX3>
+template <int D, class NSX = NSSplit<D>>
 GMDN_DEV void muon_pre_body(const MuonSegArgs& sa, int64_t blk) {
   const float* __restrict__ U = sa.U;
   const float* __restrict__ K = sa.K;
@@ -96,10 +93,8 @@ GMDN_DEV void muon_pre_body(const MuonSegArgs& sa, int64_t blk) {
   float* __restrict__ ws = sa.ws;
   const int64_t BH = sa.BH;
   const int N = sa.N, ns = sa.ns, i0 = sa.j0, ncur = sa.jcur;
-  using NSX = NSSplit<D, P>;
-  using Op = typename P::Op;
-  using PK = std::conditional_t<P::SCALED, PrecF32, PrecX3>;  // the products with K_i
-  using OpK = typename PK::Op;
+  using P = typename NSX::P;
+  using Op = typename NSX::Op;
   constexpr int NT = D / 16, NKB = D / 32, NW = D / 16;
   extern __shared__ __align__(16) float msmem[];
   const lds_ptr SA = lds_base(msmem), SB = SA + NSX::BYTES;
@@ -114,20 +109,15 @@ GMDN_DEV void muon_pre_body(const MuonSegArgs& sa, int64_t blk) {
   const int64_t mat = (int64_t)D * D;
   auto roff = [&](int t) { return (int64_t)(r0 + rl) * D + 16 * t + 4 * G; };
 
-  float* const KB = msmem + NSX::BYTES / 4;  // B as a float32 matrix (SwzMat)
-  if constexpr (P::SCALED)
-    lds_dma_matrix<D, D * 4>(KB, K + si * mat);
-  else
-    NSX::template stage<D * 4>(SB, K + si * mat);
-  OpK Bop[NKB];
+  NSX::template stage<D * 4>(SB, K + si * mat);
+  Op Bop[NKB];
   {
     f32x4 Si[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) Si[t] = *reinterpret_cast<const f32x4*>(S_all + si * mat + roff(t));
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) Bop[kb] = PK::pack(-Si[2 * kb], -Si[2 * kb + 1]);
+    for (int kb = 0; kb < NKB; ++kb) Bop[kb] = P::pack(-Si[2 * kb], -Si[2 * kb + 1]);
   }
-  if constexpr (P::SCALED) wait_vmem();
   __syncthreads();  // K_i staged
   const float gm = mv[si];
   float* WM = W.M(ws, sl, ns);
@@ -137,13 +127,8 @@ GMDN_DEV void muon_pre_body(const MuonSegArgs& sa, int64_t blk) {
   for (int t = 0; t < NT; ++t) {
     f32x4 g = *reinterpret_cast<const f32x4*>(U + si * mat + roff(t));
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      if constexpr (P::SCALED)
-        g = PK::mma(col_op<PK, SwzMat<D>>(KB, 32 * kb, 16 * t), Bop[kb], g);
-      else
-        g = PK::mma(nsx.col(SB, kb, t), Bop[kb], g);
-    }
-    if constexpr (P::SCALED) __builtin_amdgcn_sched_barrier(0);  // a tile's operands at a time
+    for (int kb = 0; kb < NKB; ++kb) g = P::mma(nsx.col(SB, kb, t), Bop[kb], g);
+    if constexpr (std::is_same_v<P, PrecF32>) __builtin_amdgcn_sched_barrier(0);  // a tile's operands at a time
     const f32x4 Mp = *reinterpret_cast<const f32x4*>(M_all + si * mat + roff(t));
     X[t] = gm * Mp + g;
     *reinterpret_cast<f32x4*>(WM + roff(t)) = X[t];
@@ -154,23 +139,15 @@ GMDN_DEV void muon_pre_body(const MuonSegArgs& sa, int64_t blk) {
   const float scale = 1.f / (nf + 1e-7f);
 #pragma unroll
   for (int t = 0; t < NT; ++t) X[t] = X[t] * scale;
-  if constexpr (P::SCALED) {
-    for (int k = 0; k < ns; ++k)
-      nsx.step_scaled(X, SA, SB, NSScale(nf * scale, k), W.X(ws, sl, k), W.Z(ws, sl, ns, k), W.P(ws, sl, ns, k));
-    // X_ns is read for db_i only: float32 rows
-#pragma unroll
-    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(W.X(ws, sl, ns) + roff(t)) = X[t];
-  } else {
-    for (int k = 0; k < ns; ++k) {
-      NSX::store_own(W.X(ws, sl, k), X);
-      nsx.step(X, SA, SB, W.Z(ws, sl, ns, k), W.P(ws, sl, ns, k));
-    }
-    NSX::store_own(W.X(ws, sl, ns), X);
+  for (int k = 0; k < ns; ++k) {
+    NSX::store_own(W.X(ws, sl, k), X);
+    nsx.step(X, SA, SB, W.Z(ws, sl, ns, k), W.P(ws, sl, ns, k));
   }
+  NSX::store_own(W.X(ws, sl, ns), X);
 }
 
 // The reverse pass of head bh over chunks i1 - 1 .. i0.
-template <int D, class P = PrecX3>
+template <int D, class NSX = NSSplit<D>>
 GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
   const float* __restrict__ K = sa.K;
   const float* __restrict__ av = sa.av;
@@ -187,10 +164,8 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
   float* __restrict__ ws = sa.ws;
   const int64_t BH = sa.BH;
   const int N = sa.N, ns = sa.ns, i0 = sa.i0, i1 = sa.i1, xbuf = sa.xbuf;
-  using NSX = NSSplit<D, P>;
-  using Op = typename P::Op;
-  using PK = std::conditional_t<P::SCALED, PrecF32, PrecX3>;  // the products with K_i
-  using OpK = typename PK::Op;
+  using P = typename NSX::P;
+  using Op = typename NSX::Op;
   constexpr int NT = D / 16, NKB = D / 32, NW = D / 16;
   extern __shared__ __align__(16) float msmem[];
   const lds_ptr SA = lds_base(msmem), SB = SA + NSX::BYTES;
@@ -223,14 +198,14 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
   // together and one chunk ahead (at the end of the previous chunk's tail),
   // so that their latency is not exposed at the chunk's start.
   f32x4 Si[NT], Gs[NT];
-  bf16x8 Xn[NT];
+  typename NSX::Piece Xn[NT];
   auto request_start = [&](int i) {
     const int64_t si = bh * N + i;
     const float* Xs = W.X(ws, W.slot(bh, i - i0, xbuf), ns);
 #pragma unroll
     for (int t = 0; t < NT; ++t) Si[t] = *reinterpret_cast<const f32x4*>(S_all + si * mat + roff(t));
 #pragma unroll
-    for (int t = 0; t < NT; ++t) Xn[t] = *reinterpret_cast<const bf16x8*>(Xs + roff(t));
+    for (int t = 0; t < NT; ++t) Xn[t] = *reinterpret_cast<const typename NSX::Piece*>(Xs + roff(t));
 #pragma unroll
     for (int t = 0; t < NT; ++t) Gs[t] = *reinterpret_cast<const f32x4*>(gS + si * mat + roff(t));
   };
@@ -243,7 +218,7 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
     float pda = 0.f, pdb = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const f32x4 Xs = P::SCALED ? __builtin_bit_cast(f32x4, Xn[t]) : unsplit_piece(Xn[t]);
+      const f32x4 Xs = NSX::value(Xn[t]);
       pda += Sb[t][0] * Si[t][0] + Sb[t][1] * Si[t][1] + Sb[t][2] * Si[t][2] + Sb[t][3] * Si[t][3];
       pdb += Sb[t][0] * Xs[0] + Sb[t][1] * Xs[1] + Sb[t][2] * Xs[2] + Sb[t][3] * Xs[3];
     }
@@ -259,32 +234,9 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(WSb + roff(t)) = ga * Sb[t] + Gs[t];
     };
-    // P = PrecH: Xbar enters a VJP step as sx Xbar, sx the power of two that
-    // puts its largest entry in [8, 16).  Its Frobenius norm is then below
-    // 16 D <= 2048 and every entry of the step's intermediates below 26 times
-    // that (|b Bs| <= 4.775 2.4 |Xbar|, |c (Y + Y^T)| <= 2.03 7 |Xbar|), inside
-    // half's 65504, with the low pieces of typical entries normal numbers.
-    // X holds sx Xbar through the steps.
-    float sx = 1.f, x0 = 1.f;
-    auto scale_x = [&] {
-      float mx = 0.f;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(X[t][0]), fabsf(X[t][1])), fmaxf(fabsf(X[t][2]), fabsf(X[t][3]))));
-      mx = block_max<NW>(mx, red);
-      int e = mx > 0.f && mx < INFINITY ? 3 - ilogbf(mx) : 0;
-      e = e > 100 ? 100 : e < -100 ? -100 : e;
-      NSX::scale_all(X, ldexpf(1.f, e));
-      sx = ldexpf(sx, e);
-    };
     if (ns > 0) {
-      if constexpr (P::SCALED) {
-        const float nf = W.norm(ws)[sl];
-        x0 = nf * (1.f / (nf + 1e-7f));
-        scale_x();
-      }
       nsx.publish(SA, X);
-      bf16x8 xs[NT];
+      typename NSX::Piece xs[NT];
       NSX::load_pieces(W.X(ws, sl, ns - 1), xs);
       park_sb();
       nsx.store_pieces(SB, xs);
@@ -311,7 +263,7 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
       // Z_k's and P_k's own rows as pieces, P_k in flight through the first
       // two products (Z_k requested a step ahead, in flight through the last
       // product, measured slower: that product's operand reads wait behind it)
-      bf16x8 zr[NT], pr[NT];
+      typename NSX::Piece zr[NT], pr[NT];
       NSX::load_pieces(W.Z(ws, sl, ns, k), zr);
       NSX::load_pieces(W.P(ws, sl, ns, k), pr);
       {
@@ -322,11 +274,9 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
         for (int tr = 0; tr < NT; ++tr) Bs[tr] = zero4();
         nsx.rowprod_own(SA, SB, Bs);
       }
-      [[maybe_unused]] const NSScale sc(x0, k);
-      if constexpr (P::SCALED) NSX::scale_all(Bs, 1.f / sc.x);
       __builtin_amdgcn_sched_barrier(0);  // keep the phases' operands apart
 #pragma unroll
-      for (int tc = 0; tc < NT; ++tc) Q[tc] = (P::SCALED ? NS_A * sc.z : NS_A) * X[tc];
+      for (int tc = 0; tc < NT; ++tc) Q[tc] = NS_A * X[tc];
       {
         Op Bz[NKB];
         NSX::own_ops(zr, Bz);
@@ -337,7 +287,7 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
       __syncthreads();
       // Bs = Bbar + Bbar^T, the transpose read back from the published copy
 #pragma unroll
-      for (int tr = 0; tr < NT; ++tr) Bs[tr] += NSX::tview(SA, tb, tr);
+      for (int tr = 0; tr < NT; ++tr) Bs[tr] += nsx.tview(SA, tb, tr);
       __syncthreads();  // every transposed read of A done
       nsx.publish(SA, Bs);  // Bs is symmetric
       __syncthreads();
@@ -350,11 +300,10 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
         __builtin_amdgcn_sched_barrier(0);
         NSX::own_ops(pr, Bp);
         nsx.rowprod_all(SA, Bp, Y);
-        if constexpr (P::SCALED) NSX::scale_all(Y, 1.f / sc.p);
       }
       // the next step's X_{k-1} pieces for B (after the last step: the tail's
       // rows), in flight through the Y exchange and the last product
-      bf16x8 xn[NT];
+      typename NSX::Piece xn[NT];
       if constexpr (!LAST) {
         NSX::load_pieces(W.X(ws, sl, k - 1), xn);
       } else {
@@ -366,17 +315,14 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
       {
         Op So[NKB];
 #pragma unroll
-        for (int tr = 0; tr < NT; ++tr) Bs[tr] = NS_B * Bs[tr] + NS_C * (Y[tr] + NSX::tview(SA, tb, tr));
+        for (int tr = 0; tr < NT; ++tr) Bs[tr] = NS_B * Bs[tr] + NS_C * (Y[tr] + nsx.tview(SA, tb, tr));
         NSX::pack_all(Bs, So);
-        if constexpr (P::SCALED) NSX::scale_all(Q, sc.x / sc.z);
         nsx.colprod_all(SB, So, Q);
 #pragma unroll
         for (int tc = 0; tc < NT; ++tc) X[tc] = Q[tc];
-        if constexpr (P::SCALED) NSX::scale_all(X, 1.f / sc.x);
       }
       __syncthreads();  // every read of A and B done
       if constexpr (!LAST) {
-        if constexpr (P::SCALED) scale_x();
         nsx.publish(SA, X);
         nsx.store_pieces(SB, xn);
         __syncthreads();
@@ -387,22 +333,15 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
       vjp_step(0, std::true_type{});
     else
       request_tail();
-    if constexpr (P::SCALED) NSX::scale_all(X, 1.f / sx);
     // ---- 3. normalisation: Mbar = Xbar/nrm - <Xbar, M_i>/nrm^2 * M_i/max(|M_i|, 1e-12)
     const float nf = W.norm(ws)[sl];
     const float nrm = nf + 1e-7f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) Sb[t] = *reinterpret_cast<const f32x4*>(WSb + roff(t));  // a Sb + gS
-    // K_i, for the row reads of the Sb update
-    float* const KB = msmem + NSX::BYTES / 4;  // B as a float32 matrix (SwzMat)
-    if constexpr (P::SCALED)
-      lds_dma_matrix<D, D * 4>(KB, K + si * mat);
-    else
-      NSX::template stage<D * 4>(SB, K + si * mat);
+    NSX::template stage<D * 4>(SB, K + si * mat);  // K_i, for the row reads of the Sb update
     float pdot = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) pdot += X[t][0] * Mi[t][0] + X[t][1] * Mi[t][1] + X[t][2] * Mi[t][2] + X[t][3] * Mi[t][3];
-    if constexpr (P::SCALED) wait_vmem();
     const float dot = block_sum<NW>(pdot, red);     // (its barriers also publish K_i in B)
     const float cM = dot / (nrm * nrm) / fmaxf(nf, 1e-12f);
     // M_{i-1} for dm, in flight through the Sb update
@@ -413,20 +352,11 @@ GMDN_DEV void muon_x3_body(const MuonSegArgs& sa, int64_t bh) {
     const float rn = 1.f / nrm;
 #pragma unroll
     for (int t = 0; t < NT; ++t) Mt[t] = Mb[t] + X[t] * rn - cM * Mi[t];
-    OpK Bg[NKB];
+    Op Bg[NKB];
 #pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) Bg[kb] = PK::pack(-Mt[2 * kb], -Mt[2 * kb + 1]);
+    for (int kb = 0; kb < NKB; ++kb) Bg[kb] = P::pack(-Mt[2 * kb], -Mt[2 * kb + 1]);
     // Sb <- a Sb + gS - Gb K^T : A = K rows
-    if constexpr (P::SCALED) {
-#pragma unroll
-      for (int tr = 0; tr < NT; ++tr) {
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) Sb[tr] = PK::mma(row_op<PK, SwzMat<D>>(KB, 16 * tr, 32 * kb), Bg[kb], Sb[tr]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-      nsx.rowprod_all(SB, Bg, Sb);
-    }
+    nsx.rowprod_all(SB, Bg, Sb);
     __builtin_amdgcn_sched_barrier(0);  // dm's wait for M_{i-1} after the product, not inside it
     float pdm = 0.f;
 #pragma unroll

@@ -37,20 +37,6 @@ GMDN_DEV float block_sum(float x, float* red) {
   return t;
 }
 
-// Largest value of the block (x >= 0); red as for block_sum.
-template <int NW>
-GMDN_DEV float block_max(float x, float* red) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
-  if (lane_id() == 0) red[wave_id()] = x;
-  __syncthreads();
-  float t = 0.f;
-#pragma unroll
-  for (int q = 0; q < NW; ++q) t = fmaxf(t, red[q]);
-  __syncthreads();
-  return t;
-}
-
 // block_sum of two values under one pair of barriers (red: 2 NW floats); each
 // sum is formed in the order block_sum uses
 template <int NW>
@@ -184,27 +170,9 @@ struct NSBlock {
   }
 };
 
-// Scales of a half-piece Newton-Schulz step.  X_0 = M / (|M| + eps) has
-// Frobenius norm x0 <= 1 (below 1/2 only when |M| is not far above eps), and
-// a step grows its singular values at most 3.4445-fold up to about 1.2, so
-// entries of X_k are at most min(1.3, x0 4^k): e_k = max(0, e_0 - 2 k) spare
-// binary places, e_0 = -log2 x0 (at most 24).  Then |X| 2^(12 + e) <= 5400,
-// |P| 2^(12 + 2e) <= 8000 and |Z| = |b P + c P^2| <= 3.5 at 2^(12 + 2e) stay
-// below half's 65504, with the low pieces of typical entries normal numbers.
-struct NSScale {
-  float x, p, z;
-  GMDN_DEV NSScale(float x0, int k) {
-    int e = x0 > 0.f && x0 < 0.5f ? -ilogbf(x0) - 1 : 0;
-    e = (e < 24 ? e : 24) - 2 * k;
-    e = e > 0 ? e : 0;
-    x = ldexpf(1.f, 12 + e);
-    p = z = ldexpf(1.f, 12 + 2 * e);
-  }
-};
-
-// The forward quintic step with split products and the shared matrices kept
-// as split planes in LDS (bf16 pieces, or half pieces of scaled values; hi
-// plane then lo plane, each D x D in the 16-byte-group XOR swizzle RowSwz).  Within every 32 columns
+// The forward quintic step with bf16x3 products and the shared matrices kept
+// as split bf16 planes in LDS (hi plane then lo plane, each D x D in the
+// 16-byte-group XOR swizzle RowSwz).  Within every 32 columns
 // the 4-column blocks are stored in the order 0 4 1 5 2 6 3 7, so the eight
 // values of a row operand in the pair k order of the register operands
 // (columns 4G .. 4G+3 and 16+4G .. 16+4G+3) are one 16-byte row read per
@@ -212,7 +180,7 @@ struct NSScale {
 // publishing wave splits its own rows once.  A row's swizzle depends only on
 // the row modulo 16, so each lane keeps one LDS base per distinct column
 // pattern and row tiles are immediate offsets.
-template <int D, class P_ = PrecX3>
+template <int D>
 struct NSSplit {
   static constexpr int NT = D / 16;
   static constexpr int NKB = D / 32;
@@ -220,8 +188,10 @@ struct NSSplit {
   static constexpr uint32_t BYTES = 2 * PLANE;             // one published matrix
   static constexpr uint32_t ROWB = D * 2;                  // bytes per row of a plane
   using L = RowSwz<D>;
-  using P = P_;  // PrecX3 (bf16 pieces) or PrecH (half pieces of scaled values)
-  using Op = typename P::Op;
+  using P = PrecX3;
+  using Op = P::Op;
+  using Piece = bf16x8;  // four values of a row in global memory: hi and lo
+  static GMDN_DEV f32x4 value(const Piece& x) { return unsplit_piece(x); }
   static_assert(L::MASK < 16, "row tiles of 16 must keep the swizzle");
 
   uint32_t prow[NKB];  // row reads: row lc, columns 32 kb + {4G .. 4G+3, 16+4G .. 16+4G+3}
@@ -269,7 +239,7 @@ struct NSSplit {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       bf16x4 hi, lo;
-      P::split(x[q], hi, lo);
+      split4(x[q], hi, lo);
       lds_st<bf16x4>(m + (dst + q * RSTEP * ROWB), hi);
       lds_st<bf16x4>(m + (dst + q * RSTEP * ROWB + PLANE), lo);
     }
@@ -282,8 +252,8 @@ struct NSSplit {
 #pragma unroll
     for (int c = 0; c < NT; c += 2) {
       bf16x4 h0, l0, h1, l1;
-      P::split(t[c], h0, l0);
-      P::split(t[c + 1], h1, l1);
+      split4(t[c], h0, l0);
+      split4(t[c + 1], h1, l1);
       const bf16x8 hi = cat8(h0, h1), lo = cat8(l0, l1);
       lds_st<bf16x8>(m + ppub[c], hi);
       lds_st<bf16x8>(m + (ppub[c] + PLANE), lo);
@@ -399,11 +369,7 @@ struct NSSplit {
   static GMDN_DEV void store_own(float* g, const f32x4 (&t)[NT]) {
     const int l = lane_id(), row = 16 * wave_id() + (l & 15);
 #pragma unroll
-    for (int c = 0; c < NT; ++c) {
-      bf16x4 hi, lo;
-      P::split(t[c], hi, lo);
-      *reinterpret_cast<bf16x8*>(g + row * D + 16 * c + 4 * (l >> 4)) = cat8(hi, lo);
-    }
+    for (int c = 0; c < NT; ++c) *reinterpret_cast<bf16x8*>(g + row * D + 16 * c + 4 * (l >> 4)) = split_piece(t[c]);
   }
   // operands of the wave's rows from pieces already loaded by load_pieces
   // (register moves only: placed right before their product, they do not
@@ -433,9 +399,11 @@ struct NSSplit {
     const int l = lane_id(), lc = l & 15;
     return off(4 * (l >> 4) + (lc >> 2), 16 * wave_id() + 4 * (lc & 3));
   }
-  static GMDN_DEV f32x4 tview(lds_cptr m, uint32_t tb, int tr) {
+  GMDN_DEV f32x4 tview(lds_cptr m, uint32_t tb, int tr) const {
     const lds_cptr a = m + tb + tr * 16 * ROWB;
-    return P::join(lds_tr16(a), lds_tr16(a + PLANE));
+    const bf16x4 h = lds_tr16(a), o = lds_tr16(a + PLANE);
+    return f32x4{(float)h[0] + (float)o[0], (float)h[1] + (float)o[1], (float)h[2] + (float)o[2],
+                 (float)h[3] + (float)o[3]};
   }
   // One quintic step on the wave's rows XT (D-layout tiles of X^T); the same
   // products as NSBlock::step.  With zst / pst, Z = b P + c P^2 and P = X X^T
@@ -470,43 +438,182 @@ struct NSSplit {
     colprod_all(XM, Bz, XT);
     __syncthreads();
   }
+};
 
-  GMDN_DEV static void scale_all(f32x4 (&t)[NT], float s) {
+// The same engine in exact float32: the shared matrices as float32 in LDS
+// (SwzMat, the bytes of the two planes), operands read straight from them,
+// rows in global memory as float32.  The products of NSBlock, in its order of
+// summation; every operand read is issued PIPE products ahead, as in NSSplit.
+template <int D>
+struct NSFull {
+  static constexpr int NT = D / 16;
+  static constexpr int NKB = D / 32;
+  static constexpr uint32_t ROWB = D * 4;
+  static constexpr uint32_t BYTES = (uint32_t)D * D * 4;
+  using L = SwzMat<D>;
+  using P = PrecF32;
+  using Op = P::Op;
+  using Piece = f32x4;
+  static GMDN_DEV f32x4 value(const Piece& x) { return x; }
+
+  // LDS byte offset of (row r, column c); a row's swizzle depends on r modulo
+  // 16 only, so row tiles are immediate offsets
+  static GMDN_DEV uint32_t off(int r, int c) { return 4 * (uint32_t)L::off(r, c); }
+  static constexpr int NP = NT < 4 ? NT : 4;
+  uint32_t prow[NP];  // row lc, columns 16 t + 4G .., t modulo 4 (the rest is an immediate)
+  uint32_t pcol[4];   // row 4G + s, column lc of column tile 0, without its tile's bits
+  uint32_t ptile[4];  // the bits of column tile t, likewise
+  uint32_t own;       // the wave's first row
+  // column tile t's part of a column read's offset, the lane's rows being 4G + s
+  static GMDN_DEV uint32_t tile_bits(int t) { return (uint32_t)(t ^ (lane_id() >> 4 & L::SW >> 2)) << 6; }
+
+  GMDN_DEV NSFull() {
+    const int l = lane_id(), lc = l & 15, G = l >> 4;
 #pragma unroll
-    for (int c = 0; c < NT; ++c) t[c] = s * t[c];
+    for (int t = 0; t < NP; ++t) prow[t] = off(lc, 16 * t + 4 * G);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) pcol[s] = (4 * G + s) * ROWB + ((((lc >> 2) ^ s) << 4) | 4 * (lc & 3));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) ptile[t] = tile_bits(t);
+    own = 16 * wave_id() * ROWB;
   }
-  // The step on half pieces (PrecH).  X, P and Z enter the products as
-  // sc.x X, sc.p P, sc.z Z (NSScale): power-of-two factors, so scaling and
-  // unscaling are exact, and XT stays unscaled between the steps.  xst: X
-  // itself as the wave's rows in pieces of sc.x X.
-  GMDN_DEV void step_scaled(f32x4 (&XT)[NT], lds_ptr XM, lds_ptr PM, const NSScale& sc, float* xst = nullptr,
-                            float* zst = nullptr, float* pst = nullptr) const {
-    scale_all(XT, sc.x);
+
+  template <int N>
+  static GMDN_DEV void pack_all(const f32x4 (&t)[N], Op (&o)[N / 2]) {
+#pragma unroll
+    for (int kb = 0; kb < N / 2; ++kb) o[kb] = P::pack(t[2 * kb], t[2 * kb + 1]);
+  }
+  // All NTHR threads: a row-major fp32 D x D matrix in global memory -> m
+  template <int NTHR>
+  static GMDN_DEV void stage(lds_ptr m, const float* g) {
+    constexpr int PR = D / 4;  // 16-byte pieces per row
+    static_assert((D * PR) % NTHR == 0 && NTHR % PR == 0 && (NTHR / PR) % 16 == 0,
+                  "pieces split evenly, in row steps that keep the swizzle");
+    const int j = threadIdx.x, r = j / PR, c = (j % PR) * 4;
+    constexpr int NQ = D * PR / NTHR, RSTEP = NTHR / PR;
+    const uint32_t dst = off(r, c);
+    f32x4 x[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) x[q] = *reinterpret_cast<const f32x4*>(g + (r + q * RSTEP) * D + c);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) lds_st<f32x4>(m + (dst + q * RSTEP * ROWB), x[q]);
+  }
+  // the wave's rows 16 w .. 16 w + 15 (D-layout tiles t of M^T) -> m
+  GMDN_DEV void publish(lds_ptr m, const f32x4 (&t)[NT]) const {
+#pragma unroll
+    for (int c = 0; c < NT; ++c) lds_st<f32x4>(m + (prow[c % NP] + own + c / NP * 256), t[c]);
+  }
+  // lane (r, G) takes M[16 tr + r][32 kb + pair(G, s)]
+  GMDN_DEV Op row(lds_cptr m, int tr, int kb) const {
+    const auto half = [&](int t) { return lds_ld<f32x4>(m + prow[t % NP] + (tr * 16 * ROWB + t / NP * 256)); };
+    return P::pack(half(2 * kb), half(2 * kb + 1));
+  }
+  // lane (c, G) takes M[32 kb + pair(G, s)][16 tc + c]
+  GMDN_DEV Op col(lds_cptr m, int kb, int tc) const {
+    Op o;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      o.v[s] = lds_ld<float>(m + pcol[s & 3] + ptile[tc & 3] + ((32 * kb + 16 * (s >> 2)) * ROWB + (tc >> 2) * 256));
+    return o;
+  }
+  static constexpr int PIPE = 2;
+  // acc[tr] += tile [r'][r] = sum_k pub[r'][k] B[k][r]
+  GMDN_DEV void rowprod_all(lds_cptr pub, const Op (&B)[NKB], f32x4 (&acc)[NT]) const {
+    constexpr int NJ = NKB * NT;
+    Op a[PIPE];
+#pragma unroll
+    for (int j = 0; j < PIPE; ++j) a[j] = row(pub, j % NT, j / NT);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const Op cur = a[j % PIPE];
+      if (j + PIPE < NJ) a[j % PIPE] = row(pub, (j + PIPE) % NT, (j + PIPE) / NT);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[j % NT] = P::mma(cur, B[j / NT], acc[j % NT]);
+    }
+  }
+  // rowprod_all with the B operand the wave's own rows of the matrix at bm
+  GMDN_DEV void rowprod_own(lds_cptr pub, lds_cptr bm, f32x4 (&acc)[NT]) const {
+    constexpr int NJ = NKB * NT;
+    Op a[PIPE], b[2];
+    b[0] = row(bm + own, 0, 0);
+#pragma unroll
+    for (int j = 0; j < PIPE; ++j) a[j] = row(pub, j % NT, j / NT);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const Op cur = a[j % PIPE];
+      if (j + PIPE < NJ) a[j % PIPE] = row(pub, (j + PIPE) % NT, (j + PIPE) / NT);
+      if (j % NT == 0 && j / NT + 1 < NKB) b[(j / NT + 1) & 1] = row(bm + own, 0, j / NT + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[j % NT] = P::mma(cur, b[(j / NT) & 1], acc[j % NT]);
+    }
+  }
+  // acc[tc] += tile [c][r] = sum_k pub[k][c] B[k][r]
+  GMDN_DEV void colprod_all(lds_cptr pub, const Op (&B)[NKB], f32x4 (&acc)[NT]) const {
+    constexpr int NJ = NKB * NT;
+    Op a[PIPE];
+#pragma unroll
+    for (int j = 0; j < PIPE; ++j) a[j] = col(pub, j / NT, j % NT);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const Op cur = a[j % PIPE];
+      if (j + PIPE < NJ) a[j % PIPE] = col(pub, (j + PIPE) / NT, (j + PIPE) % NT);
+      __builtin_amdgcn_sched_barrier(0);
+      acc[j % NT] = P::mma(cur, B[j / NT], acc[j % NT]);
+    }
+  }
+  static GMDN_DEV void load_pieces(const float* g, Piece (&pc)[NT]) {
+    const int l = lane_id(), row = 16 * wave_id() + (l & 15);
+#pragma unroll
+    for (int c = 0; c < NT; ++c) pc[c] = *reinterpret_cast<const f32x4*>(g + row * D + 16 * c + 4 * (l >> 4));
+  }
+  GMDN_DEV void store_pieces(lds_ptr m, const Piece (&pc)[NT]) const { publish(m, pc); }
+  static GMDN_DEV void store_own(float* g, const f32x4 (&t)[NT]) {
+    const int l = lane_id(), row = 16 * wave_id() + (l & 15);
+#pragma unroll
+    for (int c = 0; c < NT; ++c) *reinterpret_cast<f32x4*>(g + row * D + 16 * c + 4 * (l >> 4)) = t[c];
+  }
+  static GMDN_DEV void own_ops(const Piece (&pc)[NT], Op (&o)[NKB]) { pack_all(pc, o); }
+  // D-layout tile [r'][r] (r' = 16 tr + .., r = the wave's rows) of the
+  // transpose of the matrix at m: the wave's columns, four rows a lane (tb:
+  // column tile w's bits, `tbase`)
+  static GMDN_DEV uint32_t tbase() { return tile_bits(wave_id()); }
+  GMDN_DEV f32x4 tview(lds_cptr m, uint32_t tb, int tr) const {
+    f32x4 x;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x[s] = lds_ld<float>(m + pcol[s] + tb + tr * 16 * ROWB);
+    return x;
+  }
+  // One quintic step on the wave's rows XT, as NSBlock::step; zst / pst as in
+  // NSSplit::step.
+  GMDN_DEV void step(f32x4 (&XT)[NT], lds_ptr XM, lds_ptr PM, float* zst = nullptr, float* pst = nullptr) const {
     publish(XM, XT);
-    if (xst) store_own(xst, XT);
     __syncthreads();
-    Op Bx[NKB];
-    pack_all(XT, Bx);
     f32x4 Pc[NT];
 #pragma unroll
     for (int tr = 0; tr < NT; ++tr) Pc[tr] = zero4();
-    rowprod_all(XM, Bx, Pc);
-    scale_all(Pc, sc.p / (sc.x * sc.x));
+    {
+      Op Bx[NKB];
+      pack_all(XT, Bx);
+      rowprod_all(XM, Bx, Pc);
+    }
+    // P is symmetric: the column block is also the wave's rows of P
     publish(PM, Pc);
     if (pst) store_own(pst, Pc);
     __syncthreads();
+    f32x4 Z[NT];
+#pragma unroll
+    for (int tr = 0; tr < NT; ++tr) Z[tr] = zero4();
     Op Bp[NKB];
     pack_all(Pc, Bp);
-    // c ((b / c) P + P^2) in units of sc.p^2, then of sc.z
-    scale_all(Pc, (NS_B / NS_C) * sc.p);
-    rowprod_all(PM, Bp, Pc);
-    scale_all(Pc, NS_C * (sc.z / (sc.p * sc.p)));
-    if (zst) store_own(zst, Pc);
+    rowprod_all(PM, Bp, Z);
+#pragma unroll
+    for (int tr = 0; tr < NT; ++tr) Z[tr] = NS_B * Pc[tr] + NS_C * Z[tr];
+    if (zst) store_own(zst, Z);
     Op Bz[NKB];
-    pack_all(Pc, Bz);
-    scale_all(XT, NS_A * sc.z);
+    pack_all(Z, Bz);
+#pragma unroll
+    for (int tc = 0; tc < NT; ++tc) XT[tc] = NS_A * XT[tc];
     colprod_all(XM, Bz, XT);
-    scale_all(XT, 1.f / (sc.x * sc.z));
     __syncthreads();
   }
 };

@@ -43,12 +43,6 @@ struct PrecX3 {
     acc = mfma(a.lo, b.hi, acc);
     return acc;
   }
-  static constexpr bool SCALED = false;
-  static GMDN_DEV void split(const f32x4& x, bf16x4& hi, bf16x4& lo) { split4(x, hi, lo); }
-  static GMDN_DEV f32x4 join(const bf16x4& hi, const bf16x4& lo) {
-    return f32x4{(float)hi[0] + (float)lo[0], (float)hi[1] + (float)lo[1], (float)hi[2] + (float)lo[2],
-                 (float)hi[3] + (float)lo[3]};
-  }
 };
 
 struct PrecF32 {
@@ -75,58 +69,6 @@ struct PrecF32 {
     for (int s = 0; s < 8; ++s) acc = mfma_f32(a.v[s], b.v[s], acc);
     return acc;
   }
-};
-
-// Split half precision: x = hi + lo, both IEEE half (11 significant bits
-// each, so about 2^-23 relative where lo is a normal number), three products
-// a*b ~ ah*bh + ah*bl + al*bh accumulated in float32.  Half has five exponent
-// bits: the operands are scaled by powers of two first (callers: NSSplit's
-// scaled step and the muon reverse scan), the way a block floating point
-// keeps its entries near the top of the range.  The pieces travel in the
-// same containers and LDS planes as bf16 ones.
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-
-GMDN_DEV void split4h(const f32x4& x, bf16x4& hi, bf16x4& lo) {
-  const half4 h = __builtin_convertvector(x, half4);
-  hi = __builtin_bit_cast(bf16x4, h);
-  lo = __builtin_bit_cast(bf16x4, __builtin_convertvector(x - __builtin_convertvector(h, f32x4), half4));
-}
-GMDN_DEV f32x4 mfma_h(const bf16x8& a, const bf16x8& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
-}
-
-struct PrecH {
-  using Op = PrecX3::Op;
-  static constexpr bool SCALED = true;  // operands need power-of-two scales
-  static GMDN_DEV void split(const f32x4& x, bf16x4& hi, bf16x4& lo) { split4h(x, hi, lo); }
-  static GMDN_DEV f32x4 join(const bf16x4& hi, const bf16x4& lo) {
-    return __builtin_convertvector(__builtin_bit_cast(half4, hi), f32x4) +
-           __builtin_convertvector(__builtin_bit_cast(half4, lo), f32x4);
-  }
-  static GMDN_DEV Op pack(const f32x4& t0, const f32x4& t1) {
-    bf16x4 h0, l0, h1, l1;
-    split4h(t0, h0, l0);
-    split4h(t1, h1, l1);
-    return Op{cat8(h0, h1), cat8(l0, l1)};
-  }
-  static GMDN_DEV f32x4 mma(const Op& a, const Op& b, f32x4 acc) {
-    acc = mfma_h(a.hi, b.hi, acc);
-    acc = mfma_h(a.hi, b.lo, acc);
-    acc = mfma_h(a.lo, b.hi, acc);
-    return acc;
-  }
-};
-
-template <int PREC>
-struct PrecSel;
-template <>
-struct PrecSel<0> {
-  using T = PrecX3;
-};
-template <>
-struct PrecSel<1> {
-  using T = PrecF32;
 };
 
 // ------------------------------------------------ swizzled fp32 LDS matrix

@@ -25,9 +25,10 @@ hipError_t scan_bwd_dk_launch(const ScanArgs& s, const float* part);
 hipError_t scan_fwd_muon_launch(const ScanArgs& s);
 hipError_t scan_bwd_muon_launch(const ScanArgs& s, float* ws, int64_t ws_floats);
 
-// workspace floats per (b, h) of the fp32 ('ieee') muon backward: 4 + ns matrices
+// workspace floats per (b, h) of the muon backward chunk by chunk ('ieee' at
+// dh = 32, or where less than a one-chunk segment is given): 4 + ns matrices
 __host__ __device__ inline int64_t muon_bwd_ws_floats(int dh, int ns) { return (int64_t)(4 + ns) * dh * dh; }
-// The bf16x3 muon backward keeps, per chunk of a segment, the iterates
+// The segmented muon backward keeps, per chunk of a segment, the iterates
 // X_0 .. X_ns, the products Z_0 .. Z_{ns-1}, P_0 .. P_{ns-1} and M_i
 // (3 ns + 2 matrices) and |M_i|, in nbuf buffers (two let one segment's
 // iterates be formed while the previous segment's reverse pass runs); per
@@ -55,7 +56,7 @@ inline MuonBwdPlan muon_bwd_plan(int64_t BH, int64_t N, int dh, int ns, int64_t 
 }
 // The default workspace: two buffers of segments of as many chunks as fit in
 // MUON_BWD_WS_BUDGET bytes each (at least one chunk; one buffer of all N
-// chunks if they fit), or the fp32 kernel's per-(b, h) matrices if larger.
+// chunks if they fit), or the chunk-by-chunk kernel's matrices if larger.
 constexpr int64_t MUON_BWD_WS_BUDGET = (int64_t)512 << 20;
 inline int64_t muon_bwd_ws_total(int64_t BH, int64_t N, int dh, int ns) {
   const int64_t mat = (int64_t)dh * dh;

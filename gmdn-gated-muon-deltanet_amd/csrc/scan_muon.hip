@@ -4,24 +4,21 @@
 // M (D-layout tiles of the transposes) and the waves cooperate on the
 // Newton-Schulz iterations through shared matrices.
 //
-// Forward: X and P live in LDS as split planes of the Newton-Schulz engine
-// (NSSplit): bf16 pieces for 'tf32', half pieces of scaled values for 'ieee'
-// at D >= 64.  ('ieee' at D = 32, which serves d = 16 too, keeps exact float32
-// products, NSBlock: sums that short round so little in float32 that the
-// pieces' 2^-23 shows, 1.5 times its error at d = 16 where D >= 64 measures
-// 0.7 to 1.0 times.)
-// K_i is staged in the P store before the first step publishes P: split
-// planes ('tf32'), or float32 for exact products ('ieee').
+// Forward: X and P live in LDS (2 D^2 fp32 worth) in the Newton-Schulz
+// engine's layout: split bf16 planes for the bf16x3 precision (NSSplit),
+// swizzled float32 for the exact one (NSFull).  K_i is staged in the P store
+// before the first step publishes P.
 // Backward: the stages of muon_bwd.h (iterate rebuild, serial reverse scan)
-// in either precision; scan_bwd_muon_seg runs them a segment at a time.  An
+// on either engine; scan_bwd_muon_seg runs them a segment at a time.  An
 // 'ieee' caller whose workspace holds less than one chunk's iterates (4 + ns
-// matrices per (b, h) are accepted), and D = 32, get scan_bwd_muon: exact
-// float32 products through four matrices in that workspace.
-// 'ieee' measured (8 heads, 8 chunks, d = 128, ns = 3): forward 946 -> 333 us,
-// backward 10.1 ms -> 0.58 ms against float32 MFMAs (1/16 of the half rate)
-// through a global workspace; error against float64 0.55 to 1.0 times the
-// float32 products' (the 32-term half MFMA rounds its sum once, eight
-// float32 MFMAs eight times).
+// matrices per (b, h) are accepted), and D = 32, get scan_bwd_muon: the same
+// float32 products, chunk after chunk, through four matrices in that
+// workspace.
+// 'ieee' is bound by the float32 MFMAs (1/16 of the bfloat16 rate): 20.5 us
+// of them a Newton-Schulz step at D = 128, 61 of a chunk's 79 us at ns = 3.
+// Measured (8 heads, 8 chunks, D = 128, ns = 3) against P through four
+// matrices in a global workspace, everything serial: forward 946 -> 631 us,
+// backward 10.1 -> 1.02 ms, the forward's bits the same.
 #include "muon_bwd.h"
 #include "ns.h"
 #include "scan_a.h"
@@ -36,8 +33,8 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
               const float* __restrict__ av, const float* __restrict__ bv,
               const float* __restrict__ mv, float* __restrict__ S_all,
               float* __restrict__ M_all, int N, int ns) {
-  using P = typename PrecSel<PREC>::T;                          // products with K_i
-  using NSX = NSSplit<D, std::conditional_t<PREC == 0, PrecX3, PrecH>>;  // Newton-Schulz products
+  using NSX = std::conditional_t<PREC == 0, NSSplit<D>, NSFull<D>>;
+  using P = typename NSX::P;
   constexpr int NT = D / 16, NKB = D / 32, NW = D / 16;
   extern __shared__ __align__(16) float smem[];
   __shared__ float red[NW];
@@ -53,16 +50,12 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
   for (int t = 0; t < NT; ++t) S[t] = M[t] = zero4();
   const NSX nsx;  // per-lane LDS bases of the engine
   const lds_ptr base = lds_base(smem), KP = base + NSX::BYTES;
-  float* const KF = smem + NSX::BYTES / 4;
 
   for (int i = 0; i < N; ++i) {
     const int64_t si = bh * N + i;
     const float* Ki = K + si * mat;
     // K_i into the P store (free until the first NS step publishes P)
-    if constexpr (PREC == 0)
-      NSX::template stage<D * 4>(KP, Ki);
-    else
-      lds_dma_matrix<D, D * 4>(KF, Ki);
+    NSX::template stage<D * 4>(KP, Ki);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       *reinterpret_cast<f32x4*>((S_all + si * mat + roff(t))) = S[t];
@@ -72,35 +65,22 @@ scan_fwd_muon(const float* __restrict__ U, const float* __restrict__ K,
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) Bop[kb] = P::pack(-S[2 * kb], -S[2 * kb + 1]);
     const float a = av[si], b = bv[si], m = mv[si];
-    if constexpr (PREC != 0) wait_vmem();
     __syncthreads();
     float sq = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       f32x4 g = *reinterpret_cast<const f32x4*>((U + si * mat + roff(t)));
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        if constexpr (PREC == 0)
-          g = P::mma(nsx.col(KP, kb, t), Bop[kb], g);
-        else
-          g = P::mma(col_op<P, SwzMat<D>>(KF, 32 * kb, 16 * t), Bop[kb], g);
-      }
+      for (int kb = 0; kb < NKB; ++kb) g = P::mma(nsx.col(KP, kb, t), Bop[kb], g);
       if constexpr (PREC != 0) __builtin_amdgcn_sched_barrier(0);  // a tile's operands at a time
       M[t] = m * M[t] + g;
       sq += M[t][0] * M[t][0] + M[t][1] * M[t][1] + M[t][2] * M[t][2] + M[t][3] * M[t][3];
     }
-    const float nf = sqrtf(block_sum<NW>(sq, red));
-    const float scale = 1.f / (nf + 1e-7f);
+    const float scale = 1.f / (sqrtf(block_sum<NW>(sq, red)) + 1e-7f);
     f32x4 X[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) X[t] = M[t] * scale;
-    if constexpr (PREC == 0) {
-      for (int s = 0; s < ns; ++s) nsx.step(X, base, KP);
-    } else if constexpr (D == 32) {
-      for (int s = 0; s < ns; ++s) NSBlock<PrecF32, SwzMat<D>, D>::step(X, smem, KF);
-    } else {
-      for (int s = 0; s < ns; ++s) nsx.step_scaled(X, base, KP, NSScale(nf * scale, s));
-    }
+    for (int s = 0; s < ns; ++s) nsx.step(X, base, KP);
 #pragma unroll
     for (int t = 0; t < NT; ++t) S[t] = a * S[t] + b * X[t];
     if (ns == 0) __syncthreads();  // K_i read before the next chunk's copy (a step ends with a barrier)
@@ -233,13 +213,13 @@ scan_bwd_muon(const float* __restrict__ U, const float* __restrict__ K,
 
 // Blocks 0 .. nx3 - 1: the reverse pass of their head over segment [i0, i1);
 // the rest: the iterates of one chunk of segment [j0, j0 + jcur) each.
-template <int D, class P>
+template <int D, class NSX>
 __global__ void __launch_bounds__(D * 4) scan_bwd_muon_seg(MuonSegArgs sa) {
   const int64_t b = blockIdx.x;
   if (b < sa.nx3)
-    muon_x3_body<D, P>(sa, b);
+    muon_x3_body<D, NSX>(sa, b);
   else
-    muon_pre_body<D, P>(sa, b - sa.nx3);
+    muon_pre_body<D, NSX>(sa, b - sa.nx3);
 }
 
 template <int D, int PREC>
@@ -253,56 +233,59 @@ static hipError_t launch_fwd_muon(const ScanArgs& s) {
   return hipGetLastError();
 }
 
+template <int D, class NSX>
+static hipError_t launch_bwd_muon_seg(const ScanArgs& s, float* ws, const MuonBwdPlan& plan) {
+  const int lds = 2 * NSX::BYTES + 64;
+  auto k = scan_bwd_muon_seg<D, NSX>;
+  hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return e;
+  // Segments of nseg chunks from the end; Sb and Mbar carry from one
+  // segment's reverse pass to the next through the workspace.  With two
+  // iterate buffers the iterates of segment k + 1 are formed in the launch
+  // that runs segment k's reverse pass (only the first segment's run
+  // alone); with one, each segment's iterates and then its reverse pass.
+  if (plan.nseg < 1) return hipErrorInvalidValue;
+  const int nseg = (int)plan.nseg;
+  MuonSegArgs sa{};
+  sa.U = s.U; sa.K = s.K; sa.av = s.a; sa.bv = s.b; sa.mv = s.m; sa.S_all = s.S_all; sa.M_all = s.M_all;
+  sa.gS = s.gS; sa.dU = s.dU; sa.da = s.da; sa.db = s.db; sa.dm = s.dm; sa.dn = s.dn; sa.ws = ws;
+  sa.BH = s.BH; sa.N = (int)s.N; sa.ns = s.ns; sa.nseg = nseg; sa.nbuf = plan.nbuf;
+  auto launch = [&](int nx3, int i0, int i1, int xbuf, int j0, int jcur, int pbuf) {
+    sa.nx3 = nx3; sa.i0 = i0; sa.i1 = i1; sa.xbuf = xbuf;
+    sa.j0 = j0; sa.jcur = jcur; sa.pbuf = pbuf;
+    const int64_t blocks = (int64_t)nx3 + s.BH * jcur;
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(D * 4), lds, s.stream, sa);
+    return hipGetLastError();
+  };
+  const int bh = (int)s.BH;
+  int i1 = (int)s.N, i0 = i1 > nseg ? i1 - nseg : 0;
+  if (plan.nbuf == 2) {
+    e = launch(0, 0, 0, 0, i0, i1 - i0, 0);
+    for (int seg = 0; e == hipSuccess && i1 > 0; ++seg) {
+      const int j1 = i0, j0 = j1 > nseg ? j1 - nseg : 0;
+      e = launch(bh, i0, i1, seg & 1, j0, j1 - j0, (seg + 1) & 1);
+      i1 = i0;
+      i0 = j0;
+    }
+  } else {
+    for (; e == hipSuccess && i1 > 0; i1 = i0, i0 = i1 > nseg ? i1 - nseg : 0) {
+      e = launch(0, 0, 0, 0, i0, i1 - i0, 0);
+      if (e == hipSuccess) e = launch(bh, i0, i1, 0, 0, 0, 0);
+    }
+  }
+  return e;
+}
+
 template <int D, int PREC>
 static hipError_t launch_bwd_muon(const ScanArgs& s, float* ws, int64_t ws_floats) {
   const MuonBwdPlan plan = muon_bwd_plan(s.BH, s.N, D, s.ns, ws_floats);
-  if (PREC == 0 || (D >= 64 && plan.nseg >= 1)) {
-    using P = std::conditional_t<PREC == 0, PrecX3, PrecH>;
-    const int lds = 2 * NSSplit<D>::BYTES + 64;
-    auto k = scan_bwd_muon_seg<D, P>;
-    hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return e;
-    // Segments of nseg chunks from the end; Sb and Mbar carry from one
-    // segment's reverse pass to the next through the workspace.  With two
-    // iterate buffers the iterates of segment k + 1 are formed in the launch
-    // that runs segment k's reverse pass (only the first segment's run
-    // alone); with one, each segment's iterates and then its reverse pass.
-    if (plan.nseg < 1) return hipErrorInvalidValue;
-    const int nseg = (int)plan.nseg;
-    MuonSegArgs sa{};
-    sa.U = s.U; sa.K = s.K; sa.av = s.a; sa.bv = s.b; sa.mv = s.m; sa.S_all = s.S_all; sa.M_all = s.M_all;
-    sa.gS = s.gS; sa.dU = s.dU; sa.da = s.da; sa.db = s.db; sa.dm = s.dm; sa.dn = s.dn; sa.ws = ws;
-    sa.BH = s.BH; sa.N = (int)s.N; sa.ns = s.ns; sa.nseg = nseg; sa.nbuf = plan.nbuf;
-    auto launch = [&](int nx3, int i0, int i1, int xbuf, int j0, int jcur, int pbuf) {
-      sa.nx3 = nx3; sa.i0 = i0; sa.i1 = i1; sa.xbuf = xbuf;
-      sa.j0 = j0; sa.jcur = jcur; sa.pbuf = pbuf;
-      const int64_t blocks = (int64_t)nx3 + s.BH * jcur;
-      hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(D * 4), lds, s.stream, sa);
-      return hipGetLastError();
-    };
-    const int bh = (int)s.BH;
-    int i1 = (int)s.N, i0 = i1 > nseg ? i1 - nseg : 0;
-    if (plan.nbuf == 2) {
-      e = launch(0, 0, 0, 0, i0, i1 - i0, 0);
-      for (int seg = 0; e == hipSuccess && i1 > 0; ++seg) {
-        const int j1 = i0, j0 = j1 > nseg ? j1 - nseg : 0;
-        e = launch(bh, i0, i1, seg & 1, j0, j1 - j0, (seg + 1) & 1);
-        i1 = i0;
-        i0 = j0;
-      }
-    } else {
-      for (; e == hipSuccess && i1 > 0; i1 = i0, i0 = i1 > nseg ? i1 - nseg : 0) {
-        e = launch(0, 0, 0, 0, i0, i1 - i0, 0);
-        if (e == hipSuccess) e = launch(bh, i0, i1, 0, 0, 0, 0);
-      }
-    }
-    return e;
-  } else {
-    auto kern = scan_bwd_muon<D>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)s.BH), dim3(D * 4), 0, s.stream, s.U, s.K, s.a, s.b, s.m,
-                       s.S_all, s.M_all, s.gS, s.dU, s.da, s.db, s.dm, s.dn, ws, (int)s.N, s.ns);
-    return hipGetLastError();
+  if constexpr (PREC == 0) return launch_bwd_muon_seg<D, NSSplit<D>>(s, ws, plan);
+  if constexpr (D >= 64) {
+    if (plan.nseg >= 1) return launch_bwd_muon_seg<D, NSFull<D>>(s, ws, plan);
   }
+  hipLaunchKernelGGL((scan_bwd_muon<D>), dim3((unsigned)s.BH), dim3(D * 4), 0, s.stream, s.U, s.K, s.a, s.b, s.m,
+                     s.S_all, s.M_all, s.gS, s.dU, s.da, s.db, s.dm, s.dn, ws, (int)s.N, s.ns);
+  return hipGetLastError();
 }
 
 hipError_t scan_fwd_muon_launch(const ScanArgs& s) {

@@ -90,16 +90,19 @@ int gmdn_scan_fwd(const float* U, const float* K, const float* a, const float* b
                   int32_t ns, int32_t precision, void* stream);
 
 /* Workspace bytes gmdn_scan_bwd needs for these sizes (0 if none): adam
- * keeps per-row-tile partial sums of its scalar gradients.  Muon ('tf32')
- * runs the chunks in segments from the end and keeps, per chunk of a segment
+ * keeps per-row-tile partial sums of its scalar gradients.  Muon ('tf32',
+ * and 'ieee' at dh >= 64) runs the chunks in segments from the end and keeps, per chunk of a segment
  * and (b, h), the Newton-Schulz iterates X_0 .. X_ns, the products
  * Z_0 .. Z_{ns-1}, P_0 .. P_{ns-1} and M_i (3 ns + 2 dh^2 floats) and |M_i|,
  * plus two carried
  * dh^2 matrices per (b, h); the size returned here has as many chunks per
  * segment as fit in 512 MiB (at least one, at most N), and gmdn_scan_bwd also
  * accepts any smaller workspace down to one-chunk segments, using as many
- * chunks per segment as it holds.  Muon ('ieee'): 4 + ns dh^2 matrices per
- * (b, h). */
+ * chunks per segment as it holds, with the same bits.  Muon in 'ieee' takes
+ * still less, down to 4 + ns dh^2 matrices per (b, h): below a one-chunk
+ * segment (and at dh = 32) the chunks run one after another, with the same
+ * float32 products summed in another order and about ten times slower at
+ * dh = 128. */
 size_t gmdn_scan_bwd_workspace_bytes(int64_t BH, int64_t N, int32_t dh, int32_t rule,
                                      int32_t ns);
 
@@ -127,12 +130,13 @@ int gmdn_scan_bwd(const float* U, const float* K, const float* a, const float* b
  * workspace lives in a file-scope device array of GMDN_NOALLOC_SCRATCH_BYTES
  * (64 MiB), one per GPU the library runs on, held until the process ends;
  * the call allocates nothing.  Problems whose smallest workspace (for muon
- * in 'tf32', one-chunk segments; otherwise gmdn_scan_bwd_workspace_bytes)
- * exceeds that size are refused with GMDN_ERR_WORKSPACE before any launch.  Every call on one GPU shares that
+ * one-chunk segments in 'tf32', 4 + ns matrices per (b, h) in 'ieee';
+ * otherwise gmdn_scan_bwd_workspace_bytes) exceeds that size are refused with
+ * GMDN_ERR_WORKSPACE before any launch.  Every call on one GPU shares that
  * GPU's scratch: calls that overlap on one GPU (other streams, other host
  * threads) race and must be serialised by the caller.  Nothing a previous
  * call left in the scratch is read.  Same arguments, results and error codes
- * as gmdn_scan_bwd otherwise. */
+ * as gmdn_scan_bwd with a workspace of that size otherwise. */
 int gmdn_scan_bwd_noalloc(const float* U, const float* K, const float* a, const float* b,
                           const float* m, const float* n, const float* S_all,
                           const float* M_all, const float* V_all, const float* gS,
@@ -219,7 +223,10 @@ int gmdn_wy_bwd(const gmdn_chunk_desc* desc, const void* q, const void* k, const
  * in 'tf32' also runs with any smaller workspace down to one-chunk segments
  * of its reverse scan (the results do not depend on the segment length);
  * this size gives segments of up to 512 MiB of iterates, in two buffers
- * when they do not hold every chunk.  Adam (rule 2) at d = 64 on bfloat16
+ * when they do not hold every chunk.  Muon on float32 streams also runs
+ * with 4 + ns d^2 matrices per (b, h) in place of the reverse scan's part of
+ * it (the same float32 products in another order of summation, slower: see
+ * gmdn_scan_bwd_workspace_bytes).  Adam (rule 2) at d = 64 on bfloat16
  * streams: this size ends with a carry of the reverse scan's cotangents
  * (B H d d * 3 floats), with which the scan runs in chunk segments and each
  * segment's token gradients run on a second stream of the library's (one

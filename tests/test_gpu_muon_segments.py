@@ -179,9 +179,9 @@ def _bwd_ieee(lib, ins, S_all, M_all, gS, ns, ws_bytes):
 @pytest.mark.parametrize("N,dh,ns", [(5, 64, 3), (4, 128, 5), (3, 128, 0), (3, 64, 8), (4, 32, 5)])
 def test_muon_backward_ieee_workspaces(N, dh, ns, gscale):
     """'ieee': segments give the default workspace's bits, and the smallest
-    accepted workspace (4 + ns matrices per head: exact float32 products
-    throughout) the same gradients to float32 accuracy at any scale of the
-    cotangent -- both within 2e-4 of each other relative to the largest entry,
+    accepted workspace (4 + ns matrices per head: the same float32 products
+    summed in another order) the same gradients to float32 accuracy at any
+    scale of the cotangent -- both within 2e-4 of each other relative to the largest entry,
     four times the largest float32 error of this shape (ns = 8 amplifies
     rounding by up to 3.4445^8 in small singular directions: 1e-2 there)."""
     dev = _dev()
@@ -215,3 +215,57 @@ def test_muon_scan_ieee_scales(dh, vscale):
     want = osc.scan_forward(*[t.double() for t in ins], 1, 3)
     floor = osc.rel_err(osc.scan_forward(*ins, 1, 3), want)
     assert osc.rel_err(got, want) <= max(1e-4, 2 * floor)
+
+
+@pytest.mark.parametrize("down", ["rows", "columns"])
+@pytest.mark.parametrize("dh,ns", [(32, 3), (64, 3), (128, 3), (128, 5)])
+def test_muon_scan_ieee_graded(dh, ns, down):
+    """Rows (columns) of the momentum from 1 down to 2^-40 of the largest: each
+    keeps float32's relative accuracy in msign, which scales it by much the
+    same factor as the large ones.  Per row against float64, within
+    3.4445^ns sqrt(d) 2^-24: a step grows a small direction, and a rounding in
+    it, at most 3.4445-fold, and a sum of d float32 products rounds to about
+    sqrt(d) 2^-24 (1.1e-6 to 2.6e-6 at ns = 3 for float32 on the host, where
+    22-bit pieces of one scale lose such rows altogether)."""
+    from gmdn_amd.scan import hip_state_scan
+    dev = _dev()
+    gen = torch.Generator().manual_seed(dh + ns)
+    U, K, *gates = osc.make_scan_inputs(1, 2, 3, 64, dh, generator=gen)
+    g = 2.0 ** -(torch.arange(dh) % 41).float()
+    U = U * (g[:, None] if down == "rows" else g)
+    K = K * 0  # G = U: every chunk's momentum keeps the grading
+    got = hip_state_scan(*[t.to(dev) for t in (U, K, *gates)], 1, ns, precision="ieee").cpu().double()
+    want = osc.scan_forward(*[t.double() for t in (U, K, *gates)], 1, ns)
+    ref = osc.scan_forward(U, K, *gates, 1, ns).double()
+    dim = -1 if down == "rows" else -2
+
+    def err(x):
+        return ((x - want)[:, :, 1:].norm(dim=dim) / want[:, :, 1:].norm(dim=dim)).max().item()
+
+    print(f"graded {down} d{dh} ns{ns}: {err(got):.2e}, float32 reference {err(ref):.2e}", flush=True)
+    assert err(got) <= 3.4445**ns * dh**0.5 * 2.0**-24
+
+
+@pytest.mark.parametrize("d,ns", [(32, 3), (64, 3), (128, 5)])
+def test_float32_muon_core_smallest_workspace(d, ns):
+    """gmdn_chunk_bwd on float32 streams: the smallest accepted workspace (the
+    three d x d planes and the scalars of every chunk, and 4 + ns matrices per
+    head) gives the default's gradients to float32 accuracy; one byte less is
+    refused."""
+    from gmdn_amd import ops
+    from gmdn_amd.workloads import Workload, make_inputs
+    dev = _dev()
+    lib = nat.load()
+    B, H, N = 1, 2, 3
+    inp = make_inputs(Workload("min", "muon", B, H, N * 64, d, ns=ns), seed=d, with_grad_out=True)
+    ins = [inp[n].to(dev).float().contiguous() for n in ("q", "k", "v", "beta", "g", "gmu", "dO")]
+    _, states = torch.ops.gmdn.chunk_fwd(*ins[:6], None, 1, ns, 1e-6, True)
+    full = lib.gmdn_chunk_bwd_workspace_bytes(ops_desc(ins, ns))
+    least = 4 * (B * H * N * (3 * d * d + 4) + B * H * (4 + ns) * d * d)
+    assert least <= full
+    want = _fused_bwd(lib, ins, states, ns, full)
+    got = _fused_bwd(lib, ins, states, ns, least)
+    for name, x, y in zip("dq dk dv dbeta dg dgmu".split(), got, want):
+        assert torch.isfinite(y).all() and osc.rel_err(x.cpu(), y.cpu()) <= 2e-4, name
+    with pytest.raises(RuntimeError, match="workspace"):
+        _fused_bwd(lib, ins, states, ns, least - 1)
