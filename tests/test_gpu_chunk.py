@@ -401,3 +401,46 @@ def test_muon_grads_config_heads():
             if e_hip > max(TOL, 2.0 * e_f32):
                 bad[(b, h, n)] = (e_hip, e_f32)
     assert not bad, bad
+
+
+@pytest.mark.parametrize("dtype,d", [("bf16", 64), ("bf16", 128), ("f32", 32), ("f32", 64), ("f32", 128)])
+@pytest.mark.parametrize("T", [128, 320])
+def test_adam_grads_well_conditioned(dtype, d, T):
+    """Adam's core where sqrt(V) stays away from zero, so that every gradient
+    has a typical size and a dropped term shows: k close to one unit direction
+    s / sqrt(d) and |v| in [1, 2] 256 of one sign a row make |U| at least
+    64 * 256 / sqrt(d) * 0.5, above twice |S K| <= 256 * 4.  Frobenius error
+    against float64: the results' rounding (bf16: uniform within half an ulp,
+    at most 2^-8 of a value, so below 2^-8 / sqrt(3) in the mean), and for the
+    products 2^-16 (split bf16, d = 64) or float32, grown at most 100-fold by
+    the division and the cancelling sums."""
+    dev = _dev()
+    B, H = 1, 2
+    gen = torch.Generator().manual_seed(d + T)
+
+    def rand(*s):
+        return torch.rand(*s, generator=gen)
+
+    sgn, row = (torch.sign(rand(d) - 0.5) for _ in range(2))
+    k = sgn * (1 + 0.2 * (rand(B, H, T, d) - 0.5))
+    q = torch.randn(B, H, T, d, generator=gen)
+    q, k = (t / t.norm(dim=-1, keepdim=True) for t in (q, k))
+    v = 256 * row * (1 + rand(B, H, T, d))
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    q, k, v, dO = (t.to(dt) for t in (q, k, v, torch.randn(B, H, T, d, generator=gen)))
+    gates = [torch.sigmoid(torch.randn(B, H, T, generator=gen)), torch.log(0.9 + 0.1 * rand(B, H, T)) / 8,
+             torch.log(0.9 + 0.1 * rand(B, H, T)) / 8, torch.log(0.99 + 0.01 * rand(B, H, T)) / 8]
+    xs = [t.to(dev).requires_grad_() for t in (q, k, v, *gates)]
+    o = gc.chunk_scan(*xs, rule="adam")
+    got = [o.detach(), *torch.autograd.grad(o, xs, dO.to(dev))]
+    rs = [t.double().requires_grad_() for t in (q, k, v, *gates)]
+    ro = oc.mixer_core(*rs, rule=2, ns=3, C=64)
+    want = [ro.detach(), *torch.autograd.grad(ro, rs, dO.double())]
+    errs = {}
+    for n, x, y in zip(("o", *ALL_INPUTS), got, want):
+        # (two chunks: the first one's decay multiplies the zero state)
+        errs[n] = ((x.double().cpu() - y).norm() / y.norm()).item() if y.any() else x.norm().item()
+    print(f"adam {dtype} d{d} T{T}: " + " ".join(f"{n} {e:.1e}" for n, e in errs.items()), flush=True)
+    bound = 100 * (2.0**-16 if (dtype, d) == ("bf16", 64) else 2.0**-23)
+    for n, e in errs.items():
+        assert e <= bound + (2.0**-8 / 3**0.5 if dtype == "bf16" and n in ("o", "q", "k", "v") else 0), (n, e)
