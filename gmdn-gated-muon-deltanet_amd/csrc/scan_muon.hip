@@ -15,10 +15,10 @@
 // float32 products, chunk after chunk, through four matrices in that
 // workspace.
 // 'ieee' is bound by the float32 MFMAs (1/16 of the bfloat16 rate): 20.5 us
-// of them a Newton-Schulz step at D = 128, 61 of a chunk's 79 us at ns = 3.
-// Measured (8 heads, 8 chunks, D = 128, ns = 3) against P through four
-// matrices in a global workspace, everything serial: forward 946 -> 631 us,
-// backward 10.1 -> 1.02 ms, the forward's bits the same.
+// of them a Newton-Schulz step at D = 128, 61 of a chunk's 81 us at ns = 3.
+// Measured (8 heads, 8 chunks, D = 128, ns = 3) against products through four
+// matrices in a global workspace, everything serial: forward 946 -> 652 us,
+// backward 10.1 -> 1.07 ms.
 #include "muon_bwd.h"
 #include "ns.h"
 #include "scan_a.h"
