@@ -177,6 +177,21 @@ def _head_norm_bwd_fake(x, weight, rstd, dout):
     return torch.empty_like(x, memory_format=torch.contiguous_format), weight.new_empty(weight.shape)
 
 
+_FAKES = {
+    "state_scan": _state_scan_fake,
+    "state_scan_bwd": _state_scan_bwd_fake,
+    "chunk_fwd": _chunk_fwd_fake,
+    "chunk_bwd": _chunk_bwd_fake,
+    "chunk_bwd_muon": _chunk_bwd_muon_fake,
+    "wy_fwd": _wy_fwd_fake,
+    "wy_bwd": _wy_bwd_fake,
+    "front_fwd": _front_fwd_fake,
+    "front_bwd": _front_bwd_fake,
+    "gates_fwd": _gates_fwd_fake,
+    "gates_bwd": _gates_bwd_fake,
+    "head_norm_fwd": _head_norm_fwd_fake,
+    "head_norm_bwd": _head_norm_bwd_fake,
+}
 # Set by _register_fakes.  Without the native libraries the operators do not
 # exist: every entry point calls ensure(), which raises what _native.load raises.
 REGISTERED = False
@@ -184,21 +199,7 @@ REGISTERED = False
 
 def _register_fakes():
     global REGISTERED
-    for name, fake in (
-            ("state_scan", _state_scan_fake),
-            ("state_scan_bwd", _state_scan_bwd_fake),
-            ("chunk_fwd", _chunk_fwd_fake),
-            ("chunk_bwd", _chunk_bwd_fake),
-            ("chunk_bwd_muon", _chunk_bwd_muon_fake),
-            ("wy_fwd", _wy_fwd_fake),
-            ("wy_bwd", _wy_bwd_fake),
-            ("front_fwd", _front_fwd_fake),
-            ("front_bwd", _front_bwd_fake),
-            ("gates_fwd", _gates_fwd_fake),
-            ("gates_bwd", _gates_bwd_fake),
-            ("head_norm_fwd", _head_norm_fwd_fake),
-            ("head_norm_bwd", _head_norm_bwd_fake),
-    ):
+    for name, fake in _FAKES.items():
         torch.library.register_fake(f"gmdn::{name}", fake)
     REGISTERED = True
 
@@ -212,6 +213,14 @@ def ensure() -> None:
     have been built after this module's import)."""
     if not REGISTERED:
         nat.load()
+
+
+def __getattr__(name: str):
+    """The C++ operators by name, as ``msign`` is: ``ops.chunk_fwd(...)``."""
+    if name in _FAKES:
+        ensure()
+        return getattr(torch.ops.gmdn, name)
+    raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
 
 
 def _dtype_code(t: Tensor) -> int:

@@ -40,6 +40,13 @@ CHUNK = 64
 LOG_FLOOR = math.log(1e-6)
 
 
+def __getattr__(name: str):
+    """The operators ``wy_fwd`` and ``wy_bwd``."""
+    if name in ("wy_fwd", "wy_bwd"):
+        return getattr(ops, name)
+    raise AttributeError(f"module {__name__!r} has no attribute {name!r}")
+
+
 def wy_chunk_terms(q, k, v, beta, g):
     """Per chunk, in float32: a (B, H, N), U_A, K_A (B, H, N, d, d), Qt, Ov
     (B, H, N, C, d) -- the quantities the prep kernel forms."""

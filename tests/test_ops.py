@@ -210,3 +210,15 @@ def test_compiled_autograd_traces_the_backward(name):
         finally:
             scan.set_precision("tf32")
         assert len(traces) == 2
+
+
+def test_operators_by_module_name():
+    from gmdn_amd import wy
+    for name in ("state_scan", "state_scan_bwd", "chunk_fwd", "chunk_bwd", "chunk_bwd_muon", "front_fwd", "front_bwd",
+                 "gates_fwd", "gates_bwd", "head_norm_fwd", "head_norm_bwd", "msign"):
+        assert callable(getattr(ops, name)), name
+    q, g = torch.empty(1, 2, 128, 64, device="meta", dtype=torch.bfloat16), torch.empty(1, 2, 128, device="meta")
+    o, ckpt = wy.wy_fwd(q, q, q, g, g, True)
+    assert o.shape == q.shape and len(wy.wy_bwd(q, q, q, g, g, ckpt, o)) == 5
+    with pytest.raises(AttributeError):
+        ops.no_such_operator
